@@ -1,6 +1,7 @@
 """Builds the native parts of rustautograd_amd in-tree.
 
-    python -m rustautograd_amd.build          # engine module + librg_hip.so (gfx950)
+    python -c "import __graft_entry__; __graft_entry__.build()"   # this module's build_all, and the oracle
+    python -m rustautograd_amd.build                              # build_all again, once the package imports
 
 - `_rg*.so`: the C++ engine (graph, autodiff, optimizer, planner, validation, run loop) as a
   pybind11 module, built with g++.

@@ -27,8 +27,8 @@ def _ensure_built():
     import subprocess
     if not glob.glob(os.path.join(ROOT, "rustautograd_amd", "_rg*.so")):
         sys.path.insert(0, ROOT)
-        from rustautograd_amd import build
-        build.build_engine()
+        import __graft_entry__
+        __graft_entry__.native_build().build_engine()
     if not os.path.exists(ORACLE):
         subprocess.run(["bash", os.path.join(ROOT, "oracle", "build.sh")], check=True)
 
