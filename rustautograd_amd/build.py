@@ -1,6 +1,6 @@
 """Builds the native parts of rustautograd_amd in-tree.
 
-    python -c "import __graft_entry__; __graft_entry__.build()"   # this module's build_all, and the oracle
+    python -c "import __graft_entry__; __graft_entry__.build()"   # on a fresh checkout
     python -m rustautograd_amd.build                              # build_all again, once the package imports
 
 - `_rg*.so`: the C++ engine (graph, autodiff, optimizer, planner, validation, run loop) as a
@@ -82,8 +82,8 @@ def build_hip():
     os.makedirs(os.path.join(BUILD, "hip"), exist_ok=True)
     os.makedirs(LIB, exist_ok=True)
     src = os.path.join(CSRC, "hip")
-    embedded = os.path.join(BUILD, "hip", "gemm_mfma_source.cpp")
-    embed_source(os.path.join(src, "gemm_mfma.h"), "rg_gemm_mfma_source", embedded)
+    embedded = os.path.join(BUILD, "hip", "gemm_split_source.cpp")
+    embed_source(os.path.join(src, "gemm_split.h"), "rg_gemm_split_source", embedded)
 
     def compile_one(name):
         obj = os.path.join(BUILD, "hip", os.path.basename(name) + ".o")
