@@ -1,9 +1,10 @@
 // Dense products for MatMul / MatMulT (reference src/plan.rs:1453-1493, flags from
 // src/optimize.rs:338-350).
 //
-// fp32: block tiles from 128x128 down to 128x32 / 32x128, four or eight wave64s per block, each
-// wave owning a grid of 16x16 MFMA tiles (v_mfma_f32_16x16x4f32), or of 32x32 ones
-// (v_mfma_f32_32x32x2f32) for some shapes. Global loads run two K steps ahead through two register
+// fp32: most products run on the bf16 matrix cores, every operand value split exactly into three
+// bf16 values (gemm_split.h: block tiles of 128x128, 128x64 and 64x64). Products of too few tiles
+// for that take fp32 MFMA tiles (gemm_mfma.h), of four wave64s, each owning a grid of 16x16 MFMA
+// tiles (v_mfma_f32_16x16x4_f32). There global loads run two K steps ahead through two register
 // stages, and operands are staged through double-buffered LDS in their own global layout, so no
 // operand is transposed while staging:
 //  - a K-contiguous operand (A, or B when transposed) sits in LDS as [rows][BK + 4]; one 16-byte
@@ -12,10 +13,10 @@
 //    columns at one k, one for each of the wave's T tiles (tile t holds columns t, t + T, ...).
 // Global loads are 16-byte vectors without branches: a vector lies wholly inside or outside the
 // operand (leading dimensions are multiples of 4), and an outside vector reads a valid address
-// and is replaced by zeros; products whose tiles divide M, N and K skip even that check. The tile
-// is chosen per product to fill 256 CUs with little padding (32-wide tiles for 32-wide attention
-// heads); products whose output still has too few tiles split K and combine the partial sums in a
-// fixed order (deterministic). Unaligned operands take the same kernel with scalar loads.
+// and is replaced by zeros; products whose tiles divide M, N and K skip even that check. Unaligned
+// operands take the same kernel with scalar loads. The tile is chosen per product to fill 256 CUs
+// with little padding; products whose output has too few tiles split K and combine the partial
+// sums in a fixed order (deterministic).
 // fp32 products with at most 16 rows and a long K, or a K of at most 16, stream through the
 // skinny kernels below (HBM-bound shapes); fp64 and the remaining tiny products use a plain
 // kernel, one thread per output element.
@@ -26,6 +27,7 @@
 #include <string>
 
 #include "gemm_mfma.h"
+#include "gemm_split.h"
 #include "kernels.h"
 #include "ops.h"
 
@@ -36,14 +38,30 @@ namespace {
 using namespace rgg;
 
 template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB, int MODE, int MS>
-__global__ void __launch_bounds__(64 * WM * WN) k_gemm_mfma(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C,
+__global__ void __launch_bounds__(64 * WM * WN) k_gemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C,
                                                            int M, int N, int K, const int64_t* a_off, const int64_t* b_off,
                                                            uint64_t a_stride, uint64_t b_stride, int splits, int k_per_split,
-                                                           float* __restrict__ partial, const float* __restrict__ bias, uint32_t tiles_m,
-                                                           uint32_t tiles_n, int swizzle) {
+                                                          float* __restrict__ partial, const float* __restrict__ bias, uint32_t tiles_m,
+                                                          uint32_t tiles_n, int swizzle) {
   rgg::StoreC epi{C, partial, splits, (uint64_t)M * N};
-  rgg::gemm_mfma_block<BM, BN, BK, WM, WN, TA, TB, MODE, MS>(A, B, M, N, K, a_off, b_off, a_stride, b_stride, splits, k_per_split, bias,
+  rgg::gemm_f32_block<BM, BN, BK, WM, WN, TA, TB, MODE, MS>(A, B, M, N, K, a_off, b_off, a_stride, b_stride, splits, k_per_split, bias,
                                                               tiles_m, tiles_n, swizzle, epi);
+}
+
+// Blocks per SIMD's worth of waves the registers must leave room for: two 128x128 blocks of eight
+// waves, three 128x64 or four 64x64 blocks of four per CU.
+constexpr int split_waves(int bm, int bn) { return bm * bn >= 128 * 128 ? 4 : bm * bn >= 128 * 64 ? 3 : 4; }
+
+template <int BM, int BN, int WM, int WN, bool TA, bool TB, bool TAIL>
+__global__ void __launch_bounds__(64 * WM * WN, split_waves(BM, BN)) k_gemm_mfma(const float* __restrict__ A, const float* __restrict__ B,
+                                                                               float* __restrict__ C, int M, int N, int K,
+                                                                               const int64_t* a_off, const int64_t* b_off, uint64_t a_stride,
+                                                                               uint64_t b_stride, int splits, int k_per_split,
+                                                                               float* __restrict__ partial, const float* __restrict__ bias,
+                                                                               uint32_t tiles_m, uint32_t tiles_n) {
+  rgg::StoreC epi{C, partial, splits, (uint64_t)M * N};
+  rgg::gemm_mfma_block<BM, BN, WM, WN, TA, TB, TAIL>(A, B, M, N, K, a_off, b_off, a_stride, b_stride, splits, k_per_split, bias, tiles_m,
+                                                     tiles_n, epi);
 }
 
 // One unbatched product's share of a grouped launch (k_gemm_mfma_group).
@@ -60,34 +78,34 @@ struct GroupParts {
 };
 
 // Part I of a grouped launch: flags bits 2I (TB) and 2I + 1 (TA).
-template <int BM, int BN, int BK, int WM, int WN, int FLAGS, int I>
-__device__ __forceinline__ void group_part(const GroupPart& p, uint32_t bid, float* smem) {
+template <int BM, int BN, int WM, int WN, int FLAGS, int I>
+__device__ __forceinline__ void group_part(const GroupPart& p, uint32_t bid, cell* smem) {
   constexpr bool TA = (FLAGS >> (2 * I + 1)) & 1, TB = (FLAGS >> (2 * I)) & 1;
   StoreC epi{p.c, p.part, p.splits, (uint64_t)p.m * p.n};
-  gemm_mfma_tile<BM, BN, BK, WM, WN, TA, TB, LOAD_EVEN, 16>(p.a, p.b, p.m, p.n, p.k, nullptr, nullptr, 0, 0, p.splits, p.kps, p.bias, p.tm,
-                                                             p.tn, 1, epi, bid, p.blocks, smem);
+  gemm_split_tile<BM, BN, WM, WN, TA, TB, false>(p.a, p.b, p.m, p.n, p.k, nullptr, nullptr, 0, 0, p.splits, p.kps, p.bias, p.tm, p.tn, epi, bid,
+                                                 p.blocks, smem);
 }
 
-template <int BM, int BN, int BK, int FLAGS, int I>
+template <int BM, int BN, int WM, int WN, int FLAGS, int I>
 constexpr int part_lds() {
-  return TileLds<BM, BN, BK, ((FLAGS >> (2 * I + 1)) & 1) != 0, ((FLAGS >> (2 * I)) & 1) != 0>::FLOATS;
+  return SplitLds<BM, BN, WM, WN, ((FLAGS >> (2 * I + 1)) & 1) != 0, ((FLAGS >> (2 * I)) & 1) != 0>::CELLS;
 }
 
 // N independent unbatched products on one tile shape in one launch: part i takes the next
 // p[i].blocks blocks, all staging through the same LDS. Each block runs the code of a single
 // product's launch, so every output gets the same bits; the launch's fixed cost is paid once,
-// and the parts' grids (each about one block per CU) run side by side.
-template <int BM, int BN, int BK, int WM, int WN, int N, int FLAGS>
-__global__ void __launch_bounds__(64 * WM * WN) k_gemm_mfma_group(GroupParts g) {
-  constexpr int F0 = part_lds<BM, BN, BK, FLAGS, 0>(), F1 = part_lds<BM, BN, BK, FLAGS, 1>();
-  constexpr int F2 = N > 2 ? part_lds<BM, BN, BK, FLAGS, 2>() : 0;
+// and the parts' grids (each one or two blocks per CU) run side by side.
+template <int BM, int BN, int WM, int WN, int N, int FLAGS>
+__global__ void __launch_bounds__(64 * WM * WN, split_waves(BM, BN)) k_gemm_mfma_group(GroupParts g) {
+  constexpr int F0 = part_lds<BM, BN, WM, WN, FLAGS, 0>(), F1 = part_lds<BM, BN, WM, WN, FLAGS, 1>();
+  constexpr int F2 = N > 2 ? part_lds<BM, BN, WM, WN, FLAGS, 2>() : 0;
   constexpr int F01 = F0 > F1 ? F0 : F1;
-  __shared__ float smem[F01 > F2 ? F01 : F2];
+  __shared__ cell smem[F01 > F2 ? F01 : F2];
   uint32_t bid = blockIdx.x;
-  if (bid < g.p[0].blocks) return group_part<BM, BN, BK, WM, WN, FLAGS, 0>(g.p[0], bid, smem);
+  if (bid < g.p[0].blocks) return group_part<BM, BN, WM, WN, FLAGS, 0>(g.p[0], bid, smem);
   bid -= g.p[0].blocks;
-  if (N == 2 || bid < g.p[1].blocks) return group_part<BM, BN, BK, WM, WN, FLAGS, 1>(g.p[1], bid, smem);
-  if constexpr (N > 2) group_part<BM, BN, BK, WM, WN, FLAGS, 2>(g.p[2], bid - g.p[1].blocks, smem);
+  if (N == 2 || bid < g.p[1].blocks) return group_part<BM, BN, WM, WN, FLAGS, 1>(g.p[1], bid, smem);
+  if constexpr (N > 2) group_part<BM, BN, WM, WN, FLAGS, 2>(g.p[2], bid - g.p[1].blocks, smem);
 }
 
 // Sums the K-split partial products in split order. Four outputs per thread (16-byte loads when
@@ -534,43 +552,51 @@ int skinny_rows_splits(uint64_t n, uint64_t k) {
 }
 
 struct TileCfg {
-  int bm, bn, bk, wm, wn, ms = 16;
+  int bm, bn, bk, wm, wn;
+  bool split;  // bf16 terms (gemm_split.h); otherwise fp32 MFMA (gemm_mfma.h)
 };
+constexpr TileCfg SPLIT_128x128 = {128, 128, SPLIT_BK, 2, 4, true}, SPLIT_128x64 = {128, 64, SPLIT_BK, 2, 2, true},
+                  SPLIT_64x64 = {64, 64, SPLIT_BK, 2, 2, true};
 
-int split_count(const TileCfg& t, uint64_t m, uint64_t n, uint64_t k, uint64_t batch);
+uint64_t tile_count(const TileCfg& t, uint64_t m, uint64_t n, uint64_t batch) { return ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn) * batch; }
 
-// Block tile, from measurements of C4's products on MI355X: 32-wide tiles for outputs 32..96 wide
-// or 32 tall (attention heads, the vocabulary); 128x128 when that still yields two blocks per CU
-// (512), then 128x64 at two blocks per CU; 128x64 with eight waves (two per SIMD) at one block per
-// CU, and for long-K products with at least 32 such tiles (split over K to 256 blocks); 64x128 at
-// one block per CU; 64x64 (split over K when that leaves the CUs idle); 32x32 when even split
-// 64x64 tiles come to fewer than 256 blocks (C3's products). The same shapes whichever operand is
-// K-contiguous: with the non-temporal output stores, 64x64 tiles of 32x32 MFMAs, once faster for a
-// K-contiguous B, are 1-9 % slower than 128x64 ones on C4's input-gradient products.
-TileCfg pick_tile(uint64_t m, uint64_t n, uint64_t k, uint64_t batch) {
-  auto blocks = [&](int bm, int bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn) * batch; };
-  if (n <= 96 && n % 32 == 0) return {128, 32, 32, 4, 1};
-  if (m <= 32) return {32, 128, 32, 1, 4};
-  if (blocks(128, 128) >= 512) return {128, 128, 16, 2, 2};
-  if (blocks(128, 64) >= 512) return {128, 64, 16, 2, 2};
-  if (blocks(128, 64) >= 256 || (blocks(128, 64) >= 32 && k >= 4096)) return {128, 64, 32, 2, 4};
-  if (blocks(64, 128) >= 256) return {64, 128, 32, 2, 2};
-  // Small outputs: 32x32 tiles when 64x64 ones, split over K where K allows, would leave most
-  // CUs idle (C3's products: 4096 x 128 over K <= 512, 128 x 128 weight gradients).
-  const TileCfg t64 = {64, 64, 32, 2, 2};
-  if (blocks(64, 64) * (uint64_t)split_count(t64, m, n, k, batch) < 256) return {32, 32, 32, 2, 2};
-  return t64;
-}
-
-// K splits for products with too few tiles: about 256 blocks of eight waves or 768 of four, each
-// split at least 512 deep, at most 16.
+// K splits for products with too few tiles: about 512 blocks of 128x128 (two per CU), 768 of the
+// smaller tiles, each split at least 512 deep, at most 16.
 int split_count(const TileCfg& t, uint64_t m, uint64_t n, uint64_t k, uint64_t batch) {
-  uint64_t tiles = ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn) * batch;
+  uint64_t tiles = tile_count(t, m, n, batch);
   if (tiles >= 256 || k < 1024) return 1;
-  uint64_t target = t.wm * t.wn == 8 ? 256 : 768;
+  uint64_t target = t.bm * t.bn >= 128 * 128 ? 512 : 768;
   uint64_t want = (target + tiles - 1) / tiles;
   uint64_t most = k / 512;
   return (int)std::max<uint64_t>(1, std::min<uint64_t>(std::min(want, most), 16));
+}
+
+// Block tile, from measurements on MI355X (us; M x N x K, T: that operand transposed).
+// Products whose 64x64 tiles, split over K where K allows, come to a block per CU run on the bf16
+// terms:
+//  - 128x128 at two blocks per CU and K over 256 (4096x2048x2048: 183 against 223 on 128x64;
+//    4096x2048x512: 53 and 57), or a K of 2048 and more whose splits give most CUs a block
+//    (T 256x1024x8192: 34 against 36 on 128x64, 46 on 64x64; T 2048x2048x4096: 203 and 221);
+//  - 128x64 at three blocks per CU (8192x768x256: 24.0 against 25.3 on 128x128 and 25.8 on 64x64),
+//    and at four for K up to 256 (8192x1024x256, T: 27.8 against 29.1 on 128x128);
+//  - 64x64 otherwise (8192x256x256: 11.1 against 11.7 on 128x64; fp32 MFMA tiles 11.7).
+// Below that a block runs alone on its CU and fp32 MFMA tiles are faster: 32-wide ones for outputs
+// 32..96 wide or 32 tall (attention heads, the vocabulary), 32x32 otherwise (256x768x256: 4.3
+// against 7.1 on bf16 terms; 4096x128x512: 8.6 and 13), or 64x64 where a side under 64 keeps a
+// large output off the tiles above.
+TileCfg pick_tile(uint64_t m, uint64_t n, uint64_t k, uint64_t batch) {
+  auto filled = [&](const TileCfg& t) { return tile_count(t, m, n, batch) * (uint64_t)split_count(t, m, n, k, batch); };
+  // A column-contiguous operand's offsets within 24 rows are 32-bit: sides of less than 2^25.
+  if (m >= 64 && n >= 64 && m < (1u << 25) && n < (1u << 25) && filled(SPLIT_64x64) >= 256) {
+    if (m >= 128 && n >= 128 && ((tile_count(SPLIT_128x128, m, n, batch) >= 512 && k > 256) || (k >= 2048 && filled(SPLIT_128x128) >= 192)))
+      return SPLIT_128x128;
+    if (m >= 128 && tile_count(SPLIT_128x64, m, n, batch) >= 768) return SPLIT_128x64;
+    return SPLIT_64x64;
+  }
+  if (n <= 96 && n % 32 == 0) return {128, 32, 32, 4, 1, false};
+  if (m <= 32) return {32, 128, 32, 1, 4, false};
+  const TileCfg t64 = {64, 64, 32, 2, 2, false};
+  return filled(t64) < 256 ? TileCfg{32, 32, 32, 2, 2, false} : t64;
 }
 
 struct Launch {
@@ -586,39 +612,50 @@ struct Launch {
   uint32_t tm, tn;
 };
 
-template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB, int MS>
+// `mode`: the fp32 tile's load mode, or whether some K range of the split tile is no multiple of 32.
+template <int BM, int BN, int WM, int WN, bool TA, bool TB, bool SPLIT>
 void launch_mode(hipStream_t s, int mode, const Launch& l) {
-#define RG_GEMM(MODE_)                                                                                                       \
-  hipLaunchKernelGGL((k_gemm_mfma<BM, BN, BK, WM, WN, TA, TB, MODE_, MS>), l.grid, dim3(64 * WM * WN), 0, s, l.a, l.b, l.c, l.m, l.n, \
-                     l.k, l.a_off, l.b_off, l.as, l.bs, l.splits, l.kps, l.part, l.bias, l.tm, \
-                     l.tn, 1)
-  if (mode == LOAD_EVEN) RG_GEMM(LOAD_EVEN);
-  else if (mode == LOAD_VEC) RG_GEMM(LOAD_VEC);
-  else RG_GEMM(LOAD_SCALAR);
+  const dim3 block(64 * WM * WN);
+  if constexpr (SPLIT) {
+#define RG_GEMM(TAIL_)                                                                                                              \
+  hipLaunchKernelGGL((k_gemm_mfma<BM, BN, WM, WN, TA, TB, TAIL_>), l.grid, block, 0, s, l.a, l.b, l.c, l.m, l.n, l.k, l.a_off, l.b_off, \
+                     l.as, l.bs, l.splits, l.kps, l.part, l.bias, l.tm, l.tn)
+    if (mode) RG_GEMM(true);
+    else RG_GEMM(false);
 #undef RG_GEMM
+  } else {
+#define RG_GEMM(MODE_)                                                                                                                \
+  hipLaunchKernelGGL((k_gemm_f32<BM, BN, 32, WM, WN, TA, TB, MODE_, 16>), l.grid, block, 0, s, l.a, l.b, l.c, l.m, l.n, l.k, l.a_off, l.b_off, \
+                     l.as, l.bs, l.splits, l.kps, l.part, l.bias, l.tm, l.tn, 1)
+    if (mode == LOAD_EVEN) RG_GEMM(LOAD_EVEN);
+    else if (mode == LOAD_VEC) RG_GEMM(LOAD_VEC);
+    else RG_GEMM(LOAD_SCALAR);
+#undef RG_GEMM
+  }
 }
 
-template <int BM, int BN, int BK, int WM, int WN, int MS = 16>
+template <int BM, int BN, int WM, int WN, bool SPLIT>
 void launch_flags(hipStream_t s, bool ta, bool tb, int mode, const Launch& l) {
-  if (!ta && !tb) launch_mode<BM, BN, BK, WM, WN, false, false, MS>(s, mode, l);
-  else if (ta && !tb) launch_mode<BM, BN, BK, WM, WN, true, false, MS>(s, mode, l);
-  else if (!ta && tb) launch_mode<BM, BN, BK, WM, WN, false, true, MS>(s, mode, l);
-  else launch_mode<BM, BN, BK, WM, WN, true, true, MS>(s, mode, l);
+  if (!ta && !tb) launch_mode<BM, BN, WM, WN, false, false, SPLIT>(s, mode, l);
+  else if (ta && !tb) launch_mode<BM, BN, WM, WN, true, false, SPLIT>(s, mode, l);
+  else if (!ta && tb) launch_mode<BM, BN, WM, WN, false, true, SPLIT>(s, mode, l);
+  else launch_mode<BM, BN, WM, WN, true, true, SPLIT>(s, mode, l);
 }
 
 // Instantiates the tile shapes pick_tile can return.
 void launch_mfma(hipStream_t s, const TileCfg& t, bool ta, bool tb, int mode, const Launch& l) {
-#define RG_TILE(BM_, BN_, BK_, WM_, WN_) \
-  if (t.bm == BM_ && t.bn == BN_ && t.bk == BK_ && t.wm == WM_ && t.wn == WN_ && t.ms == 16) return launch_flags<BM_, BN_, BK_, WM_, WN_>(s, ta, tb, mode, l)
-  RG_TILE(128, 128, 16, 2, 2);
-  RG_TILE(128, 64, 16, 2, 2);
-  RG_TILE(128, 64, 32, 2, 4);
-  RG_TILE(64, 128, 32, 2, 2);
-  RG_TILE(64, 64, 32, 2, 2);
-  RG_TILE(128, 32, 32, 4, 1);
-  RG_TILE(32, 128, 32, 1, 4);
-  RG_TILE(32, 32, 32, 2, 2);
+#define RG_TILE(BM_, BN_, WM_, WN_, SPLIT_)                                                        \
+  if (t.bm == BM_ && t.bn == BN_ && t.wm == WM_ && t.wn == WN_ && t.bk == 32 && t.split == SPLIT_) \
+  return launch_flags<BM_, BN_, WM_, WN_, SPLIT_>(s, ta, tb, mode, l)
+  RG_TILE(128, 128, 2, 4, true);
+  RG_TILE(128, 64, 2, 2, true);
+  RG_TILE(64, 64, 2, 2, true);
+  RG_TILE(64, 64, 2, 2, false);
+  RG_TILE(128, 32, 4, 1, false);
+  RG_TILE(32, 128, 1, 4, false);
+  RG_TILE(32, 32, 2, 2, false);
 #undef RG_TILE
+  throw std::runtime_error("product tile without a kernel");
 }
 
 }  // namespace
@@ -650,18 +687,13 @@ bool gemm_epilogue_tile(int dtype, uint64_t m, uint64_t n, uint64_t k, bool ta, 
   if (m == 0 || n == 0 || m >= (1ull << 31) || n >= (1ull << 31) || k >= (1ull << 31)) return false;
   if (skinny_plan(dtype, m, n, k, 1, ta, tb).kind != SKINNY_NONE || !use_mfma(dtype, m, n, k)) return false;
   TileCfg t = pick_tile(m, n, k, 1);
+  if (!t.split || split_count(t, m, n, k, 1) != 1) return false;
   // Short K: 128x64 tiles rather than 128x128, twice the blocks, so that the second round's
-  // products run while the first round's epilogues read and write (C4's GELU backward: 3 % off
-  // the combined kernels on MI355X, results unchanged).
-  if (t.bm == 128 && t.bn == 128 && k <= 1024) t = TileCfg{128, 64, 16, 2, 2};
-  if (split_count(t, m, n, k, 1) != 1) return false;
-  // Runs of adjacent output columns per lane: four with a K-contiguous B (the transposed product
-  // form); with an N-contiguous B one per tile the wave holds across N, which must be two or four.
-  if (!tb && (t.bn / t.wn) / t.ms != 4 && (t.bn / t.wn) / t.ms != 2) return false;
-  const bool vec = k % 4 == 0 && (!ta || m % 4 == 0) && (tb || n % 4 == 0) && n % 4 == 0;
-  if (!vec) return false;
-  const bool even = m % t.bm == 0 && n % t.bn == 0 && k % t.bk == 0;
-  *out = GemmTile{t.bm, t.bn, t.bk, t.wm, t.wn, t.ms, even ? LOAD_EVEN : LOAD_VEC, (int)((k + t.bk - 1) / t.bk * t.bk),
+  // products run while the first round's epilogues read and write.
+  if (t.bm == 128 && t.bn == 128 && k <= 1024) t = SPLIT_128x64;
+  // The epilogue's loads and stores are aligned vectors of four columns.
+  if (n % 4 != 0) return false;
+  *out = GemmTile{t.bm, t.bn, t.wm, t.wn, k % SPLIT_BK != 0, m % t.bm == 0 && n % t.bn == 0, (int)((k + t.bk - 1) / t.bk * t.bk),
                   (uint32_t)((m + t.bm - 1) / t.bm), (uint32_t)((n + t.bn - 1) / t.bn)};
   return true;
 }
@@ -752,10 +784,8 @@ bool gemm_skinny(hipStream_t s, const GemmArgs& g, const Skinny& sk) {
 
 namespace {
 
-// The MFMA tile launch of product `g`: its tile, load mode and launch arguments.
-void mfma_launch(const GemmArgs& g, TileCfg* tile, int* load_mode, Launch* launch) {
-  TileCfg t = pick_tile(g.m, g.n, g.k, g.batch);
-  int splits = split_count(t, g.m, g.n, g.k, g.batch);
+// The MFMA tile launch of product `g` on tile `t` with `splits` K splits: its load mode and launch arguments.
+void mfma_launch(const GemmArgs& g, const TileCfg& t, int splits, int* load_mode, Launch* launch) {
   int kps = (int)(((g.k + splits - 1) / splits + t.bk - 1) / t.bk * t.bk);
   splits = (int)((g.k + kps - 1) / kps);
   if (g.defer_split && splits != g.planned_splits)
@@ -767,7 +797,7 @@ void mfma_launch(const GemmArgs& g, TileCfg* tile, int* load_mode, Launch* launc
   bool vec = aligned(g.a) && aligned(g.b) && g.k % 4 == 0 && (!g.ta || g.m % 4 == 0) && (g.tb || g.n % 4 == 0) &&
              (g.a_off ? g.a_off4 : g.a_stride % 4 == 0) && (g.b_off ? g.b_off4 : g.b_stride % 4 == 0);
   bool even = g.m % t.bm == 0 && g.n % t.bn == 0 && g.k % t.bk == 0 && kps % t.bk == 0;
-  int mode = !vec ? LOAD_SCALAR : even ? LOAD_EVEN : LOAD_VEC;
+  int mode = t.split ? (g.k % SPLIT_BK != 0) : !vec ? LOAD_SCALAR : even ? LOAD_EVEN : LOAD_VEC;
   Launch l;
   l.tm = (uint32_t)((g.m + t.bm - 1) / t.bm);
   l.tn = (uint32_t)((g.n + t.bn - 1) / t.bn);
@@ -786,7 +816,6 @@ void mfma_launch(const GemmArgs& g, TileCfg* tile, int* load_mode, Launch* launc
   l.kps = kps;
   l.part = splits > 1 ? (float*)g.workspace : nullptr;
   l.bias = splits > 1 ? nullptr : (const float*)g.bias;
-  *tile = t;
   *load_mode = mode;
   *launch = l;
 }
@@ -812,10 +841,10 @@ void gemm(hipStream_t s, const GemmArgs& g) {
     if (g.defer_split) throw std::runtime_error("deferred K-split product: the streaming kernel refused its operands");
   }
   if (use_mfma(g.dtype, g.m, g.n, g.k)) {
-    TileCfg t;
+    const TileCfg t = pick_tile(g.m, g.n, g.k, g.batch);
     int mode;
     Launch l;
-    mfma_launch(g, &t, &mode, &l);
+    mfma_launch(g, t, split_count(t, g.m, g.n, g.k, g.batch), &mode, &l);
     const int splits = l.splits;
     launch_mfma(s, t, g.ta, g.tb, mode, l);
     if (splits > 1 && !g.defer_split) {
@@ -920,32 +949,31 @@ bool gemm_group(hipStream_t s, const GemmArgs* g, int count, bool launch) {
       return true;
     }
   }
-  TileCfg t[GROUP_MAX];
-  int mode[GROUP_MAX];
+  // One split tile for all, 128x128: every split tile sums a K range's terms in the same order, so a
+  // product picked for a smaller one keeps its bits, and its K splits. K-split partials, if any, must
+  // be the deferred kind: a split sum after the grouped launch would be a second launch anyway.
+  const TileCfg t = SPLIT_128x128;
+  int mode;
   Launch l[GROUP_MAX];
   int flags = 0;
+  bool small = false, large = false;  // weight gradients of fewer than 256 blocks, and of more
   for (int i = 0; i < count; i++) {
-    if (!on_mfma_tiles(g[i]) || g[i].batch != 1) return false;
-    mfma_launch(g[i], &t[i], &mode[i], &l[i]);
-    // K-split partials, if any, must be the deferred kind: a split sum after the grouped launch
-    // would be a second launch anyway.
-    if (l[i].splits > 1 && !g[i].defer_split) return false;
-    if (mode[i] != LOAD_EVEN || t[i].bm != t[0].bm || t[i].bn != t[0].bn || t[i].bk != t[0].bk || t[i].wm != t[0].wm ||
-        t[i].wn != t[0].wn || t[i].ms != 16 || (i + 1 < count && l[i].grid.x % 8 != 0))
-      return false;
+    if (!on_mfma_tiles(g[i]) || g[i].batch != 1 || g[i].m % t.bm || g[i].n % t.bn) return false;
+    const TileCfg own = pick_tile(g[i].m, g[i].n, g[i].k, 1);
+    const int own_splits = split_count(own, g[i].m, g[i].n, g[i].k, 1);
+    if (!own.split || (own_splits > 1 && !g[i].defer_split)) return false;
+    mfma_launch(g[i], t, own_splits, &mode, &l[i]);
+    if (mode != 0 || (i + 1 < count && l[i].grid.x % 8 != 0)) return false;
     flags |= ((g[i].ta ? 2 : 0) | (g[i].tb ? 1 : 0)) << (2 * i);
+    (g[i].ta && !g[i].tb && l[i].grid.x < 256 ? small : large) |= g[i].ta;
   }
-  // The shapes and flag sequences instantiated, from C4's backward pass: on 128x64 tiles of
-  // eight waves, fc1's input and weight gradients as a pair, with fc2's weight gradient ahead of
-  // them as a triple; on 64x64 tiles of four waves, the attention projection's weight gradient
-  // with the q, k, v projection's.
+  // The flag sequences instantiated, from C4's backward pass: fc1's input and weight gradients as a
+  // pair, with fc2's weight gradient ahead of them as a triple; and the attention projection's
+  // weight gradient with the q, k, v projection's, which do not fill the chip alone (64 and 192
+  // blocks) and so go together rather than each with its input gradient.
+  if (small && (large || flags != (2 | 2 << 2))) return false;
   constexpr int T = 2, N = 1;  // (ta, tb) = (true, false) and (false, true)
-  const bool wide = t[0].bm == 128 && t[0].bn == 64 && t[0].bk == 32 && t[0].wm == 2 && t[0].wn == 4;
-  const bool small = t[0].bm == 64 && t[0].bn == 64 && t[0].bk == 32 && t[0].wm == 2 && t[0].wn == 2;
-  const bool known = (wide && ((count == 2 && (flags == (N | T << 2) || flags == (T | N << 2))) ||
-                               (count == 3 && flags == (T | N << 2 | T << 4)))) ||
-                     (small && count == 2 && flags == (T | T << 2));
-  if (!launch || !known) return known;
+  const dim3 block(64 * t.wm * t.wn);
   GroupParts parts{};
   uint32_t blocks = 0;
   for (int i = 0; i < count; i++) {
@@ -953,16 +981,17 @@ bool gemm_group(hipStream_t s, const GemmArgs* g, int count, bool launch) {
                            l[i].grid.x};
     blocks += l[i].grid.x;
   }
-  const dim3 grid(blocks);
-  if (small)
-    hipLaunchKernelGGL((k_gemm_mfma_group<64, 64, 32, 2, 2, 2, T | T << 2>), grid, dim3(256), 0, s, parts);
-  else if (count == 2 && flags == (N | T << 2))
-    hipLaunchKernelGGL((k_gemm_mfma_group<128, 64, 32, 2, 4, 2, N | T << 2>), grid, dim3(512), 0, s, parts);
-  else if (count == 2)
-    hipLaunchKernelGGL((k_gemm_mfma_group<128, 64, 32, 2, 4, 2, T | N << 2>), grid, dim3(512), 0, s, parts);
-  else
-    hipLaunchKernelGGL((k_gemm_mfma_group<128, 64, 32, 2, 4, 3, T | N << 2 | T << 4>), grid, dim3(512), 0, s, parts);
-  return true;
+#define RG_GROUP(COUNT_, FLAGS_)                                                                                      \
+  if (count == COUNT_ && flags == (FLAGS_)) {                                                                         \
+    if (launch) hipLaunchKernelGGL((k_gemm_mfma_group<128, 128, 2, 4, COUNT_, FLAGS_>), dim3(blocks), block, 0, s, parts); \
+    return true;                                                                                                      \
+  }
+  RG_GROUP(2, N | T << 2)
+  RG_GROUP(2, T | N << 2)
+  RG_GROUP(2, T | T << 2)
+  RG_GROUP(3, T | N << 2 | T << 4)
+#undef RG_GROUP
+  return false;
 }
 
 }  // namespace rgk

@@ -1,53 +1,11 @@
-// The fp32 MFMA product tile (`gemm_mfma_block`) and what it is built from, shared by the
-// precompiled product kernels (gemm.hip, where every tile shape and the plain epilogue are
-// instantiated) and by the JIT-compiled products whose epilogue applies the elementwise group
-// that reads the product (jit.cpp: the same tile, the group's operations applied to each finished
-// output before it is stored). Self-contained device code: no includes, so that hiprtc can
-// compile it from its text (rg_gemm_mfma_source).
+// The fp32 MFMA product tile (`gemm_f32_tile`), for products of too few tiles to fill the chip: a
+// block is then alone on its CU, and the split tile's (gemm_split.h) conversions and second barrier
+// lengthen each of its K steps (256 x 768 x 256: 4.3 us on 32x32 tiles here, 7.1 there).
 #pragma once
 
+#include "gemm_split.h"
+
 namespace rgg {
-
-#if defined(__HIPCC_RTC__)
-// hiprtc declares the fixed-width integer types in its own namespace.
-typedef __hip_internal::int64_t int64_t;
-typedef __hip_internal::uint64_t uint64_t;
-typedef __hip_internal::uint32_t uint32_t;
-#endif
-
-template <int V>
-struct IC {
-  static constexpr int value = V;
-};
-
-typedef float floatx2 __attribute__((ext_vector_type(2)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ int64_t batch_offset(const int64_t* offs, uint64_t stride, uint32_t b) {
-  return offs ? offs[b] : (int64_t)(stride * b);
-}
-
-// Which output tile a block computes. The dispatcher deals consecutive blocks round-robin over
-// the 8 XCDs, each with its own L2; with `swizzle`, XCD x instead receives the contiguous run
-// x*nb/8 ... (x+1)*nb/8 - 1 of tiles, and within a batch the tiles run in groups of 8 M-panels
-// per N sweep, so blocks resident on one XCD share their A and B panels in its L2.
-struct TileIndex {
-  uint32_t tm, tn, z;
-};
-
-// Block `bid` of a product launched as `nb` blocks (its share of the grid).
-__device__ __forceinline__ TileIndex tile_of(uint32_t bid, uint32_t nb, uint32_t tiles_m, uint32_t tiles_n, int swizzle) {
-  uint32_t per_batch = tiles_m * tiles_n;
-  if (!swizzle) return {(bid % per_batch) / tiles_n, bid % tiles_n, bid / per_batch};
-  uint32_t lid = (nb % 8 == 0) ? (bid % 8) * (nb / 8) + bid / 8 : bid;
-  uint32_t z = lid / per_batch, t = lid % per_batch;
-  constexpr uint32_t GROUP = 8;
-  uint32_t span = GROUP * tiles_n;
-  uint32_t first = (t / span) * GROUP;
-  uint32_t rows = min(tiles_m - first, GROUP);
-  uint32_t in = t % span;
-  return {first + in % rows, in / rows, z};
-}
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
@@ -130,25 +88,6 @@ __device__ __forceinline__ void lds_read(const float* p, float* v) {
 // TM x TN MFMA tiles of 16x16. The grid is one-dimensional: tiles_m * tiles_n * batch * splits
 // blocks (tile_of); split `sp` covers K range [sp * k_per_split, (sp + 1) * k_per_split).
 
-// The plain epilogue: each finished output (flat index `e` within the block's output matrix) is
-// stored into C, or into the block's split of the K-split partials. Non-temporal stores: every
-// block writes its whole tile at the end, all at once; written past the L2 they leave less for the
-// end of the kernel to write back (4-10 % off C4's products with 1024- and 768-wide outputs on
-// MI355X, results unchanged).
-struct StoreC {
-  float* C;
-  float* partial;
-  int splits;
-  uint64_t mn;
-  float* out = nullptr;
-  __device__ __forceinline__ void begin(uint32_t b, uint32_t sp) {
-    out = splits > 1 ? partial + ((uint64_t)b * splits + sp) * mn : C + (uint64_t)b * mn;
-  }
-  __device__ __forceinline__ void put4(uint64_t e, float4 v, int) { __builtin_nontemporal_store(floatx4{v.x, v.y, v.z, v.w}, (floatx4*)(out + e)); }
-  __device__ __forceinline__ void put2(uint64_t e, float2 v) { __builtin_nontemporal_store(floatx2{v.x, v.y}, (floatx2*)(out + e)); }
-  __device__ __forceinline__ void put1(uint64_t e, float v) { __builtin_nontemporal_store(v, out + e); }
-};
-
 // LDS of one tile: two buffers of each operand's K step, in the operand's own layout (rows padded
 // by 4 floats where K is contiguous).
 template <int BM, int BN, int BK, bool TA, bool TB>
@@ -162,7 +101,7 @@ struct TileLds {
 // TileLds<...>::FLOATS floats of LDS): a kernel that runs two products side by side gives each
 // its share of the grid and the same LDS.
 template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB, int MODE, int MS, class Epi>
-__device__ __forceinline__ void gemm_mfma_tile(const float* __restrict__ A, const float* __restrict__ B, int M, int N, int K,
+__device__ __forceinline__ void gemm_f32_tile(const float* __restrict__ A, const float* __restrict__ B, int M, int N, int K,
                                                const int64_t* a_off, const int64_t* b_off, uint64_t a_stride, uint64_t b_stride, int splits,
                                                int k_per_split, const float* __restrict__ bias, uint32_t tiles_m, uint32_t tiles_n,
                                                int swizzle, Epi& epi, uint32_t bid, uint32_t nb, float* smem) {
@@ -370,12 +309,12 @@ __device__ __forceinline__ void gemm_mfma_tile(const float* __restrict__ A, cons
 
 // One product over the whole grid, with its own LDS.
 template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB, int MODE, int MS, class Epi>
-__device__ __forceinline__ void gemm_mfma_block(const float* __restrict__ A, const float* __restrict__ B, int M, int N, int K,
+__device__ __forceinline__ void gemm_f32_block(const float* __restrict__ A, const float* __restrict__ B, int M, int N, int K,
                                                 const int64_t* a_off, const int64_t* b_off, uint64_t a_stride, uint64_t b_stride, int splits,
                                                 int k_per_split, const float* __restrict__ bias, uint32_t tiles_m, uint32_t tiles_n,
                                                 int swizzle, Epi& epi) {
   __shared__ float smem[TileLds<BM, BN, BK, TA, TB>::FLOATS];
-  gemm_mfma_tile<BM, BN, BK, WM, WN, TA, TB, MODE, MS>(A, B, M, N, K, a_off, b_off, a_stride, b_stride, splits, k_per_split, bias, tiles_m,
+  gemm_f32_tile<BM, BN, BK, WM, WN, TA, TB, MODE, MS>(A, B, M, N, K, a_off, b_off, a_stride, b_stride, splits, k_per_split, bias, tiles_m,
                                                       tiles_n, swizzle, epi, blockIdx.x, gridDim.x, smem);
 }
 

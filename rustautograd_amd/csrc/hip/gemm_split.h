@@ -1,0 +1,383 @@
+// The fp32 product tile on the bf16 matrix cores (`gemm_mfma_block`), shared by the precompiled
+// product kernels (gemm.hip) and by the JIT-compiled products whose epilogue applies the
+// elementwise group that reads the product (jit.cpp). Self-contained device code: no includes, so
+// that hiprtc can compile it from its text (rg_gemm_split_source).
+//
+// Every fp32 operand value is split exactly into three bf16 values, each the rounding of what the
+// ones before it left (8 bits of the 24 each): x = x1 + x2 + x3. A product is the sum of the six
+// terms a1 b1, a1 b2, a2 b1, a2 b2, a1 b3 and a3 b1; what is left out, a2 b3 + a3 b2 + a3 b3, is at
+// most 2^-25 of it, half an fp32 rounding. v_mfma_f32_16x16x32_bf16 sums a lane's eight exact terms
+// on the largest one's scale (bits below 2^-24 of it cut off) and adds the four lanes' sums to the
+// accumulator one after the other, each addition rounded, with a small bias downwards. So the terms
+// of one K step of 32 are summed from zero, small terms first, and the step's sum is added to the
+// running one by an ordinary addition: the MFMA's roundings are then on the scale of one step. Odd
+// steps form the sum of a (-b) and subtract it, which turns their bias the other way (without that
+// it made up a quarter of the error at K = 5000 and showed in sums over a gradient's rows). Against
+// 64-bit sums the relative error is 0.25-0.3 of the fp32 MFMA tile's for K = 256 to 8192 (normal
+// operands, 2048: 1.8e-7 against 7.9e-7). bf16 has fp32's exponent range; only operand values below
+// 2^-109 lose low bits of x3 (or x2) to its underflow.
+// A value that is not finite, or that rounds past the largest bf16 value, leaves NaN in every sum
+// it enters, so a wave that ends with a sum that is not finite forms its outputs again with fp32
+// MFMAs straight from memory: such outputs are the fp32 tile's.
+//
+// What bounds it: six bf16 terms at 2.5 PFLOP/s are 417 TFLOP/s of fp32 products against 157 on the
+// fp32 MFMA; a large bf16 product of the vendor library reaches 1.2 PFLOP/s on this chip, a sixth of
+// which is 201. This tile reaches 188-198 at 4096 x 2048 x 2048 (the fp32 tile: 127) and 130-160 at
+// K = 256 to 1024, where the launch, the first loads and the stores weigh (the fp32 tile: 90-107).
+#pragma once
+
+namespace rgg {
+
+#if defined(__HIPCC_RTC__)
+// hiprtc declares the fixed-width integer types in its own namespace.
+typedef __hip_internal::int64_t int64_t;
+typedef __hip_internal::uint64_t uint64_t;
+typedef __hip_internal::uint32_t uint32_t;
+#endif
+
+template <int V>
+struct IC {
+  static constexpr int value = V;
+};
+
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float rowx2 __attribute__((ext_vector_type(2), aligned(4)));
+typedef float rowx4 __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ int64_t batch_offset(const int64_t* offs, uint64_t stride, uint32_t b) {
+  return offs ? offs[b] : (int64_t)(stride * b);
+}
+
+// Which output tile a block computes. The dispatcher deals consecutive blocks round-robin over
+// the 8 XCDs, each with its own L2; with `swizzle`, XCD x instead receives the contiguous run
+// x*nb/8 ... (x+1)*nb/8 - 1 of tiles, and within a batch the tiles run in groups of 8 M-panels
+// per N sweep, so blocks resident on one XCD share their A and B panels in its L2.
+struct TileIndex {
+  uint32_t tm, tn, z;
+};
+
+// Block `bid` of a product launched as `nb` blocks (its share of the grid).
+__device__ __forceinline__ TileIndex tile_of(uint32_t bid, uint32_t nb, uint32_t tiles_m, uint32_t tiles_n, int swizzle) {
+  uint32_t per_batch = tiles_m * tiles_n;
+  if (!swizzle) return {(bid % per_batch) / tiles_n, bid % tiles_n, bid / per_batch};
+  uint32_t lid = (nb % 8 == 0) ? (bid % 8) * (nb / 8) + bid / 8 : bid;
+  uint32_t z = lid / per_batch, t = lid % per_batch;
+  constexpr uint32_t GROUP = 8;
+  uint32_t span = GROUP * tiles_n;
+  uint32_t first = (t / span) * GROUP;
+  uint32_t rows = min(tiles_m - first, GROUP);
+  uint32_t in = t % span;
+  return {first + in % rows, in / rows, z};
+}
+
+// The plain epilogue: each finished output (flat index `e` within the block's output matrix) is
+// stored into C, or into the block's split of the K-split partials. Non-temporal stores: every
+// block writes its whole tile at the end, all at once; written past the L2 they leave less for the
+// end of the kernel to write back (4-10 % off C4's products with 1024- and 768-wide outputs on
+// MI355X, results unchanged). Rows of C need only 4-byte alignment.
+struct StoreC {
+  float* C;
+  float* partial;
+  int splits;
+  uint64_t mn;
+  float* out = nullptr;
+  __device__ __forceinline__ void begin(uint32_t b, uint32_t sp) {
+    out = splits > 1 ? partial + ((uint64_t)b * splits + sp) * mn : C + (uint64_t)b * mn;
+  }
+  __device__ __forceinline__ void put4(uint64_t e, float4 v, int) { __builtin_nontemporal_store(rowx4{v.x, v.y, v.z, v.w}, (rowx4*)(out + e)); }
+  __device__ __forceinline__ void put2(uint64_t e, float2 v) { __builtin_nontemporal_store(floatx2{v.x, v.y}, (floatx2*)(out + e)); }
+  __device__ __forceinline__ void put1(uint64_t e, float v) { __builtin_nontemporal_store(v, out + e); }
+};
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t cell __attribute__((ext_vector_type(4)));  // eight bf16 values: one row's or column's next 8 k
+
+// Two values' three bf16 parts, packed in pairs.
+__device__ __forceinline__ uint32_t pack_bf16(float x0, float x1) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2{x0, x1}), bf16x2));
+}
+__device__ __forceinline__ void split_bf16(float x0, float x1, uint32_t& p1, uint32_t& p2, uint32_t& p3) {
+  p1 = pack_bf16(x0, x1);
+  const float r0 = x0 - __builtin_bit_cast(float, p1 << 16), r1 = x1 - __builtin_bit_cast(float, p1 & 0xffff0000u);
+  p2 = pack_bf16(r0, r1);
+  const float s0 = r0 - __builtin_bit_cast(float, p2 << 16), s1 = r1 - __builtin_bit_cast(float, p2 & 0xffff0000u);
+  p3 = pack_bf16(s0, s1);
+}
+
+constexpr int SPLIT_BK = 32;  // K step
+
+// Layout of R rows (or columns) x 32 k of one operand in LDS: three planes of cells (16 bytes,
+// eight consecutive k), [k / 8][row], the k / 8 groups two cells further apart than R so that the
+// stores of a K-contiguous operand (four lanes per row) spread over all banks; the MFMA's reads are
+// 16 consecutive rows of one group. NT threads stage it, each thread taking units of 8 k for VN
+// adjacent columns (K-contiguous: one row), VN chosen so that every thread has one.
+template <int R, bool KC, int NT>
+struct SplitGeo {
+  static constexpr int VN = KC ? 1 : (R * 4 / NT >= 2 ? 2 : 1);
+  static constexpr int UNITS = R / VN * 4, PER = UNITS / NT;
+  static_assert(UNITS % NT == 0, "whole units per thread");
+  static constexpr int GROUP = R + 2, PLANE = 4 * GROUP, CELLS = 3 * PLANE;
+  // Two adjacent columns of one thread trade places in every second eight, so that eight lanes'
+  // stores of their first (or second) column reach eight different banks.
+  static __device__ __forceinline__ int place(int r) { return VN == 1 ? r : r ^ ((r >> 3) & 1); }
+};
+
+template <int R, bool KC, int NT>
+struct SplitStage {
+  typedef SplitGeo<R, KC, NT> G;
+  float v[G::PER][G::VN][8];
+  // The R x 32 tile at `base` (its first row or column, k = 0) and k0. Every row or column lies
+  // inside the operand; with `partial` the tile's k reach past `kend` and are zeros there. Loads
+  // need only 4-byte alignment. A column's eight k share one 32-bit offset (rows of the operand
+  // have less than 2^25 columns), each k its own scalar base.
+  __device__ __forceinline__ void load(const float* base, int64_t ld, int k0, int kend, bool partial, int tid) {
+#pragma unroll
+    for (int q = 0; q < G::PER; q++) {
+      const int u = q * NT + tid;
+      if constexpr (KC) {
+        const int64_t off = (int64_t)(u >> 2) * ld + (u & 3) * 8;
+        if (!partial) {
+          const float* p = base + off + k0;
+          const rowx4 x = *(const rowx4*)p, y = *(const rowx4*)(p + 4);
+#pragma unroll
+          for (int e = 0; e < 4; e++) v[q][0][e] = x[e], v[q][0][4 + e] = y[e];
+        } else {
+          const int k = k0 + (u & 3) * 8;
+          const float* row = base + (int64_t)(u >> 2) * ld;
+#pragma unroll
+          for (int e = 0; e < 8; e++) {
+            const float x = row[min(k + e, kend - 1)];
+            v[q][0][e] = k + e < kend ? x : 0.0f;
+          }
+        }
+      } else {
+        constexpr int W = R / G::VN;
+        const int g = u / W, c = (u % W) * G::VN;
+        if (!partial) {
+          const uint32_t off = ((uint32_t)g * 8 * (uint32_t)ld + (uint32_t)c) * 4;
+#pragma unroll
+          for (int e = 0; e < 8; e++) {
+            const char* p = (const char*)(base + (int64_t)(k0 + e) * ld) + off;
+            if constexpr (G::VN == 1) {
+              v[q][0][e] = *(const float*)p;
+            } else {
+              const rowx2 x = *(const rowx2*)p;
+              v[q][0][e] = x[0], v[q][1][e] = x[1];
+            }
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; e++) {
+            const int k = k0 + g * 8 + e;
+            const float* p = base + (int64_t)min(k, kend - 1) * ld + c;
+#pragma unroll
+            for (int j = 0; j < G::VN; j++) {
+              const float x = p[j];
+              v[q][j][e] = k < kend ? x : 0.0f;
+            }
+          }
+        }
+      }
+    }
+  }
+  // `sign` (1 or -1) times the staged values, split, into LDS.
+  template <bool SIGNED>
+  __device__ __forceinline__ void store(cell* lds, int tid, float sign) const {
+#pragma unroll
+    for (int q = 0; q < G::PER; q++) {
+      const int u = q * NT + tid;
+      constexpr int W = R / G::VN;
+      const int g = KC ? u & 3 : u / W, r = KC ? u >> 2 : (u % W) * G::VN;
+#pragma unroll
+      for (int j = 0; j < G::VN; j++) {
+        cell p1, p2, p3;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          uint32_t x1, x2, x3;
+          const float x = v[q][j][2 * e], y = v[q][j][2 * e + 1];
+          split_bf16(SIGNED ? x * sign : x, SIGNED ? y * sign : y, x1, x2, x3);
+          p1[e] = x1, p2[e] = x2, p3[e] = x3;
+        }
+        cell* d = lds + g * G::GROUP + G::place(r + j);
+        d[0] = p1, d[G::PLANE] = p2, d[2 * G::PLANE] = p3;
+      }
+    }
+  }
+};
+
+template <int BM, int BN, int WM, int WN, bool TA, bool TB>
+struct SplitLds {
+  static constexpr int CELLS = SplitGeo<BM, !TA, 64 * WM * WN>::CELLS + SplitGeo<BN, TB, 64 * WM * WN>::CELLS;
+};
+
+// C = op(A) op(B), the BM x BN tile of block `bid` of a product launched as `nb` blocks, staged
+// through `smem` (SplitLds<...>::CELLS cells): WM x WN wave64s, each owning (BM/WM) x (BN/WN) as
+// 16x16 MFMA tiles. M >= BM and N >= BN: the last tile along an edge that BM or BN does not divide
+// is moved inwards, so that no load of a row or column is out of range, and stores only what the
+// tile before it does not. Split `sp` covers K range [sp * k_per_split, (sp + 1) * k_per_split), a
+// multiple of 32 long except the last; TAIL: some range is not a multiple of 32.
+//
+// One LDS buffer: the next tile's values wait in registers while this one is multiplied, are
+// converted and stored between two barriers, and the loads after them go out at once. Two or three
+// blocks share a CU, so that one's conversions run beside another's MFMAs (two LDS buffers and one
+// barrier per step, at half the blocks per CU, measured 3-6 % slower at 4096 x 2048 x 2048).
+// The product is formed transposed (B supplies the MFMA rows), so that each lane holds runs of
+// four adjacent output columns: put4's third argument names the run (the same for every row the
+// lane stores), so that an epilogue can keep per-column sums in registers.
+template <int BM, int BN, int WM, int WN, bool TA, bool TB, bool TAIL, class Epi>
+__device__ __forceinline__ void gemm_split_tile(const float* __restrict__ A, const float* __restrict__ B, int M, int N, int K,
+                                                const int64_t* a_off, const int64_t* b_off, uint64_t a_stride, uint64_t b_stride, int splits,
+                                                int k_per_split, const float* __restrict__ bias, uint32_t tiles_m, uint32_t tiles_n, Epi& epi,
+                                                uint32_t bid, uint32_t nb, cell* smem) {
+  constexpr int NT = 64 * WM * WN;
+  constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 16, TN = WTN / 16;
+  typedef SplitGeo<BM, !TA, NT> GA;
+  typedef SplitGeo<BN, TB, NT> GB;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave / WN, wn = wave % WN, li = lane & 15, lo = lane >> 4;
+  const TileIndex ti = tile_of(bid, nb, tiles_m, tiles_n, 1);
+  const uint32_t b = ti.z / splits, sp = ti.z % splits;
+  const int m_first = ti.tm * BM, n_first = ti.tn * BN, m0 = min(m_first, M - BM), n0 = min(n_first, N - BN);
+  const int64_t lda = TA ? M : K, ldb = TB ? K : N;
+  const float* Ab = A + batch_offset(a_off, a_stride, b) + (TA ? (int64_t)m0 : (int64_t)m0 * K);
+  const float* Bb = B + batch_offset(b_off, b_stride, b) + (TB ? (int64_t)n0 * K : (int64_t)n0);
+  const int kbeg = sp * k_per_split, kend = min(K, kbeg + k_per_split);
+  const int nk = (kend - kbeg + SPLIT_BK - 1) / SPLIT_BK;
+  SplitStage<BM, !TA, NT> sa;
+  SplitStage<BN, TB, NT> sb;
+  auto load = [&](int t) __attribute__((always_inline)) {
+    const int k0 = kbeg + t * SPLIT_BK;
+    const bool partial = TAIL && k0 + SPLIT_BK > kend;
+    sa.load(Ab, lda, k0, kend, partial, tid);
+    sb.load(Bb, ldb, k0, kend, partial, tid);
+  };
+  // Odd steps' B is stored negated, and their sums subtracted (multiply's sign).
+  auto store = [&](float sign) __attribute__((always_inline)) {
+    sa.template store<false>(smem, tid, 1.0f);
+    sb.template store<true>(smem + GA::CELLS, tid, sign);
+  };
+  floatx4 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int n = 0; n < TN; n++) acc[i][n] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  auto multiply = [&](float sign) __attribute__((always_inline)) {
+    const cell* as = smem + lo * GA::GROUP;
+    const cell* bs = smem + GA::CELLS + lo * GB::GROUP;
+    bf16x8 y[3][TN];
+#pragma unroll
+    for (int p = 0; p < 3; p++)
+#pragma unroll
+      for (int n = 0; n < TN; n++) y[p][n] = __builtin_bit_cast(bf16x8, bs[p * GB::PLANE + GB::place(wn * WTN + n * 16 + li)]);
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+      bf16x8 x[3];
+#pragma unroll
+      for (int p = 0; p < 3; p++) x[p] = __builtin_bit_cast(bf16x8, as[p * GA::PLANE + GA::place(wm * WTM + i * 16 + li)]);
+      constexpr int PX[6] = {0, 2, 1, 0, 1, 0}, PY[6] = {2, 0, 1, 1, 0, 0};
+      floatx4 step[TN];
+#pragma unroll
+      for (int n = 0; n < TN; n++) step[n] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int q = 0; q < 6; q++)
+#pragma unroll
+        for (int n = 0; n < TN; n++) step[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(y[PY[q]][n], x[PX[q]], step[n], 0, 0, 0);
+#pragma unroll
+      for (int n = 0; n < TN; n++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[i][n][r] = __builtin_fmaf(step[n][r], sign, acc[i][n][r]);
+    }
+  };
+  load(0);
+  float sign = 1.0f;  // of the tile in LDS
+  store(sign);
+  if (nk > 1) load(1);
+  __syncthreads();
+  for (int t = 0; t < nk - 1; t++) {
+    multiply(sign);
+    __syncthreads();
+    sign = -sign;
+    store(sign);
+    if (t + 2 < nk) load(t + 2);
+    __syncthreads();
+  }
+  multiply(sign);
+  // Lane l of the wave's tile (i, n) holds output row 16 i + l % 16, columns 16 n + 4 (l / 16) .. + 3.
+  // A sum that is not finite: this wave's outputs again, in fp32.
+  float finite = 0.0f;  // NaN once any sum is infinite or NaN
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int n = 0; n < TN; n++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) finite = __builtin_fmaf(acc[i][n][r], 0.0f, finite);
+  if (__ballot(!(finite == 0.0f)) != 0) {
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int n = 0; n < TN; n++) acc[i][n] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+    for (int k0 = kbeg; k0 < kend; k0 += 4) {
+      const int k = min(k0 + lo, kend - 1);
+      const bool live = k0 + lo < kend;
+      float y[TN];
+#pragma unroll
+      for (int n = 0; n < TN; n++) {
+        const int64_t c = wn * WTN + n * 16 + li;
+        const float v = Bb[TB ? c * K + k : (int64_t)k * N + c];
+        y[n] = live ? v : 0.0f;
+      }
+#pragma unroll
+      for (int i = 0; i < TM; i++) {
+        const int64_t r = wm * WTM + i * 16 + li;
+        const float v = Ab[TA ? (int64_t)k * M + r : r * K + k];
+        const float x = live ? v : 0.0f;
+#pragma unroll
+        for (int n = 0; n < TN; n++) acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[n], x, acc[i][n], 0, 0, 0);
+      }
+    }
+  }
+  epi.begin(b, sp);
+  // A per-column bias (unsplit products only) added to the finished sums, as one fp32 addition.
+  if (bias) {
+#pragma unroll
+    for (int n = 0; n < TN; n++) {
+      const float* p = bias + n0 + wn * WTN + n * 16 + 4 * lo;
+      const floatx4 x = {p[0], p[1], p[2], p[3]};
+#pragma unroll
+      for (int i = 0; i < TM; i++) acc[i][n] = acc[i][n] + x;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < TM; i++) {
+    const int row = m0 + wm * WTM + i * 16 + li;
+    if (row < m_first) continue;
+    const uint64_t erow = (uint64_t)row * N;
+#pragma unroll
+    for (int n = 0; n < TN; n++) {
+      const int col = n0 + wn * WTN + n * 16 + 4 * lo;
+      const floatx4 c = acc[i][n];
+      if (col >= n_first) {
+        epi.put4(erow + col, make_float4(c[0], c[1], c[2], c[3]), n);
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          if (col + r >= n_first) epi.put1(erow + col + r, c[r]);
+      }
+    }
+  }
+}
+
+// One product over the whole grid, with its own LDS.
+template <int BM, int BN, int WM, int WN, bool TA, bool TB, bool TAIL, class Epi>
+__device__ __forceinline__ void gemm_mfma_block(const float* __restrict__ A, const float* __restrict__ B, int M, int N, int K,
+                                                const int64_t* a_off, const int64_t* b_off, uint64_t a_stride, uint64_t b_stride, int splits,
+                                                int k_per_split, const float* __restrict__ bias, uint32_t tiles_m, uint32_t tiles_n, Epi& epi) {
+  __shared__ cell smem[SplitLds<BM, BN, WM, WN, TA, TB>::CELLS];
+  gemm_split_tile<BM, BN, WM, WN, TA, TB, TAIL>(A, B, M, N, K, a_off, b_off, a_stride, b_stride, splits, k_per_split, bias, tiles_m, tiles_n,
+                                                epi, blockIdx.x, gridDim.x, smem);
+}
+
+}  // namespace rgg

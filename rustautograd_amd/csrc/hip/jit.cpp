@@ -14,8 +14,8 @@
 
 namespace rgjit {
 
-// The text of gemm_mfma.h (generated at build time), for products compiled with an epilogue.
-extern const char* const rg_gemm_mfma_source;
+// The text of gemm_split.h (generated at build time), for products compiled with an epilogue.
+extern const char* const rg_gemm_split_source;
 
 namespace {
 
@@ -184,10 +184,9 @@ std::string generate_gemm(const rgplan::Fused& f, int64_t c_slot, bool store_c, 
                           FusedKernel* k, int col_sum) {
   if (f.dtype != RG_F32) throw std::runtime_error("product epilogue: fp32 groups only");
   const std::string E = name + "_epi";
-  // Column sums (col_sum >= 0): a K-contiguous B's transposed form, where each lane stores runs
-  // of four columns, the same runs for every row (put4's slot: tile n across N, register group).
-  const int slots = (t.bn / t.wn / t.ms) * (t.ms / 16) * (t.ms == 32 ? 4 : 1);
-  if (col_sum >= 0 && (!t.tb || t.ms != 16)) throw std::runtime_error("product epilogue column sums: needs a K-contiguous B and 16x16 tiles");
+  // Column sums (col_sum >= 0): each lane stores runs of four columns, the same runs for every row
+  // (put4's slot: tile n across N).
+  const int slots = t.bn / t.wn / 16;
   std::ostringstream s;
   s << "struct " << E << " {\n  float* c;\n";
   for (size_t j = 0; j < f.inputs.size(); j++) s << "  const float* in" << j << ";\n";
@@ -212,7 +211,6 @@ std::string generate_gemm(const rgplan::Fused& f, int64_t c_slot, bool store_c, 
         b << "    float " << x << "[" << W << "];\n";
         if (W == 4) b << "    { const float4 t = *(const float4*)(in" << j << " + " << at << "); " << x << "[0] = t.x; " << x << "[1] = t.y; " << x
                       << "[2] = t.z; " << x << "[3] = t.w; }\n";
-        else if (W == 2) b << "    { const float2 t = *(const float2*)(in" << j << " + " << at << "); " << x << "[0] = t.x; " << x << "[1] = t.y; }\n";
         else b << "    " << x << "[0] = in" << j << "[" << at << "];\n";
         in_expr[j] = x + "[v]";
       } else {
@@ -238,7 +236,6 @@ std::string generate_gemm(const rgplan::Fused& f, int64_t c_slot, bool store_c, 
     b << "    }\n";
     for (size_t j = 0; j < f.outputs.size(); j++) {
       if (W == 4) b << "    *(float4*)(out" << j << " + e) = make_float4(o" << j << "[0], o" << j << "[1], o" << j << "[2], o" << j << "[3]);\n";
-      else if (W == 2) b << "    *(float2*)(out" << j << " + e) = make_float2(o" << j << "[0], o" << j << "[1]);\n";
       else b << "    out" << j << "[e] = o" << j << "[0];\n";
     }
     return b.str();
@@ -255,9 +252,6 @@ std::string generate_gemm(const rgplan::Fused& f, int64_t c_slot, bool store_c, 
   s << "  __device__ __forceinline__ void put1(unsigned long long e, float acc) {\n";
   if (store_c) s << "    c[e] = acc;\n";
   s << "    const float a[1] = {acc};\n" << body(1) << "  }\n";
-  s << "  __device__ __forceinline__ void put2(unsigned long long e, float2 acc) {\n";
-  if (store_c) s << "    *(float2*)(c + e) = acc;\n";
-  s << "    const float a[2] = {acc.x, acc.y};\n" << body(2) << "  }\n";
   s << "};\n";
   const int nt = 64 * t.wm * t.wn;
   // At least two waves per SIMD (at most 256 registers a wave, far above what the tile uses): with
@@ -275,7 +269,7 @@ std::string generate_gemm(const rgplan::Fused& f, int64_t c_slot, bool store_c, 
   s << "extern \"C\" __global__ void __launch_bounds__(" << nt << ") __attribute__((amdgpu_waves_per_eu(2))) " << name
     << "(const float* __restrict__ A, const float* __restrict__ B, int M, int N, int K, const rgg::int64_t* a_off, const rgg::int64_t* b_off, "
        "rgg::uint64_t a_stride, rgg::uint64_t b_stride, int splits, int kps, const float* __restrict__ bias, rgg::uint32_t tiles_m, "
-       "rgg::uint32_t tiles_n, int swizzle, float* "
+       "rgg::uint32_t tiles_n, float* "
     << R << "c";
   for (size_t j = 0; j < f.inputs.size(); j++) s << ", const float* " << R << "in" << j;
   for (size_t j = 0; j < f.outputs.size(); j++) s << ", float* " << R << "out" << j;
@@ -285,9 +279,9 @@ std::string generate_gemm(const rgplan::Fused& f, int64_t c_slot, bool store_c, 
   for (size_t j = 0; j < f.outputs.size(); j++) s << ", out" << j;
   s << "};\n";
   if (col_sum >= 0) s << "  for (int q = 0; q < " << slots << "; q++) epi.colacc[q] = make_float4(0.f, 0.f, 0.f, 0.f);\n";
-  s << "  rgg::gemm_mfma_block<" << t.bm << ", " << t.bn << ", " << t.bk << ", " << t.wm << ", " << t.wn << ", " << (t.ta ? "true" : "false") << ", "
-    << (t.tb ? "true" : "false") << ", " << t.mode << ", " << t.ms
-    << ">(A, B, M, N, K, a_off, b_off, a_stride, b_stride, splits, kps, bias, tiles_m, tiles_n, swizzle, epi);\n";
+  s << "  rgg::gemm_mfma_block<" << t.bm << ", " << t.bn << ", " << t.wm << ", " << t.wn << ", " << (t.ta ? "true" : "false") << ", "
+    << (t.tb ? "true" : "false") << ", " << (t.tail ? "true" : "false")
+    << ">(A, B, M, N, K, a_off, b_off, a_stride, b_stride, splits, kps, bias, tiles_m, tiles_n, epi);\n";
   if (col_sum >= 0) {
     // The tile's column sums of output col_sum from the lanes' register sums (each lane summed
     // its rows in order): the 16 lanes holding the same columns combine by a fixed butterfly,
@@ -304,7 +298,7 @@ std::string generate_gemm(const rgplan::Fused& f, int64_t c_slot, bool store_c, 
     s << "      if ((lane & 15) == 0) *(float4*)&cs[wmi][wni * " << wtn << " + 16 * q + 4 * (lane >> 4)] = v;\n    }\n  }\n";
     s << "  __syncthreads();\n";
     s << "  if (threadIdx.x < " << t.bn << ") {\n";
-    s << "    const rgg::TileIndex ti = rgg::tile_of(blockIdx.x, gridDim.x, tiles_m, tiles_n, swizzle);\n";
+    s << "    const rgg::TileIndex ti = rgg::tile_of(blockIdx.x, gridDim.x, tiles_m, tiles_n, 1);\n";
     s << "    float v = cs[0][threadIdx.x];\n";
     s << "    for (int w = 1; w < " << t.wm << "; w++) v = v + cs[w][threadIdx.x];\n";
     s << "    colp[(rgg::uint64_t)ti.tm * N + ti.tn * " << t.bn << " + threadIdx.x] = v;\n  }\n";
@@ -673,7 +667,7 @@ std::map<std::string, hipModule_t> g_modules;
 
 std::vector<char> compile_code(const std::string& body) {
   std::string src = std::string(rg_ops_source) + "\n";
-  if (body.find("rgg::gemm_mfma_block") != std::string::npos) src += std::string(rg_gemm_mfma_source) + "\n";
+  if (body.find("rgg::gemm_mfma_block") != std::string::npos) src += std::string(rg_gemm_split_source) + "\n";
   src += body;
   hiprtcProgram prog;
   if (hiprtcCreateProgram(&prog, src.c_str(), "rg_fused.hip", 0, nullptr, nullptr) != HIPRTC_SUCCESS)

@@ -55,13 +55,13 @@ std::string generate_rows(const rgplan::Fused& f, const std::string& name, Fused
 
 // A product's tile for generate_gemm (the template arguments of rgg::gemm_mfma_block).
 struct ProductTile {
-  int bm, bn, bk, wm, wn, ms, mode;
-  bool ta, tb;
+  int bm, bn, wm, wn;
+  bool tail, ta, tb;
 };
 
 // Source of one product kernel whose epilogue computes fused group `f` (a plain fused group over
 // the product's M x N outputs, reading the product through `c_slot`) from each finished output
-// before it is stored: the tile of gemm_mfma.h with an epilogue that loads the group's other
+// before it is stored: the tile of gemm_split.h with an epilogue that loads the group's other
 // inputs at the output's position, applies its operations in its order (the values the plain
 // group kernel would compute) and stores its outputs, and the product itself when `store_c`.
 // The kernel's parameters are the tile kernel's, then the epilogue's pointers (product, the

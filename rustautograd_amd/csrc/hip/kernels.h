@@ -195,14 +195,13 @@ bool gemm_streamed(int dtype, uint64_t m, uint64_t n, uint64_t k, uint64_t batch
 int gemm_splits(int dtype, uint64_t m, uint64_t n, uint64_t k, uint64_t batch, bool ta, bool tb);
 uint64_t gemm_workspace(int dtype, uint64_t m, uint64_t n, uint64_t k, uint64_t batch, bool ta, bool tb);
 
-// The MFMA tile of a single (unbatched) fp32 product whose operands are 16-byte aligned, as plan
-// slots are, when it runs unsplit on the tile kernel and each lane's finished outputs come in
-// runs of two or four adjacent columns (the form an elementwise epilogue takes): the shape
-// arguments of the tile kernel (gemm_mfma.h). False for any other product. `mode` is the tile's
-// load mode, GEMM_WHOLE_TILES when M, N and K are multiples of the tile.
-constexpr int GEMM_WHOLE_TILES = 0;  // rgg::LOAD_EVEN
+// The split tile (gemm_split.h) of a single (unbatched) fp32 product with a multiple of four
+// columns, when it runs unsplit on that tile (the form an elementwise epilogue takes): its template
+// arguments. False for any other product. `whole`: M and N are multiples of the tile.
 struct GemmTile {
-  int bm, bn, bk, wm, wn, ms, mode, kps;
+  int bm, bn, wm, wn;
+  bool tail, whole;
+  int kps;
   uint32_t tm, tn;
 };
 bool gemm_epilogue_tile(int dtype, uint64_t m, uint64_t n, uint64_t k, bool ta, bool tb, GemmTile* t);

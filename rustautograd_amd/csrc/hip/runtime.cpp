@@ -717,21 +717,21 @@ StepFn lower_product_epilogue(const Instr& i, const rgplan::Fused& f, const rgji
     const void* A = sl[as];
     const void* B = sl[bs];
     const void* bias_p = bias >= 0 ? sl[bias] : nullptr;
-    int mm = M, nn = N, kk = K, splits = 1, kps = t.kps, swizzle = 1;
+    int mm = M, nn = N, kk = K, splits = 1, kps = t.kps;
     const void* a_off = nullptr;
     const void* b_off = nullptr;
     uint64_t a_stride = 0, b_stride = 0;
     uint32_t tm = t.tm, tn = t.tn;
     void* ptrs[129];
-    void* args[15 + 129] = {&A, &B, &mm, &nn, &kk, &a_off, &b_off, &a_stride, &b_stride, &splits, &kps, &bias_p, &tm, &tn, &swizzle};
+    void* args[14 + 129] = {&A, &B, &mm, &nn, &kk, &a_off, &b_off, &a_stride, &b_stride, &splits, &kps, &bias_p, &tm, &tn};
     size_t q = 0;
     for (; q < ptr_slots.size(); q++) {
       ptrs[q] = ptr_slots[q] >= 0 ? sl[ptr_slots[q]] : nullptr;
-      args[15 + q] = &ptrs[q];
+      args[14 + q] = &ptrs[q];
     }
     if (col_off >= 0) {  // the column sums' partial rows, in the fold area
       ptrs[q] = (char*)ws + pp->fold_base() + col_off;
-      args[15 + q] = &ptrs[q];
+      args[14 + q] = &ptrs[q];
     }
     hipModuleLaunchKernel(fk->fn, tm * tn, 1, 1, fk->block, 1, 1, 0, s, args, nullptr);
   };
@@ -933,10 +933,10 @@ Epilogues find_epilogues(const Plan& plan) {
       taken[(size_t)k] = true;
       // A column sum of one of the group's outputs a few steps later, with nothing between the
       // group and it overwriting that output: computed by the combined kernel from the values
-      // it stores, summed in registers (a K-contiguous B, whole 16x16-MFMA tiles: every output
-      // goes through put4). RG_HIP_EPILOGUE_SUMS=0 leaves it to its own kernel.
+      // it stores, summed in registers (a K-contiguous B, whole tiles: every output goes through
+      // put4). RG_HIP_EPILOGUE_SUMS=0 leaves it to its own kernel.
       const char* sums = getenv("RG_HIP_EPILOGUE_SUMS");
-      if ((sums && sums[0] == '0') || !tb || tile.ms != 16 || tile.mode != rgk::GEMM_WHOLE_TILES) break;
+      if ((sums && sums[0] == '0') || !tb || !tile.whole) break;
       for (size_t q = j + 1; q < n && q <= j + 4; q++) {
         if (steps[q].kind == RG_STEP_INSTR && is_control(steps[q].instr.op)) break;
         int out = -1;
@@ -976,7 +976,7 @@ std::string epilogue_source(const Plan& plan, size_t j, int64_t pk, const std::s
   rgk::GemmTile t;
   if (!flat_product(pi, &m, &nn, &kk, &ta, &tb) || !rgk::gemm_epilogue_tile(RG_F32, m, nn, kk, ta, tb, &t))
     throw std::runtime_error("product epilogue: the product does not fit a single tile kernel");
-  return rgjit::generate_gemm(plan.steps[j].fused, c, keep, rgjit::ProductTile{t.bm, t.bn, t.bk, t.wm, t.wn, t.ms, t.mode, ta, tb},
+  return rgjit::generate_gemm(plan.steps[j].fused, c, keep, rgjit::ProductTile{t.bm, t.bn, t.wm, t.wn, t.tail, ta, tb},
                               prefix + "rge" + std::to_string(pk), fk, col_sum);
 }
 
