@@ -48,20 +48,20 @@ __global__ void __launch_bounds__(64 * WM * WN) k_gemm_f32(const float* __restri
                                                               tiles_m, tiles_n, swizzle, epi);
 }
 
-// Blocks per SIMD's worth of waves the registers must leave room for: two 128x128 blocks of eight
-// waves, three 128x64 or four 64x64 blocks of four per CU.
-constexpr int split_waves(int bm, int bn) { return bm * bn >= 128 * 128 ? 4 : bm * bn >= 128 * 64 ? 3 : 4; }
+// Waves per SIMD the registers must leave room for: two 128x128 blocks of eight waves per CU (one
+// with two steps in LDS), three 128x64 or 64x64 blocks of four.
+constexpr int split_waves(int bm, int bn, int u) { return bm * bn >= 128 * 128 ? (u == 1 ? 4 : 2) : 3; }
 
-template <int BM, int BN, int WM, int WN, bool TA, bool TB, bool TAIL>
-__global__ void __launch_bounds__(64 * WM * WN, split_waves(BM, BN)) k_gemm_mfma(const float* __restrict__ A, const float* __restrict__ B,
-                                                                               float* __restrict__ C, int M, int N, int K,
-                                                                               const int64_t* a_off, const int64_t* b_off, uint64_t a_stride,
-                                                                               uint64_t b_stride, int splits, int k_per_split,
-                                                                               float* __restrict__ partial, const float* __restrict__ bias,
-                                                                               uint32_t tiles_m, uint32_t tiles_n) {
+template <int BM, int BN, int WM, int WN, int U, bool TA, bool TB, bool TAIL>
+__global__ void __launch_bounds__(64 * WM * WN, split_waves(BM, BN, U)) k_gemm_mfma(const float* __restrict__ A, const float* __restrict__ B,
+                                                                                  float* __restrict__ C, int M, int N, int K,
+                                                                                  const int64_t* a_off, const int64_t* b_off, uint64_t a_stride,
+                                                                                  uint64_t b_stride, int splits, int k_per_split,
+                                                                                  float* __restrict__ partial, const float* __restrict__ bias,
+                                                                                  uint32_t tiles_m, uint32_t tiles_n) {
   rgg::StoreC epi{C, partial, splits, (uint64_t)M * N};
-  rgg::gemm_mfma_block<BM, BN, WM, WN, TA, TB, TAIL>(A, B, M, N, K, a_off, b_off, a_stride, b_stride, splits, k_per_split, bias, tiles_m,
-                                                     tiles_n, epi);
+  rgg::gemm_mfma_block<BM, BN, WM, WN, U, TA, TB, TAIL>(A, B, M, N, K, a_off, b_off, a_stride, b_stride, splits, k_per_split, bias, tiles_m,
+                                                        tiles_n, epi);
 }
 
 // One unbatched product's share of a grouped launch (k_gemm_mfma_group).
@@ -78,34 +78,34 @@ struct GroupParts {
 };
 
 // Part I of a grouped launch: flags bits 2I (TB) and 2I + 1 (TA).
-template <int BM, int BN, int WM, int WN, int FLAGS, int I>
+template <int BM, int BN, int WM, int WN, int U, int FLAGS, int I>
 __device__ __forceinline__ void group_part(const GroupPart& p, uint32_t bid, cell* smem) {
   constexpr bool TA = (FLAGS >> (2 * I + 1)) & 1, TB = (FLAGS >> (2 * I)) & 1;
   StoreC epi{p.c, p.part, p.splits, (uint64_t)p.m * p.n};
-  gemm_split_tile<BM, BN, WM, WN, TA, TB, false>(p.a, p.b, p.m, p.n, p.k, nullptr, nullptr, 0, 0, p.splits, p.kps, p.bias, p.tm, p.tn, epi, bid,
+  gemm_split_tile<BM, BN, WM, WN, U, TA, TB, false>(p.a, p.b, p.m, p.n, p.k, nullptr, nullptr, 0, 0, p.splits, p.kps, p.bias, p.tm, p.tn, epi, bid,
                                                  p.blocks, smem);
 }
 
-template <int BM, int BN, int WM, int WN, int FLAGS, int I>
+template <int BM, int BN, int WM, int WN, int U, int FLAGS, int I>
 constexpr int part_lds() {
-  return SplitLds<BM, BN, WM, WN, ((FLAGS >> (2 * I + 1)) & 1) != 0, ((FLAGS >> (2 * I)) & 1) != 0>::CELLS;
+  return SplitLds<BM, BN, WM, WN, U, ((FLAGS >> (2 * I + 1)) & 1) != 0, ((FLAGS >> (2 * I)) & 1) != 0>::CELLS;
 }
 
 // N independent unbatched products on one tile shape in one launch: part i takes the next
 // p[i].blocks blocks, all staging through the same LDS. Each block runs the code of a single
 // product's launch, so every output gets the same bits; the launch's fixed cost is paid once,
 // and the parts' grids (each one or two blocks per CU) run side by side.
-template <int BM, int BN, int WM, int WN, int N, int FLAGS>
-__global__ void __launch_bounds__(64 * WM * WN, split_waves(BM, BN)) k_gemm_mfma_group(GroupParts g) {
-  constexpr int F0 = part_lds<BM, BN, WM, WN, FLAGS, 0>(), F1 = part_lds<BM, BN, WM, WN, FLAGS, 1>();
-  constexpr int F2 = N > 2 ? part_lds<BM, BN, WM, WN, FLAGS, 2>() : 0;
+template <int BM, int BN, int WM, int WN, int U, int N, int FLAGS>
+__global__ void __launch_bounds__(64 * WM * WN, split_waves(BM, BN, U)) k_gemm_mfma_group(GroupParts g) {
+  constexpr int F0 = part_lds<BM, BN, WM, WN, U, FLAGS, 0>(), F1 = part_lds<BM, BN, WM, WN, U, FLAGS, 1>();
+  constexpr int F2 = N > 2 ? part_lds<BM, BN, WM, WN, U, FLAGS, 2>() : 0;
   constexpr int F01 = F0 > F1 ? F0 : F1;
   __shared__ cell smem[F01 > F2 ? F01 : F2];
   uint32_t bid = blockIdx.x;
-  if (bid < g.p[0].blocks) return group_part<BM, BN, WM, WN, FLAGS, 0>(g.p[0], bid, smem);
+  if (bid < g.p[0].blocks) return group_part<BM, BN, WM, WN, U, FLAGS, 0>(g.p[0], bid, smem);
   bid -= g.p[0].blocks;
-  if (N == 2 || bid < g.p[1].blocks) return group_part<BM, BN, WM, WN, FLAGS, 1>(g.p[1], bid, smem);
-  if constexpr (N > 2) group_part<BM, BN, WM, WN, FLAGS, 2>(g.p[2], bid - g.p[1].blocks, smem);
+  if (N == 2 || bid < g.p[1].blocks) return group_part<BM, BN, WM, WN, U, FLAGS, 1>(g.p[1], bid, smem);
+  if constexpr (N > 2) group_part<BM, BN, WM, WN, U, FLAGS, 2>(g.p[2], bid - g.p[1].blocks, smem);
 }
 
 // Sums the K-split partial products in split order. Four outputs per thread (16-byte loads when
@@ -553,10 +553,10 @@ int skinny_rows_splits(uint64_t n, uint64_t k) {
 
 struct TileCfg {
   int bm, bn, bk, wm, wn;
-  bool split;  // bf16 terms (gemm_split.h); otherwise fp32 MFMA (gemm_mfma.h)
+  int split;  // steps in LDS of the bf16 terms' tile (gemm_split.h); 0: fp32 MFMA (gemm_mfma.h)
 };
-constexpr TileCfg SPLIT_128x128 = {128, 128, SPLIT_BK, 2, 4, true}, SPLIT_128x64 = {128, 64, SPLIT_BK, 2, 2, true},
-                  SPLIT_64x64 = {64, 64, SPLIT_BK, 2, 2, true};
+constexpr TileCfg SPLIT_128x128 = {128, 128, SPLIT_BK, 2, 4, 1}, SPLIT_128x128_2 = {128, 128, SPLIT_BK, 2, 4, 2},
+                  SPLIT_128x64 = {128, 64, SPLIT_BK, 2, 2, 1}, SPLIT_64x64 = {64, 64, SPLIT_BK, 2, 2, 2};
 
 uint64_t tile_count(const TileCfg& t, uint64_t m, uint64_t n, uint64_t batch) { return ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn) * batch; }
 
@@ -574,12 +574,12 @@ int split_count(const TileCfg& t, uint64_t m, uint64_t n, uint64_t k, uint64_t b
 // Block tile, from measurements on MI355X (us; M x N x K, T: that operand transposed).
 // Products whose 64x64 tiles, split over K where K allows, come to a block per CU run on the bf16
 // terms:
-//  - 128x128 at two blocks per CU and K over 256 (4096x2048x2048: 183 against 223 on 128x64;
-//    4096x2048x512: 53 and 57), or a K of 2048 and more whose splits give most CUs a block
-//    (T 256x1024x8192: 34 against 36 on 128x64, 46 on 64x64; T 2048x2048x4096: 203 and 221);
-//  - 128x64 at three blocks per CU (8192x768x256: 24.0 against 25.3 on 128x128 and 25.8 on 64x64),
-//    and at four for K up to 256 (8192x1024x256, T: 27.8 against 29.1 on 128x128);
-//  - 64x64 otherwise (8192x256x256: 11.1 against 11.7 on 128x64; fp32 MFMA tiles 11.7).
+//  - 128x128 at two blocks per CU (4096x2048x2048: 179 against 214 on 128x64; 8192x1024x256: 26.9
+//    and 30.7), or a K of 2048 and more whose splits give most CUs a block, then with two steps in
+//    LDS (T 256x1024x8192: 29.4 against 33.1 with one and 35.6 on 64x64; T 2048x2048x4096: 200
+//    against 232 and 252);
+//  - 128x64 at three blocks per CU (8192x768x256: 24.4 against 27.4 on 64x64);
+//  - 64x64 otherwise (8192x256x1024: 35.7 against 41 on 128x64; 8192x256x256: 11.5 and 12.9).
 // Below that a block runs alone on its CU and fp32 MFMA tiles are faster: 32-wide ones for outputs
 // 32..96 wide or 32 tall (attention heads, the vocabulary), 32x32 otherwise (256x768x256: 4.3
 // against 7.1 on bf16 terms; 4096x128x512: 8.6 and 13), or 64x64 where a side under 64 keeps a
@@ -588,15 +588,18 @@ TileCfg pick_tile(uint64_t m, uint64_t n, uint64_t k, uint64_t batch) {
   auto filled = [&](const TileCfg& t) { return tile_count(t, m, n, batch) * (uint64_t)split_count(t, m, n, k, batch); };
   // A column-contiguous operand's offsets within 24 rows are 32-bit: sides of less than 2^25.
   if (m >= 64 && n >= 64 && m < (1u << 25) && n < (1u << 25) && filled(SPLIT_64x64) >= 256) {
-    if (m >= 128 && n >= 128 && ((tile_count(SPLIT_128x128, m, n, batch) >= 512 && k > 256) || (k >= 2048 && filled(SPLIT_128x128) >= 192)))
-      return SPLIT_128x128;
+    if (m >= 128 && n >= 128) {
+      const uint64_t blocks = filled(SPLIT_128x128);
+      if (tile_count(SPLIT_128x128, m, n, batch) >= 512 || (k >= 2048 && blocks > 256)) return SPLIT_128x128;
+      if (k >= 2048 && blocks >= 192) return SPLIT_128x128_2;
+    }
     if (m >= 128 && tile_count(SPLIT_128x64, m, n, batch) >= 768) return SPLIT_128x64;
     return SPLIT_64x64;
   }
-  if (n <= 96 && n % 32 == 0) return {128, 32, 32, 4, 1, false};
-  if (m <= 32) return {32, 128, 32, 1, 4, false};
-  const TileCfg t64 = {64, 64, 32, 2, 2, false};
-  return filled(t64) < 256 ? TileCfg{32, 32, 32, 2, 2, false} : t64;
+  if (n <= 96 && n % 32 == 0) return {128, 32, 32, 4, 1, 0};
+  if (m <= 32) return {32, 128, 32, 1, 4, 0};
+  const TileCfg t64 = {64, 64, 32, 2, 2, 0};
+  return filled(t64) < 256 ? TileCfg{32, 32, 32, 2, 2, 0} : t64;
 }
 
 struct Launch {
@@ -613,12 +616,12 @@ struct Launch {
 };
 
 // `mode`: the fp32 tile's load mode, or whether some K range of the split tile is no multiple of 32.
-template <int BM, int BN, int WM, int WN, bool TA, bool TB, bool SPLIT>
+template <int BM, int BN, int WM, int WN, bool TA, bool TB, int U>
 void launch_mode(hipStream_t s, int mode, const Launch& l) {
   const dim3 block(64 * WM * WN);
-  if constexpr (SPLIT) {
+  if constexpr (U > 0) {
 #define RG_GEMM(TAIL_)                                                                                                              \
-  hipLaunchKernelGGL((k_gemm_mfma<BM, BN, WM, WN, TA, TB, TAIL_>), l.grid, block, 0, s, l.a, l.b, l.c, l.m, l.n, l.k, l.a_off, l.b_off, \
+  hipLaunchKernelGGL((k_gemm_mfma<BM, BN, WM, WN, U, TA, TB, TAIL_>), l.grid, block, 0, s, l.a, l.b, l.c, l.m, l.n, l.k, l.a_off, l.b_off, \
                      l.as, l.bs, l.splits, l.kps, l.part, l.bias, l.tm, l.tn)
     if (mode) RG_GEMM(true);
     else RG_GEMM(false);
@@ -634,26 +637,27 @@ void launch_mode(hipStream_t s, int mode, const Launch& l) {
   }
 }
 
-template <int BM, int BN, int WM, int WN, bool SPLIT>
+template <int BM, int BN, int WM, int WN, int U>
 void launch_flags(hipStream_t s, bool ta, bool tb, int mode, const Launch& l) {
-  if (!ta && !tb) launch_mode<BM, BN, WM, WN, false, false, SPLIT>(s, mode, l);
-  else if (ta && !tb) launch_mode<BM, BN, WM, WN, true, false, SPLIT>(s, mode, l);
-  else if (!ta && tb) launch_mode<BM, BN, WM, WN, false, true, SPLIT>(s, mode, l);
-  else launch_mode<BM, BN, WM, WN, true, true, SPLIT>(s, mode, l);
+  if (!ta && !tb) launch_mode<BM, BN, WM, WN, false, false, U>(s, mode, l);
+  else if (ta && !tb) launch_mode<BM, BN, WM, WN, true, false, U>(s, mode, l);
+  else if (!ta && tb) launch_mode<BM, BN, WM, WN, false, true, U>(s, mode, l);
+  else launch_mode<BM, BN, WM, WN, true, true, U>(s, mode, l);
 }
 
 // Instantiates the tile shapes pick_tile can return.
 void launch_mfma(hipStream_t s, const TileCfg& t, bool ta, bool tb, int mode, const Launch& l) {
-#define RG_TILE(BM_, BN_, WM_, WN_, SPLIT_)                                                        \
-  if (t.bm == BM_ && t.bn == BN_ && t.wm == WM_ && t.wn == WN_ && t.bk == 32 && t.split == SPLIT_) \
-  return launch_flags<BM_, BN_, WM_, WN_, SPLIT_>(s, ta, tb, mode, l)
-  RG_TILE(128, 128, 2, 4, true);
-  RG_TILE(128, 64, 2, 2, true);
-  RG_TILE(64, 64, 2, 2, true);
-  RG_TILE(64, 64, 2, 2, false);
-  RG_TILE(128, 32, 4, 1, false);
-  RG_TILE(32, 128, 1, 4, false);
-  RG_TILE(32, 32, 2, 2, false);
+#define RG_TILE(BM_, BN_, WM_, WN_, U_)                                                    \
+  if (t.bm == BM_ && t.bn == BN_ && t.wm == WM_ && t.wn == WN_ && t.bk == 32 && t.split == U_) \
+  return launch_flags<BM_, BN_, WM_, WN_, U_>(s, ta, tb, mode, l)
+  RG_TILE(128, 128, 2, 4, 1);
+  RG_TILE(128, 128, 2, 4, 2);
+  RG_TILE(128, 64, 2, 2, 1);
+  RG_TILE(64, 64, 2, 2, 2);
+  RG_TILE(64, 64, 2, 2, 0);
+  RG_TILE(128, 32, 4, 1, 0);
+  RG_TILE(32, 128, 1, 4, 0);
+  RG_TILE(32, 32, 2, 2, 0);
 #undef RG_TILE
   throw std::runtime_error("product tile without a kernel");
 }
@@ -688,13 +692,10 @@ bool gemm_epilogue_tile(int dtype, uint64_t m, uint64_t n, uint64_t k, bool ta, 
   if (skinny_plan(dtype, m, n, k, 1, ta, tb).kind != SKINNY_NONE || !use_mfma(dtype, m, n, k)) return false;
   TileCfg t = pick_tile(m, n, k, 1);
   if (!t.split || split_count(t, m, n, k, 1) != 1) return false;
-  // Short K: 128x64 tiles rather than 128x128, twice the blocks, so that the second round's
-  // products run while the first round's epilogues read and write.
-  if (t.bm == 128 && t.bn == 128 && k <= 1024) t = SPLIT_128x64;
   // The epilogue's loads and stores are aligned vectors of four columns.
   if (n % 4 != 0) return false;
-  *out = GemmTile{t.bm, t.bn, t.wm, t.wn, k % SPLIT_BK != 0, m % t.bm == 0 && n % t.bn == 0, (int)((k + t.bk - 1) / t.bk * t.bk),
-                  (uint32_t)((m + t.bm - 1) / t.bm), (uint32_t)((n + t.bn - 1) / t.bn)};
+  *out = GemmTile{t.bm, t.bn, t.wm, t.wn, t.split, k % SPLIT_BK != 0, m % t.bm == 0 && n % t.bn == 0,
+                  (int)((k + t.bk - 1) / t.bk * t.bk), (uint32_t)((m + t.bm - 1) / t.bm), (uint32_t)((n + t.bn - 1) / t.bn)};
   return true;
 }
 
@@ -952,7 +953,7 @@ bool gemm_group(hipStream_t s, const GemmArgs* g, int count, bool launch) {
   // One split tile for all, 128x128: every split tile sums a K range's terms in the same order, so a
   // product picked for a smaller one keeps its bits, and its K splits. K-split partials, if any, must
   // be the deferred kind: a split sum after the grouped launch would be a second launch anyway.
-  const TileCfg t = SPLIT_128x128;
+  const TileCfg t = SPLIT_128x128_2;
   int mode;
   Launch l[GROUP_MAX];
   int flags = 0;
@@ -983,7 +984,7 @@ bool gemm_group(hipStream_t s, const GemmArgs* g, int count, bool launch) {
   }
 #define RG_GROUP(COUNT_, FLAGS_)                                                                                      \
   if (count == COUNT_ && flags == (FLAGS_)) {                                                                         \
-    if (launch) hipLaunchKernelGGL((k_gemm_mfma_group<128, 128, 2, 4, COUNT_, FLAGS_>), dim3(blocks), block, 0, s, parts); \
+    if (launch) hipLaunchKernelGGL((k_gemm_mfma_group<128, 128, 2, 4, 2, COUNT_, FLAGS_>), dim3(blocks), block, 0, s, parts); \
     return true;                                                                                                      \
   }
   RG_GROUP(2, N | T << 2)

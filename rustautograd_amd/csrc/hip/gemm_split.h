@@ -85,7 +85,7 @@ struct StoreC {
   __device__ __forceinline__ void begin(uint32_t b, uint32_t sp) {
     out = splits > 1 ? partial + ((uint64_t)b * splits + sp) * mn : C + (uint64_t)b * mn;
   }
-  __device__ __forceinline__ void put4(uint64_t e, float4 v, int) { __builtin_nontemporal_store(rowx4{v.x, v.y, v.z, v.w}, (rowx4*)(out + e)); }
+  __device__ __forceinline__ void put4(uint64_t e, float4 v) { __builtin_nontemporal_store(rowx4{v.x, v.y, v.z, v.w}, (rowx4*)(out + e)); }
   __device__ __forceinline__ void put2(uint64_t e, float2 v) { __builtin_nontemporal_store(floatx2{v.x, v.y}, (floatx2*)(out + e)); }
   __device__ __forceinline__ void put1(uint64_t e, float v) { __builtin_nontemporal_store(v, out + e); }
 };
@@ -207,9 +207,10 @@ struct SplitStage {
   }
 };
 
-template <int BM, int BN, int WM, int WN, bool TA, bool TB>
+template <int BM, int BN, int WM, int WN, int U, bool TA, bool TB>
 struct SplitLds {
-  static constexpr int CELLS = SplitGeo<BM, !TA, 64 * WM * WN>::CELLS + SplitGeo<BN, TB, 64 * WM * WN>::CELLS;
+  static constexpr int STEP = SplitGeo<BM, !TA, 64 * WM * WN>::CELLS + SplitGeo<BN, TB, 64 * WM * WN>::CELLS;
+  static constexpr int CELLS = U * STEP;
 };
 
 // C = op(A) op(B), the BM x BN tile of block `bid` of a product launched as `nb` blocks, staged
@@ -219,14 +220,17 @@ struct SplitLds {
 // tile before it does not. Split `sp` covers K range [sp * k_per_split, (sp + 1) * k_per_split), a
 // multiple of 32 long except the last; TAIL: some range is not a multiple of 32.
 //
-// One LDS buffer: the next tile's values wait in registers while this one is multiplied, are
-// converted and stored between two barriers, and the loads after them go out at once. Two or three
-// blocks share a CU, so that one's conversions run beside another's MFMAs (two LDS buffers and one
-// barrier per step, at half the blocks per CU, measured 3-6 % slower at 4096 x 2048 x 2048).
+// One LDS buffer of U steps: the next U steps' values wait in registers while these are multiplied,
+// are converted and stored between two barriers, and the loads after them go out at once. Where
+// several blocks share a CU, one's conversions run beside another's MFMAs and U is 1 (two LDS buffers
+// and one barrier per step, at half the blocks per CU, measured 3-6 % slower at 4096 x 2048 x 2048);
+// a block with few or no others beside it takes U = 2, half the barriers and waits (T 256x1024x8192
+// on 128x128 tiles, a block per CU: 33.1 -> 29.4 us; 8192x256x1024 on 64x64: 39 -> 35.7). The sums
+// do not depend on U or on the tile's size.
 // The product is formed transposed (B supplies the MFMA rows), so that each lane holds runs of
-// four adjacent output columns: put4's third argument names the run (the same for every row the
-// lane stores), so that an epilogue can keep per-column sums in registers.
-template <int BM, int BN, int WM, int WN, bool TA, bool TB, bool TAIL, class Epi>
+// four adjacent output columns. Every put4 of a lane is of the same four columns, so that an
+// epilogue can keep per-column sums in registers.
+template <int BM, int BN, int WM, int WN, int U, bool TA, bool TB, bool TAIL, class Epi>
 __device__ __forceinline__ void gemm_split_tile(const float* __restrict__ A, const float* __restrict__ B, int M, int N, int K,
                                                 const int64_t* a_off, const int64_t* b_off, uint64_t a_stride, uint64_t b_stride, int splits,
                                                 int k_per_split, const float* __restrict__ bias, uint32_t tiles_m, uint32_t tiles_n, Epi& epi,
@@ -245,27 +249,39 @@ __device__ __forceinline__ void gemm_split_tile(const float* __restrict__ A, con
   const float* Bb = B + batch_offset(b_off, b_stride, b) + (TB ? (int64_t)n0 * K : (int64_t)n0);
   const int kbeg = sp * k_per_split, kend = min(K, kbeg + k_per_split);
   const int nk = (kend - kbeg + SPLIT_BK - 1) / SPLIT_BK;
-  SplitStage<BM, !TA, NT> sa;
-  SplitStage<BN, TB, NT> sb;
+  constexpr int STEP = SplitLds<BM, BN, WM, WN, U, TA, TB>::STEP;
+  SplitStage<BM, !TA, NT> sa[U];
+  SplitStage<BN, TB, NT> sb[U];
+  // Rounds of U steps; the last may have fewer.
+  const int rounds = (nk + U - 1) / U;
   auto load = [&](int t) __attribute__((always_inline)) {
-    const int k0 = kbeg + t * SPLIT_BK;
-    const bool partial = TAIL && k0 + SPLIT_BK > kend;
-    sa.load(Ab, lda, k0, kend, partial, tid);
-    sb.load(Bb, ldb, k0, kend, partial, tid);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (U > 1 && t * U + u >= nk) break;
+      const int k0 = kbeg + (t * U + u) * SPLIT_BK;
+      const bool partial = TAIL && k0 + SPLIT_BK > kend;
+      sa[u].load(Ab, lda, k0, kend, partial, tid);
+      sb[u].load(Bb, ldb, k0, kend, partial, tid);
+    }
   };
   // Odd steps' B is stored negated, and their sums subtracted (multiply's sign).
   auto store = [&](float sign) __attribute__((always_inline)) {
-    sa.template store<false>(smem, tid, 1.0f);
-    sb.template store<true>(smem + GA::CELLS, tid, sign);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      sa[u].template store<false>(smem + u * STEP, tid, 1.0f);
+      if constexpr (U % 2 == 1) sb[u].template store<true>(smem + u * STEP + GA::CELLS, tid, u % 2 ? -sign : sign);
+      else if (u % 2) sb[u].template store<true>(smem + u * STEP + GA::CELLS, tid, -1.0f);
+      else sb[u].template store<false>(smem + u * STEP + GA::CELLS, tid, 1.0f);
+    }
   };
   floatx4 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; i++)
 #pragma unroll
     for (int n = 0; n < TN; n++) acc[i][n] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-  auto multiply = [&](float sign) __attribute__((always_inline)) {
-    const cell* as = smem + lo * GA::GROUP;
-    const cell* bs = smem + GA::CELLS + lo * GB::GROUP;
+  auto multiply_step = [&](float sign, int u) __attribute__((always_inline)) {
+    const cell* as = smem + u * STEP + lo * GA::GROUP;
+    const cell* bs = smem + u * STEP + GA::CELLS + lo * GB::GROUP;
     bf16x8 y[3][TN];
 #pragma unroll
     for (int p = 0; p < 3; p++)
@@ -290,20 +306,27 @@ __device__ __forceinline__ void gemm_split_tile(const float* __restrict__ A, con
         for (int r = 0; r < 4; r++) acc[i][n][r] = __builtin_fmaf(step[n][r], sign, acc[i][n][r]);
     }
   };
+  auto multiply = [&](float sign, int t, bool last) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (last && U > 1 && t * U + u >= nk) break;
+      multiply_step(u % 2 ? -sign : sign, u);
+    }
+  };
   load(0);
-  float sign = 1.0f;  // of the tile in LDS
+  float sign = 1.0f;  // of the first step in LDS
   store(sign);
-  if (nk > 1) load(1);
+  if (rounds > 1) load(1);
   __syncthreads();
-  for (int t = 0; t < nk - 1; t++) {
-    multiply(sign);
+  for (int t = 0; t < rounds - 1; t++) {
+    multiply(sign, t, false);
     __syncthreads();
-    sign = -sign;
+    if (U % 2 == 1) sign = -sign;
     store(sign);
-    if (t + 2 < nk) load(t + 2);
+    if (t + 2 < rounds) load(t + 2);
     __syncthreads();
   }
-  multiply(sign);
+  multiply(sign, rounds - 1, true);
   // Lane l of the wave's tile (i, n) holds output row 16 i + l % 16, columns 16 n + 4 (l / 16) .. + 3.
   // A sum that is not finite: this wave's outputs again, in fp32.
   float finite = 0.0f;  // NaN once any sum is infinite or NaN
@@ -339,44 +362,52 @@ __device__ __forceinline__ void gemm_split_tile(const float* __restrict__ A, con
       }
     }
   }
+  // The outputs leave through LDS, 32 rows x 32 columns of a wave at a time, so that a lane stores
+  // the same four columns of every eighth row and a store covers whole 128-byte runs of eight rows
+  // (from the accumulators it would cover 64 bytes of sixteen). Each wave has its own part.
+  static_assert(WTN == 32 && TM % 2 == 0 && WM * WN * 32 * 9 <= STEP, "wave tiles");
   epi.begin(b, sp);
-  // A per-column bias (unsplit products only) added to the finished sums, as one fp32 addition.
-  if (bias) {
+  const int c4 = lane & 7, col = n0 + wn * 32 + 4 * c4;
+  floatx4 add = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (bias) add = *(const rowx4*)(bias + col);
+  floatx4* out = (floatx4*)smem + wave * 32 * 9;
+  __syncthreads();
 #pragma unroll
-    for (int n = 0; n < TN; n++) {
-      const float* p = bias + n0 + wn * WTN + n * 16 + 4 * lo;
-      const floatx4 x = {p[0], p[1], p[2], p[3]};
+  for (int i = 0; i < TM; i += 2) {
 #pragma unroll
-      for (int i = 0; i < TM; i++) acc[i][n] = acc[i][n] + x;
-    }
-  }
+    for (int h = 0; h < 2; h++)
 #pragma unroll
-  for (int i = 0; i < TM; i++) {
-    const int row = m0 + wm * WTM + i * 16 + li;
-    if (row < m_first) continue;
-    const uint64_t erow = (uint64_t)row * N;
+      for (int n = 0; n < TN; n++) out[(16 * h + li) * 9 + 4 * n + lo] = acc[i + h][n];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int n = 0; n < TN; n++) {
-      const int col = n0 + wn * WTN + n * 16 + 4 * lo;
-      const floatx4 c = acc[i][n];
+    for (int q = 0; q < 4; q++) {
+      const int r = 8 * q + (lane >> 3), row = m0 + wm * WTM + 16 * i + r;
+      floatx4 c = out[r * 9 + c4];
+      // A per-column bias (unsplit products only) added to the finished sums, as one fp32 addition.
+      if (bias) c = c + add;
+      if (row < m_first) continue;
+      const uint64_t e = (uint64_t)row * N + col;
       if (col >= n_first) {
-        epi.put4(erow + col, make_float4(c[0], c[1], c[2], c[3]), n);
+        epi.put4(e, make_float4(c[0], c[1], c[2], c[3]));
       } else {
 #pragma unroll
-        for (int r = 0; r < 4; r++)
-          if (col + r >= n_first) epi.put1(erow + col + r, c[r]);
+        for (int x = 0; x < 4; x++)
+          if (col + x >= n_first) epi.put1(e + x, c[x]);
       }
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
   }
 }
 
 // One product over the whole grid, with its own LDS.
-template <int BM, int BN, int WM, int WN, bool TA, bool TB, bool TAIL, class Epi>
+template <int BM, int BN, int WM, int WN, int U, bool TA, bool TB, bool TAIL, class Epi>
 __device__ __forceinline__ void gemm_mfma_block(const float* __restrict__ A, const float* __restrict__ B, int M, int N, int K,
                                                 const int64_t* a_off, const int64_t* b_off, uint64_t a_stride, uint64_t b_stride, int splits,
                                                 int k_per_split, const float* __restrict__ bias, uint32_t tiles_m, uint32_t tiles_n, Epi& epi) {
-  __shared__ cell smem[SplitLds<BM, BN, WM, WN, TA, TB>::CELLS];
-  gemm_split_tile<BM, BN, WM, WN, TA, TB, TAIL>(A, B, M, N, K, a_off, b_off, a_stride, b_stride, splits, k_per_split, bias, tiles_m, tiles_n,
+  __shared__ cell smem[SplitLds<BM, BN, WM, WN, U, TA, TB>::CELLS];
+  gemm_split_tile<BM, BN, WM, WN, U, TA, TB, TAIL>(A, B, M, N, K, a_off, b_off, a_stride, b_stride, splits, k_per_split, bias, tiles_m, tiles_n,
                                                 epi, blockIdx.x, gridDim.x, smem);
 }
 

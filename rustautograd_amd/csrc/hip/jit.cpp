@@ -184,14 +184,11 @@ std::string generate_gemm(const rgplan::Fused& f, int64_t c_slot, bool store_c, 
                           FusedKernel* k, int col_sum) {
   if (f.dtype != RG_F32) throw std::runtime_error("product epilogue: fp32 groups only");
   const std::string E = name + "_epi";
-  // Column sums (col_sum >= 0): each lane stores runs of four columns, the same runs for every row
-  // (put4's slot: tile n across N).
-  const int slots = t.bn / t.wn / 16;
   std::ostringstream s;
   s << "struct " << E << " {\n  float* c;\n";
   for (size_t j = 0; j < f.inputs.size(); j++) s << "  const float* in" << j << ";\n";
   for (size_t j = 0; j < f.outputs.size(); j++) s << "  float* out" << j << ";\n";
-  if (col_sum >= 0) s << "  float4 colacc[" << slots << "];\n";
+  if (col_sum >= 0) s << "  float4 colacc;\n";  // column sums: a lane stores the same four columns of every row
   s << "  __device__ __forceinline__ void begin(unsigned int, unsigned int) {}\n";
   // The group's value of element e + v for v < W, from the product's outputs `a`.
   auto body = [&](int W) {
@@ -240,13 +237,12 @@ std::string generate_gemm(const rgplan::Fused& f, int64_t c_slot, bool store_c, 
     }
     return b.str();
   };
-  s << "  __device__ __forceinline__ void put4(unsigned long long e, float4 acc, int slot) {\n";
+  s << "  __device__ __forceinline__ void put4(unsigned long long e, float4 acc) {\n";
   if (store_c) s << "    *(float4*)(c + e) = acc;\n";
   s << "    const float a[4] = {acc.x, acc.y, acc.z, acc.w};\n" << body(4);
   if (col_sum >= 0) {
     const std::string o = "o" + std::to_string(col_sum);
-    s << "    colacc[slot] = make_float4(colacc[slot].x + " << o << "[0], colacc[slot].y + " << o << "[1], colacc[slot].z + " << o
-      << "[2], colacc[slot].w + " << o << "[3]);\n";
+    s << "    colacc = make_float4(colacc.x + " << o << "[0], colacc.y + " << o << "[1], colacc.z + " << o << "[2], colacc.w + " << o << "[3]);\n";
   }
   s << "  }\n";
   s << "  __device__ __forceinline__ void put1(unsigned long long e, float acc) {\n";
@@ -256,7 +252,9 @@ std::string generate_gemm(const rgplan::Fused& f, int64_t c_slot, bool store_c, 
   const int nt = 64 * t.wm * t.wn;
   // At least two waves per SIMD (at most 256 registers a wave, far above what the tile uses): with
   // that bound the compiler keeps the MFMA accumulators in ordinary VGPRs, as the precompiled
-  // tiles are built (-amdgpu-mfma-vgpr-form), rather than copying them through AGPRs.
+  // tiles are built (-amdgpu-mfma-vgpr-form), rather than copying them through AGPRs. Eight-wave
+  // tiles of one step share a CU in pairs: at most 128 registers.
+  const char* regs = nt > 256 && t.steps == 1 ? ", amdgpu_num_vgpr(128)" : "";
   // The epilogue's pointers arrive as kernel parameters, restrict-qualified when no output shares
   // a slot with an input or the product, so that the compiler may issue an output's loads before
   // the stores of the outputs before it.
@@ -266,7 +264,7 @@ std::string generate_gemm(const rgplan::Fused& f, int64_t c_slot, bool store_c, 
     for (auto& in : f.inputs) alias |= in.slot == o.second;
   }
   const char* R = alias ? "" : "__restrict__ ";
-  s << "extern \"C\" __global__ void __launch_bounds__(" << nt << ") __attribute__((amdgpu_waves_per_eu(2))) " << name
+  s << "extern \"C\" __global__ void __launch_bounds__(" << nt << ") __attribute__((amdgpu_waves_per_eu(2)" << regs << ")) " << name
     << "(const float* __restrict__ A, const float* __restrict__ B, int M, int N, int K, const rgg::int64_t* a_off, const rgg::int64_t* b_off, "
        "rgg::uint64_t a_stride, rgg::uint64_t b_stride, int splits, int kps, const float* __restrict__ bias, rgg::uint32_t tiles_m, "
        "rgg::uint32_t tiles_n, float* "
@@ -278,24 +276,22 @@ std::string generate_gemm(const rgplan::Fused& f, int64_t c_slot, bool store_c, 
   for (size_t j = 0; j < f.inputs.size(); j++) s << ", in" << j;
   for (size_t j = 0; j < f.outputs.size(); j++) s << ", out" << j;
   s << "};\n";
-  if (col_sum >= 0) s << "  for (int q = 0; q < " << slots << "; q++) epi.colacc[q] = make_float4(0.f, 0.f, 0.f, 0.f);\n";
-  s << "  rgg::gemm_mfma_block<" << t.bm << ", " << t.bn << ", " << t.wm << ", " << t.wn << ", " << (t.ta ? "true" : "false") << ", "
+  if (col_sum >= 0) s << "  epi.colacc = make_float4(0.f, 0.f, 0.f, 0.f);\n";
+  s << "  rgg::gemm_mfma_block<" << t.bm << ", " << t.bn << ", " << t.wm << ", " << t.wn << ", " << t.steps << ", " << (t.ta ? "true" : "false") << ", "
     << (t.tb ? "true" : "false") << ", " << (t.tail ? "true" : "false")
     << ">(A, B, M, N, K, a_off, b_off, a_stride, b_stride, splits, kps, bias, tiles_m, tiles_n, epi);\n";
   if (col_sum >= 0) {
     // The tile's column sums of output col_sum from the lanes' register sums (each lane summed
-    // its rows in order): the 16 lanes holding the same columns combine by a fixed butterfly,
+    // its rows in order): the eight lanes holding the same columns combine by a fixed butterfly,
     // then the WM waves along M in order, through LDS; one partial row per tile row. Lane l of
-    // wave (wm, wn) holds, in slot n, columns wn * WTN + 16 n + 4 (l / 16) .. + 3 of the tile.
-    const int wtn = t.bn / t.wn;
+    // wave (wm, wn) holds columns 32 wn + 4 (l % 8) .. + 3 of the tile.
     s << "  __shared__ float cs[" << t.wm << "][" << t.bn << "];\n";
     s << "  {\n    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wmi = wave / " << t.wn << ", wni = wave % " << t.wn << ";\n";
-    s << "    for (int q = 0; q < " << slots << "; q++) {\n";
-    s << "      float4 v = epi.colacc[q];\n";
-    s << "      for (int x = 1; x < 16; x <<= 1) {\n";
-    s << "        v.x = v.x + __shfl_xor(v.x, x); v.y = v.y + __shfl_xor(v.y, x);\n";
-    s << "        v.z = v.z + __shfl_xor(v.z, x); v.w = v.w + __shfl_xor(v.w, x);\n      }\n";
-    s << "      if ((lane & 15) == 0) *(float4*)&cs[wmi][wni * " << wtn << " + 16 * q + 4 * (lane >> 4)] = v;\n    }\n  }\n";
+    s << "    float4 v = epi.colacc;\n";
+    s << "    for (int x = 8; x < 64; x <<= 1) {\n";
+    s << "      v.x = v.x + __shfl_xor(v.x, x); v.y = v.y + __shfl_xor(v.y, x);\n";
+    s << "      v.z = v.z + __shfl_xor(v.z, x); v.w = v.w + __shfl_xor(v.w, x);\n    }\n";
+    s << "    if (lane < 8) *(float4*)&cs[wmi][wni * 32 + 4 * lane] = v;\n  }\n";
     s << "  __syncthreads();\n";
     s << "  if (threadIdx.x < " << t.bn << ") {\n";
     s << "    const rgg::TileIndex ti = rgg::tile_of(blockIdx.x, gridDim.x, tiles_m, tiles_n, 1);\n";

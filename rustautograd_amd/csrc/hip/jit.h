@@ -55,7 +55,7 @@ std::string generate_rows(const rgplan::Fused& f, const std::string& name, Fused
 
 // A product's tile for generate_gemm (the template arguments of rgg::gemm_mfma_block).
 struct ProductTile {
-  int bm, bn, wm, wn;
+  int bm, bn, wm, wn, steps;
   bool tail, ta, tb;
 };
 

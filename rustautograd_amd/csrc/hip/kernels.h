@@ -199,7 +199,7 @@ uint64_t gemm_workspace(int dtype, uint64_t m, uint64_t n, uint64_t k, uint64_t 
 // columns, when it runs unsplit on that tile (the form an elementwise epilogue takes): its template
 // arguments. False for any other product. `whole`: M and N are multiples of the tile.
 struct GemmTile {
-  int bm, bn, wm, wn;
+  int bm, bn, wm, wn, steps;
   bool tail, whole;
   int kps;
   uint32_t tm, tn;

@@ -784,14 +784,13 @@ bool flat_product(const Instr& i, uint64_t* m, uint64_t* n, uint64_t* k, bool* t
 //    writes its output (a weight-gradient product between an input-gradient product and the
 //    activation gradient that reads it, whose output reuses the slot the weight gradient reads).
 // Groups small enough to be merged are left to the merged launches. The product's kernel also
-// stores its own output when another step reads it. Only products of at least
-// EPILOGUE_MIN_TILES tiles are taken: every block of a product ends its K loop at about the
-// same time, and the epilogue's loads and stores then run with no products beside them unless a
-// second round of blocks is still multiplying (measured on MI355X: C4's GELU forward and
-// backward, 8192 x 1024 outputs in 1024 tiles, 1.7 % off the step; C2's activation gradient and
-// its 2048 x 2048 AdamW update, 512 tiles each, 1.1 % slower fused). RG_HIP_EPILOGUE=0 turns
+// stores its own output when another step reads it. Only large products are taken, of 2^23 outputs
+// at K up to 1024 and 2^24 above: the epilogue's loads and stores run beside little matrix work, and
+// what is saved is one pass over the product's output (measured on MI355X with fp32 MFMA tiles: C4's
+// GELU forward and backward, 8192 x 1024 outputs at K = 256, 1.7 % off the step; C2's activation
+// gradient at K = 2048 and its 2048 x 2048 AdamW update 1.1 % slower fused). RG_HIP_EPILOGUE=0 turns
 // this off; RG_HIP_EPILOGUE=all takes every product that qualifies otherwise.
-constexpr uint64_t EPILOGUE_MIN_TILES = 1024;  // two rounds of two blocks on each of 256 CUs
+uint64_t epilogue_min_outputs(uint64_t k) { return k <= 1024 ? 1ull << 23 : 1ull << 24; }
 
 // Whether product k's output is read by a step other than j (or by the host) before it is next
 // written.
@@ -914,7 +913,7 @@ Epilogues find_epilogues(const Plan& plan) {
       rgk::GemmTile tile;
       if (!flat_product(sk.instr, &m, &nn, &kk, &ta, &tb) || (uint64_t)f.n != m * nn) continue;
       if (!rgk::gemm_epilogue_tile(RG_F32, m, nn, kk, ta, tb, &tile)) continue;
-      if (!every && (uint64_t)tile.tm * tile.tn < EPILOGUE_MIN_TILES) continue;
+      if (!every && m * nn < epilogue_min_outputs(kk)) continue;
       bool ok = true;
       for (auto& o : f.outputs)
         for (auto& a : sk.instr.args) ok = ok && o.second != a.slot;
@@ -976,7 +975,7 @@ std::string epilogue_source(const Plan& plan, size_t j, int64_t pk, const std::s
   rgk::GemmTile t;
   if (!flat_product(pi, &m, &nn, &kk, &ta, &tb) || !rgk::gemm_epilogue_tile(RG_F32, m, nn, kk, ta, tb, &t))
     throw std::runtime_error("product epilogue: the product does not fit a single tile kernel");
-  return rgjit::generate_gemm(plan.steps[j].fused, c, keep, rgjit::ProductTile{t.bm, t.bn, t.wm, t.wn, t.tail, ta, tb},
+  return rgjit::generate_gemm(plan.steps[j].fused, c, keep, rgjit::ProductTile{t.bm, t.bn, t.wm, t.wn, t.steps, t.tail, ta, tb},
                               prefix + "rge" + std::to_string(pk), fk, col_sum);
 }
 
