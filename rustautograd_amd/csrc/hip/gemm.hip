@@ -18,13 +18,14 @@
 // with little padding; products whose output has too few tiles split K and combine the partial
 // sums in a fixed order (deterministic).
 // fp32 products with at most 16 rows and a long K, or a K of at most 16, stream through the
-// skinny kernels below (HBM-bound shapes); fp64 and the remaining tiny products use a plain
-// kernel, one thread per output element.
+// skinny kernels below (HBM-bound shapes); fp64 products run on fp64
+// MFMA tiles; what remains is a wave per output where K is long, a thread per output otherwise.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <stdexcept>
 #include <string>
+#include <type_traits>
 
 #include "gemm_mfma.h"
 #include "gemm_split.h"
@@ -144,7 +145,7 @@ __global__ void __launch_bounds__(256) k_add_bias(float* __restrict__ C, const f
   if (e < total) C[e] = C[e] + bias[e % n];
 }
 
-// One output element per thread; k ascending.
+// One output element per thread; k ascending, eight loads of each operand in flight.
 template <class T>
 __global__ void __launch_bounds__(256) k_gemm_plain(const T* __restrict__ A, const T* __restrict__ B, T* __restrict__ C, uint32_t M,
                                                     uint32_t N, uint32_t K, bool ta, bool tb, const int64_t* a_off, const int64_t* b_off,
@@ -153,15 +154,175 @@ __global__ void __launch_bounds__(256) k_gemm_plain(const T* __restrict__ A, con
   uint64_t t = (uint64_t)blockIdx.x * 256 + threadIdx.x;
   if (t >= (uint64_t)M * N) return;
   uint32_t i = (uint32_t)(t / N), j = (uint32_t)(t % N);
-  const T* a = A + batch_offset(a_off, a_stride, b);
-  const T* bb = B + batch_offset(b_off, b_stride, b);
+  const T* a = A + batch_offset(a_off, a_stride, b) + (ta ? (uint64_t)i : (uint64_t)i * K);
+  const T* bb = B + batch_offset(b_off, b_stride, b) + (tb ? (uint64_t)j * K : (uint64_t)j);
+  const uint64_t sa = ta ? M : 1, sb = tb ? 1 : N;
   T acc = (T)0;
-  for (uint32_t p = 0; p < K; p++) {
-    T x = ta ? a[(uint64_t)p * M + i] : a[(uint64_t)i * K + p];
-    T y = tb ? bb[(uint64_t)j * K + p] : bb[(uint64_t)p * N + j];
-    acc = acc + x * y;
+  uint32_t p = 0;
+  for (; p + 8 <= K; p += 8) {
+    T x[8], y[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) x[u] = a[(p + u) * sa], y[u] = bb[(p + u) * sb];
+#pragma unroll
+    for (int u = 0; u < 8; u++) acc = acc + x[u] * y[u];
   }
+  for (; p < K; p++) acc = acc + a[p * sa] * bb[p * sb];
   C[(uint64_t)b * M * N + t] = acc;
+}
+
+// Few outputs over a longer K, any type, flags and batch: W waves per output, four outputs per block
+// of W = 1 and one otherwise. Lanes take k 64 W apart in increasing order (eight loads of each
+// operand in flight), a wave's sum by a fixed butterfly, the wave sums added in order. One thread per
+// output walked K alone: 256 x 1 x 8 transposed (linear regression's gradient) took 25 us, 3 here;
+// 1000 x 1 x 500 132 us, 4 here.
+template <class T, int W>
+__global__ void __launch_bounds__(W == 1 ? 256 : 64 * W) k_gemm_dots(const T* __restrict__ A, const T* __restrict__ B, T* __restrict__ C,
+                                                                    uint32_t M, uint32_t N, uint32_t K, bool ta, bool tb,
+                                                                    const int64_t* a_off, const int64_t* b_off, uint64_t a_stride,
+                                                                    uint64_t b_stride) {
+  constexpr int PER = W == 1 ? 4 : 1;
+  __shared__ T wsum[W];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, w = W == 1 ? 0 : wave;
+  const uint32_t b = blockIdx.y;
+  const uint64_t e = (uint64_t)blockIdx.x * PER + (W == 1 ? wave : 0);
+  if (e >= (uint64_t)M * N) return;  // whole waves; blocks of several waves have one output
+  const uint32_t i = (uint32_t)(e / N), j = (uint32_t)(e % N);
+  const T* a = A + batch_offset(a_off, a_stride, b) + (ta ? (uint64_t)i : (uint64_t)i * K);
+  const T* bb = B + batch_offset(b_off, b_stride, b) + (tb ? (uint64_t)j * K : (uint64_t)j);
+  const uint64_t sa = ta ? M : 1, sb = tb ? 1 : N;
+  T acc = (T)0;
+  uint64_t k = (uint64_t)w * 64 + lane;
+  for (; k + 7 * 64 * W < K; k += 8 * 64 * W) {
+    T x[8], y[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) x[u] = a[(k + u * 64 * W) * sa], y[u] = bb[(k + u * 64 * W) * sb];
+#pragma unroll
+    for (int u = 0; u < 8; u++) acc = fma(x[u], y[u], acc);
+  }
+  for (; k < K; k += 64 * W) acc = fma(a[k * sa], bb[k * sb], acc);
+  T sum = rg_wave_sum(acc);
+  if constexpr (W > 1) {
+    if (lane == 0) wsum[w] = sum;
+    __syncthreads();
+    if (w != 0) return;
+    sum = wsum[0];
+#pragma unroll
+    for (int q = 1; q < W; q++) sum += wsum[q];
+  }
+  if (lane == 0) C[(uint64_t)b * M * N + e] = sum;
+}
+
+// fp64 products on v_mfma_f64_16x16x4_f64: four wave64s per block, WM x WN over the BM x BN tile and
+// WK over each step of KW WK k (their sums added in order at the end). Operands are staged through
+// LDS as [k][row], one step ahead in registers, zeros outside M, N and K. The instruction takes 64
+// cycles; with one staging buffer what bounds a tile is the loads and barriers of its steps, so the
+// steps are long (T 512 x 512 x 1024 on 32x32 tiles: 46 us with 16 k a step, 30 with 64). 1024 x 512
+// products of K = 512 take 22 us (24.8 of 78.6 TFLOP/s), where a thread per output took 560.
+template <int BM, int BN, int WM, int WN, int WK, int KW, bool TA, bool TB>
+__global__ void __launch_bounds__(256) k_gemm_f64(const double* __restrict__ A, const double* __restrict__ B, double* __restrict__ C, int M, int N,
+                                                  int K, const int64_t* a_off, const int64_t* b_off, uint64_t a_stride, uint64_t b_stride,
+                                                  uint32_t tiles_m, uint32_t tiles_n) {
+  static_assert(WM * WN * WK == 4, "four waves");
+  typedef double doublex4 __attribute__((ext_vector_type(4)));
+  constexpr int BK = KW * WK, TM = BM / WM / 16, TN = BN / WN / 16, PA = BM * BK / 256, PB = BN * BK / 256;
+  constexpr int LDA = BM + 1, LDB = BN + 1;
+  __shared__ double as[BK * LDA], bs[BK * LDB];
+  __shared__ double part[WK > 1 ? (WK - 1) * BM * BN : 1];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, lo = lane >> 4;
+  const int wk = wave / (WM * WN), wm = wave / WN % WM, wn = wave % WN;
+  const TileIndex ti = tile_of(blockIdx.x, gridDim.x, tiles_m, tiles_n, 1);
+  const int m0 = ti.tm * BM, n0 = ti.tn * BN;
+  const double* a = A + batch_offset(a_off, a_stride, ti.z);
+  const double* b = B + batch_offset(b_off, b_stride, ti.z);
+  double va[PA], vb[PB];
+  // Element e of a step: along k where the operand is K-contiguous, along its rows otherwise.
+  auto load = [&](int k0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < PA; q++) {
+      const int e = q * 256 + tid, r = TA ? e % BM : e / BK, k = k0 + (TA ? e / BM : e % BK), row = m0 + r;
+      const bool ok = row < M && k < K;
+      const double x = a[ok ? (TA ? (int64_t)k * M + row : (int64_t)row * K + k) : 0];
+      va[q] = ok ? x : 0.0;
+    }
+#pragma unroll
+    for (int q = 0; q < PB; q++) {
+      const int e = q * 256 + tid, r = TB ? e / BK : e % BN, k = k0 + (TB ? e % BK : e / BN), col = n0 + r;
+      const bool ok = col < N && k < K;
+      const double x = b[ok ? (TB ? (int64_t)col * K + k : (int64_t)k * N + col) : 0];
+      vb[q] = ok ? x : 0.0;
+    }
+  };
+  auto store = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < PA; q++) {
+      const int e = q * 256 + tid;
+      as[(TA ? e / BM : e % BK) * LDA + (TA ? e % BM : e / BK)] = va[q];
+    }
+#pragma unroll
+    for (int q = 0; q < PB; q++) {
+      const int e = q * 256 + tid;
+      bs[(TB ? e % BK : e / BN) * LDB + (TB ? e / BK : e % BN)] = vb[q];
+    }
+  };
+  doublex4 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int n = 0; n < TN; n++) acc[i][n] = doublex4{0.0, 0.0, 0.0, 0.0};
+  load(0);
+  store();
+  __syncthreads();
+  for (int k0 = 0; k0 < K; k0 += BK) {
+    if (k0 + BK < K) load(k0 + BK);
+#pragma unroll
+    for (int kk = 0; kk < KW; kk += 4) {
+      const int k = wk * KW + kk + lo;
+      double x[TM], y[TN];
+#pragma unroll
+      for (int i = 0; i < TM; i++) x[i] = as[k * LDA + (wm * TM + i) * 16 + li];
+#pragma unroll
+      for (int n = 0; n < TN; n++) y[n] = bs[k * LDB + (wn * TN + n) * 16 + li];
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int n = 0; n < TN; n++) acc[i][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i], y[n], acc[i][n], 0, 0, 0);
+    }
+    __syncthreads();
+    if (k0 + BK < K) {
+      store();
+      __syncthreads();
+    }
+  }
+  // Register r of lane l holds row 4 r + l / 16, column l % 16 of its 16x16 tile.
+  if constexpr (WK > 1) {
+    if (wk > 0)
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int n = 0; n < TN; n++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) part[((wk - 1) * BM + i * 16 + 4 * r + lo) * BN + n * 16 + li] = acc[i][n][r];
+    __syncthreads();
+    if (wk > 0) return;
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int n = 0; n < TN; n++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+          for (int q = 0; q < WK - 1; q++) acc[i][n][r] += part[(q * BM + i * 16 + 4 * r + lo) * BN + n * 16 + li];
+  }
+  double* c = C + (uint64_t)ti.z * M * N;
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int n = 0; n < TN; n++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int row = m0 + (wm * TM + i) * 16 + 4 * r + lo, col = n0 + (wn * TN + n) * 16 + li;
+        if (row < M && col < N) c[(uint64_t)row * N + col] = acc[i][n][r];
+      }
 }
 
 // ---- skinny fp32 products: HBM-bound shapes streamed at full bandwidth -------------------------
@@ -171,13 +332,27 @@ __global__ void __launch_bounds__(256) k_gemm_plain(const T* __restrict__ A, con
 // speed them up, the number of bytes in flight can. Each kernel reads its large operand exactly
 // once with 16-byte loads and fixes the order of every sum, so results are deterministic.
 
-// C (M <= MR rows) = op(A) B with B row-major K x N (N % 4 == 0, 16-byte aligned). A block of
+// A lane's four columns of these kernels start at a multiple of four, the last ones moved back to
+// N - 4 where N is no multiple of four: the columns two lanes then share get the same sums from both.
+// Rows need only 4-byte alignment (rowx4).
+
+// C (M <= MR rows) = op(A) B with B row-major K x N (N >= 4). A block of
 // four waves owns 256 columns (a float4 per lane) and one K split; its waves take consecutive
 // quarters of the split, sum their k in increasing order, and combine in wave order through
 // LDS. With several splits, split s writes partials [s][M N], summed in split order afterwards.
 // The loop has no branches: a wave's K range is made uniform (readfirstlane), so op(A) values are
-// scalar loads that never wait on the B rows in flight; rows m >= M read row M - 1 and columns
-// past N read the last column, and neither is stored.
+// scalar loads that never wait on the B rows in flight; rows m >= M read row M - 1 and are not
+// stored.
+__device__ __forceinline__ float4 row4(const float* p) {
+  const rowx4 x = *(const rowx4*)p;
+  return make_float4(x[0], x[1], x[2], x[3]);
+}
+// The first `left` of four values, zeros after them.
+__device__ __forceinline__ float4 row4(const float* p, int left) {
+  if (left >= 4) return row4(p);
+  return make_float4(left > 0 ? p[0] : 0.f, left > 1 ? p[1] : 0.f, left > 2 ? p[2] : 0.f, 0.f);
+}
+
 template <int MR>
 struct RowsLds {
   static constexpr int FLOAT4S = 3 * MR * 64;  // the sums of waves 1..3; wave 0 keeps its own
@@ -208,7 +383,7 @@ __device__ __forceinline__ void skinny_rows_block(const float* __restrict__ A, c
   for (; k + UNROLL <= kw1; k += UNROLL) {
     float4 b[UNROLL];
 #pragma unroll
-    for (int u = 0; u < UNROLL; u++) b[u] = *(const float4*)(B + (uint64_t)(k + u) * N + colr);
+    for (int u = 0; u < UNROLL; u++) b[u] = row4(B + (uint64_t)(k + u) * N + colr);
 #pragma unroll
     for (int u = 0; u < UNROLL; u++)
 #pragma unroll
@@ -218,7 +393,7 @@ __device__ __forceinline__ void skinny_rows_block(const float* __restrict__ A, c
       }
   }
   for (; k < kw1; k++) {
-    const float4 b = *(const float4*)(B + (uint64_t)k * N + colr);
+    const float4 b = row4(B + (uint64_t)k * N + colr);
 #pragma unroll
     for (int m = 0; m < MR; m++) {
       const float a = Ac[(uint64_t)min(m, M - 1) * sm + (uint64_t)k * sk];
@@ -240,12 +415,11 @@ __device__ __forceinline__ void skinny_rows_block(const float* __restrict__ A, c
         const float4 x = red[w][m][lane];
         v = make_float4(v.x + x.x, v.y + x.y, v.z + x.z, v.w + x.w);
       }
-      *(float4*)(dst + (uint64_t)m * N + col) = v;
+      *(rowx4*)(dst + (uint64_t)m * N + colr) = rowx4{v.x, v.y, v.z, v.w};
     }
 }
 
-// C (M <= MR rows) = A B^T with A row-major M x K and B stored N x K (N % NC == 0, K % 256 == 0,
-// both 16-byte aligned): every output is the dot product of two contiguous rows. A block owns
+// C (M <= MR rows) = A B^T with A row-major M x K and B stored N x K (N >= NC): every output is the dot product of two contiguous rows. A block owns
 // 4 NC consecutive columns of C (NC per wave) and one K split of `kps` (a multiple of 256, at
 // most DOT_KPS); it copies its A panel to LDS while its first B rows load, so the loop's only
 // global loads are the B rows, four float4 steps deep. Lanes take k in float4 steps 256 apart, each lane summing its
@@ -272,20 +446,21 @@ __device__ __forceinline__ void skinny_dot_block(const float* __restrict__ A, co
   const int k0 = split * kps, len = min(K - k0, kps);
   const int n0 = (bx * 4 + (threadIdx.x >> 6)) * NC;
   const bool active = n0 < N;
-  const int nr = active ? n0 : N - NC;  // an idle wave reads valid rows and stores nothing
+  const int nr = min(n0, N - NC);  // an idle wave reads valid rows and stores nothing
   // The first four steps of B rows are issued before the panel copy, so their latency overlaps it.
   auto load = [&](float4 (&b)[4][NC], int kk) {
 #pragma unroll
     for (int h = 0; h < 4; h++)
 #pragma unroll
       for (int c = 0; c < NC; c++)
-        b[h][c] = kk + h * 256 < len ? *(const float4*)(B + (uint64_t)(nr + c) * K + k0 + kk + h * 256) : make_float4(0.f, 0.f, 0.f, 0.f);
+        b[h][c] = row4(B + (uint64_t)(nr + c) * K + k0 + kk + h * 256, len - kk - h * 256);
   };
   float4 b[4][NC];
   load(b, lane * 4);
-  for (int q = threadIdx.x; q < MR * (len / 4); q += 256) {
-    const int m = q / (len / 4), c = q % (len / 4);
-    panel[m][c] = *(const float4*)(A + (uint64_t)min(m, M - 1) * K + k0 + 4 * c);
+  const int len4 = (len + 3) / 4;
+  for (int q = threadIdx.x; q < MR * len4; q += 256) {
+    const int m = q / len4, c = q % len4;
+    panel[m][c] = row4(A + (uint64_t)min(m, M - 1) * K + k0 + 4 * c, len - 4 * c);
   }
   __syncthreads();
   if (!active) return;
@@ -313,11 +488,11 @@ __device__ __forceinline__ void skinny_dot_block(const float* __restrict__ A, co
 #pragma unroll
     for (int c = 0; c < NC; c++) {
       const float v = rg_wave_sum(acc[m][c]);
-      if (m < M && lane == 0) dst[(uint64_t)m * N + n0 + c] = v;
+      if (m < M && lane == 0) dst[(uint64_t)m * N + nr + c] = v;
     }
 }
 
-// C (M x N, N % 4 == 0) = op(A) op(B) with K <= KR (an outer product of a few vectors): write
+// C (M x N, N >= 4) = op(A) op(B) with K <= KR (an outer product of a few vectors): write
 // bound. A block of four waves owns 256 columns; each lane keeps its float4 of every op(B) row in
 // registers and walks the wave's rows, reading op(A)'s row values as wave-uniform scalars. The
 // output is written with non-temporal stores: it is large (a full matrix from a few vectors) and
@@ -329,15 +504,15 @@ __device__ __forceinline__ void outer_block(const float* __restrict__ A, const f
                                             int K, int rows_per_wave, uint32_t bx, uint32_t by) {
   const ConstOperand Ac = (ConstOperand)A;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int col = (bx * 64 + lane) * 4;
-  if (col >= N) return;
+  if ((bx * 64 + lane) * 4 >= N) return;
+  const int col = min((int)(bx * 64 + lane) * 4, N - 4);
   // Rows k >= K are zeros: the extra terms add exact zeros, so the sums are unchanged.
   float4 b[KR];
 #pragma unroll
   for (int k = 0; k < KR; k++) {
     if (k < K) {
       if (TB) b[k] = make_float4(B[(uint64_t)col * K + k], B[(uint64_t)(col + 1) * K + k], B[(uint64_t)(col + 2) * K + k], B[(uint64_t)(col + 3) * K + k]);
-      else b[k] = *(const float4*)(B + (uint64_t)k * N + col);
+      else b[k] = row4(B + (uint64_t)k * N + col);
     } else {
       b[k] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
@@ -350,7 +525,7 @@ __device__ __forceinline__ void outer_block(const float* __restrict__ A, const f
       const float a = k < K ? (TA ? Ac[(uint64_t)k * M + i] : Ac[(uint64_t)i * K + k]) : 0.f;
       acc = make_float4(fmaf(a, b[k].x, acc.x), fmaf(a, b[k].y, acc.y), fmaf(a, b[k].z, acc.z), fmaf(a, b[k].w, acc.w));
     }
-    __builtin_nontemporal_store(floatx4{acc.x, acc.y, acc.z, acc.w}, (floatx4*)(C + (uint64_t)i * N + col));
+    __builtin_nontemporal_store(rowx4{acc.x, acc.y, acc.z, acc.w}, (rowx4*)(C + (uint64_t)i * N + col));
   }
 }
 
@@ -489,12 +664,15 @@ struct Skinny {
   bool ta = false;
 };
 
+// fp32 products on matrix cores: both sides at least 32, or at least 16 at a K under 512 (attention
+// heads of 16 or 24; a longer K streams).
 bool use_mfma(int dtype, uint64_t m, uint64_t n, uint64_t k) {
-  return dtype == RG_F32 && m >= 32 && n >= 32 && k >= 8 && m * n * k >= (1u << 18);
+  const uint64_t side = k < 512 ? 16 : 32;
+  return dtype == RG_F32 && m >= side && n >= side && k >= 8 && m * n * k >= (1u << 18);
 }
 
-// Which skinny kernel a product takes, from shapes and flags alone (alignment is checked at
-// launch; an unaligned operand falls back to the general kernels).
+// Which skinny kernel a product takes, from shapes and flags alone. Every size goes: a chain of
+// 8 x 2050 x 2050 products on the plain kernel instead took 10 times as long.
 Skinny skinny_plan(int dtype, uint64_t m, uint64_t n, uint64_t k, uint64_t batch, bool ta, bool tb) {
   Skinny sk;
   if (dtype != RG_F32 || batch != 1 || m == 0 || n == 0 || k == 0) return sk;
@@ -502,13 +680,13 @@ Skinny skinny_plan(int dtype, uint64_t m, uint64_t n, uint64_t k, uint64_t batch
   sk.n = n;
   sk.k = k;
   sk.ta = ta;
-  if (k <= 16 && n % 4 == 0 && m * n >= (1ull << 14)) {
+  if (k <= 16 && n >= 4 && m * n >= (1ull << 14)) {
     sk.kind = SKINNY_OUTER;
     return sk;
   }
   if (m <= 16 && k >= 512 && n >= 64) {
-    if (!tb && n % 4 == 0) sk.kind = SKINNY_ROWS;
-    else if (tb && !ta && k % 256 == 0 && n % 4 == 0) sk.kind = SKINNY_DOT;
+    if (!tb) sk.kind = SKINNY_ROWS;
+    else if (!ta) sk.kind = SKINNY_DOT;
     if (sk.kind != SKINNY_NONE) return sk;
   }
   if (n == 1 && k >= 512 && m >= 64) {
@@ -517,10 +695,8 @@ Skinny skinny_plan(int dtype, uint64_t m, uint64_t n, uint64_t k, uint64_t batch
     sk.m = 1;
     sk.n = m;
     sk.ta = false;
-    if (ta && m % 4 == 0) sk.kind = SKINNY_ROWS;
-    else if (!ta && k % 256 == 0 && m % 4 == 0) sk.kind = SKINNY_DOT;
-    if (sk.kind != SKINNY_NONE) return sk;
-    sk = Skinny{};
+    sk.kind = ta ? SKINNY_ROWS : SKINNY_DOT;
+    return sk;
   }
   // Outputs with both sides at least 32 (a tied embedding's gradient, 96 x 128 over 4096 rows)
   // go to the MFMA tiles, which read both operands in coalesced tiles.
@@ -596,7 +772,7 @@ TileCfg pick_tile(uint64_t m, uint64_t n, uint64_t k, uint64_t batch) {
     if (m >= 128 && tile_count(SPLIT_128x64, m, n, batch) >= 768) return SPLIT_128x64;
     return SPLIT_64x64;
   }
-  if (n <= 96 && n % 32 == 0) return {128, 32, 32, 4, 1, 0};
+  if ((n <= 96 && n % 32 == 0) || n < 32) return {128, 32, 32, 4, 1, 0};
   if (m <= 32) return {32, 128, 32, 1, 4, 0};
   const TileCfg t64 = {64, 64, 32, 2, 2, 0};
   return filled(t64) < 256 ? TileCfg{32, 32, 32, 2, 2, 0} : t64;
@@ -664,8 +840,11 @@ void launch_mfma(hipStream_t s, const TileCfg& t, bool ta, bool tb, int mode, co
 
 }  // namespace
 
+// Products priced by bytes: the streamed ones, but for dot products over a K that is no multiple of
+// 256, whose price stays the operations'.
 bool gemm_streamed(int dtype, uint64_t m, uint64_t n, uint64_t k, uint64_t batch, bool ta, bool tb) {
-  return skinny_plan(dtype, m, n, k, batch, ta, tb).kind != SKINNY_NONE;
+  const Skinny sk = skinny_plan(dtype, m, n, k, batch, ta, tb);
+  return sk.kind != SKINNY_NONE && !(sk.kind == SKINNY_DOT && k % 256 != 0);
 }
 
 int gemm_splits(int dtype, uint64_t m, uint64_t n, uint64_t k, uint64_t batch, bool ta, bool tb) {
@@ -704,10 +883,9 @@ uint64_t gemm_workspace(int dtype, uint64_t m, uint64_t n, uint64_t k, uint64_t 
   return s > 1 ? (uint64_t)s * batch * m * n * sizeof(float) : 0;
 }
 
-// Launches the skinny kernel of `sk`; false when an operand is not aligned for it.
+// Launches the skinny kernel of `sk`; false for a product with a bias.
 bool gemm_skinny(hipStream_t s, const GemmArgs& g, const Skinny& sk) {
-  auto aligned = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
-  if (g.bias || g.a_off || g.b_off || !aligned(g.c)) return false;
+  if (g.bias || g.a_off || g.b_off) return false;
   // With the roles exchanged (n == 1) the vector is the left operand of one row.
   const float* A = (const float*)(sk.swapped ? g.b : g.a);
   const float* B = (const float*)(sk.swapped ? g.a : g.b);
@@ -731,7 +909,6 @@ bool gemm_skinny(hipStream_t s, const GemmArgs& g, const Skinny& sk) {
     // 16 rows per wave for tall outputs; fewer for short ones, so more waves share the work.
     const int rows = std::max(1, std::min(16, M / 256));
     dim3 grid((uint32_t)((N + 255) / 256), (uint32_t)((M + 4 * rows - 1) / (4 * rows)));
-    if (!g.tb && !aligned(B)) return false;
 #define RG_OUTER_K(KR_, TA_, TB_) hipLaunchKernelGGL((k_gemm_outer<KR_, TA_, TB_>), grid, dim3(256), 0, s, A, B, C, M, N, K, rows)
 #define RG_OUTER(TA_, TB_)                   \
   do {                                       \
@@ -760,7 +937,6 @@ bool gemm_skinny(hipStream_t s, const GemmArgs& g, const Skinny& sk) {
     }
   };
   if (kind == SKINNY_DOT) {
-    if (!aligned(A) || !aligned(B)) return false;
     constexpr int NC = 4;
     const int kps = skinny_dot_kps(sk.m, sk.k);
     const int splits = (K + kps - 1) / kps;
@@ -771,7 +947,6 @@ bool gemm_skinny(hipStream_t s, const GemmArgs& g, const Skinny& sk) {
     sum_splits(out, splits);
     return true;
   }
-  if (!aligned(B)) return false;
   const int splits0 = skinny_rows_splits(sk.n, sk.k);
   const int kps = (K + splits0 - 1) / splits0;
   const int splits = (K + kps - 1) / kps;
@@ -829,8 +1004,62 @@ bool on_mfma_tiles(const GemmArgs& g) {
 
 }  // namespace
 
-// Plan slots start 256-byte aligned, so a lowered product always meets the skinny kernels'
-// alignment. A product whose K-split partials are deferred to the fold area must leave exactly
+namespace {
+
+// fp64 tiles: 64x64 at a block and a half per CU, 32x32 at one, else 16x16 with the four waves sharing
+// each step of K (T 128 x 512 x 1024, 256 such tiles: 14 us, where a 32x32 tile walks that K in 30).
+// False for sides under 16, which waste the tile.
+bool gemm_f64(hipStream_t s, const GemmArgs& g) {
+  if (g.m < 16 || g.n < 16 || g.k < 4) return false;
+  auto tiles = [&](uint64_t t) { return ((g.m + t - 1) / t) * ((g.n + t - 1) / t) * g.batch; };
+  const int side = tiles(64) >= 384 ? 64 : tiles(32) >= 256 ? 32 : 16;
+  if (tiles(side) >= (1ull << 31)) return false;
+  const uint32_t tm = (uint32_t)((g.m + side - 1) / side), tn = (uint32_t)((g.n + side - 1) / side);
+  const dim3 grid((uint32_t)tiles(side));
+#define RG_F64(S_, WM_, WK_, KW_, TA_, TB_)                                                                                                \
+  hipLaunchKernelGGL((k_gemm_f64<S_, S_, WM_, WM_, WK_, KW_, TA_, TB_>), grid, dim3(256), 0, s, (const double*)g.a, (const double*)g.b, (double*)g.c, \
+                     (int)g.m, (int)g.n, (int)g.k, g.a_off, g.b_off, g.a_stride, g.b_stride, tm, tn)
+#define RG_F64_FLAGS(S_, WM_, WK_, KW_)                    \
+  do {                                                \
+    if (g.ta && g.tb) RG_F64(S_, WM_, WK_, KW_, true, true); \
+    else if (g.ta) RG_F64(S_, WM_, WK_, KW_, true, false); \
+    else if (g.tb) RG_F64(S_, WM_, WK_, KW_, false, true); \
+    else RG_F64(S_, WM_, WK_, KW_, false, false);          \
+  } while (0)
+  if (side == 64) RG_F64_FLAGS(64, 2, 1, 32);
+  else if (side == 32) RG_F64_FLAGS(32, 2, 1, 64);
+  else RG_F64_FLAGS(16, 1, 4, 32);
+#undef RG_F64_FLAGS
+#undef RG_F64
+  return true;
+}
+
+// Products off the fp32 tiles and the streaming kernels.
+template <class T>
+void gemm_small(hipStream_t s, const GemmArgs& g) {
+  if (std::is_same<T, double>::value && gemm_f64(s, g)) return;
+  const uint64_t outputs = g.m * g.n;
+  const bool rows = g.n == 1 && !g.ta;  // every output a contiguous row against one vector
+  // A wave per output where K gives its lanes work and the outputs alone do not fill the chip.
+  if (g.k >= 32 && (outputs * g.batch <= 16384 || rows) && outputs < (1ull << 31)) {
+    const int w = outputs * g.batch >= 2048 ? 1 : g.k <= 512 ? 1 : g.k <= 2048 ? 4 : 16;
+    const dim3 grid((uint32_t)(w == 1 ? (outputs + 3) / 4 : outputs), (uint32_t)g.batch);
+#define RG_DOTS(W_)                                                                                                                        \
+  hipLaunchKernelGGL((k_gemm_dots<T, W_>), grid, dim3(W_ == 1 ? 256 : 64 * W_), 0, s, (const T*)g.a, (const T*)g.b, (T*)g.c, (uint32_t)g.m, \
+                     (uint32_t)g.n, (uint32_t)g.k, g.ta, g.tb, g.a_off, g.b_off, g.a_stride, g.b_stride)
+    if (w == 1) RG_DOTS(1);
+    else if (w == 4) RG_DOTS(4);
+    else RG_DOTS(16);
+#undef RG_DOTS
+    return;
+  }
+  hipLaunchKernelGGL(k_gemm_plain<T>, dim3((uint32_t)((outputs + 255) / 256), (uint32_t)g.batch), dim3(256), 0, s, (const T*)g.a, (const T*)g.b,
+                     (T*)g.c, (uint32_t)g.m, (uint32_t)g.n, (uint32_t)g.k, g.ta, g.tb, g.a_off, g.b_off, g.a_stride, g.b_stride);
+}
+
+}  // namespace
+
+// A product whose K-split partials are deferred to the fold area must leave exactly
 // the planned number of partial products there: a launch that would take another path (the
 // streaming kernel refusing its operands, another split count) throws instead, and the error is
 // latched like any failed launch, rather than letting the fold overwrite C with stale partials.
@@ -856,13 +1085,8 @@ void gemm(hipStream_t s, const GemmArgs& g) {
     return;
   }
   if (g.defer_split) throw std::runtime_error("deferred K-split product on the plain kernel, which does not split K");
-  dim3 grid((uint32_t)((g.m * g.n + 255) / 256), (uint32_t)g.batch);
-  if (g.dtype == RG_F32)
-    hipLaunchKernelGGL(k_gemm_plain<float>, grid, dim3(256), 0, s, (const float*)g.a, (const float*)g.b, (float*)g.c, (uint32_t)g.m,
-                       (uint32_t)g.n, (uint32_t)g.k, g.ta, g.tb, g.a_off, g.b_off, g.a_stride, g.b_stride);
-  else
-    hipLaunchKernelGGL(k_gemm_plain<double>, grid, dim3(256), 0, s, (const double*)g.a, (const double*)g.b, (double*)g.c, (uint32_t)g.m,
-                       (uint32_t)g.n, (uint32_t)g.k, g.ta, g.tb, g.a_off, g.b_off, g.a_stride, g.b_stride);
+  if (g.dtype == RG_F32) gemm_small<float>(s, g);
+  else gemm_small<double>(s, g);
   if (g.bias && g.dtype == RG_F32) {
     const uint64_t total = g.m * g.n * g.batch;
     hipLaunchKernelGGL(k_add_bias, dim3((uint32_t)((total + 255) / 256)), dim3(256), 0, s, (float*)g.c, (const float*)g.bias, total, g.n);
@@ -873,13 +1097,11 @@ namespace {
 
 // Product `g` as a part of a grouped streaming launch: the kernel gemm_skinny would launch for
 // it, when that is the row, dot or outer-product kernel for at most 8 rows (or K), or the
-// tiny-output kernel of 4, 8 or 16 waves, its operands aligned for it, and its K splits, if any,
+// tiny-output kernel of 4, 8 or 16 waves, and its K splits, if any,
 // deferred to the fold area.
 bool stream_part_of(const GemmArgs& g, StreamPart* p) {
   if (g.m == 0 || g.n == 0 || g.batch != 1 || g.bias || g.a_off || g.b_off) return false;
-  auto aligned = [](const void* q) { return ((uintptr_t)q & 15) == 0; };
   const Skinny sk = skinny_plan(g.dtype, g.m, g.n, g.k, g.batch, g.ta, g.tb);
-  if (!aligned(g.c)) return false;
   const float* A = (const float*)(sk.swapped ? g.b : g.a);
   const float* B = (const float*)(sk.swapped ? g.a : g.b);
   const int M = (int)sk.m, N = (int)sk.n, K = (int)sk.k;
@@ -897,7 +1119,7 @@ bool stream_part_of(const GemmArgs& g, StreamPart* p) {
     q.gx = (uint32_t)(M * N);
     q.gy = 1;
   } else if (sk.kind == SKINNY_OUTER) {
-    if (K > 8 || (!g.tb && !aligned(B)) || (g.ta && g.tb) || g.defer_split) return false;
+    if (K > 8 || (g.ta && g.tb) || g.defer_split) return false;
     q.kind = g.ta ? STREAM_OUTER8_TN : g.tb ? STREAM_OUTER8_NT : STREAM_OUTER8_NN;
     // Half the single kernel's rows per wave, so twice its blocks: 8 rows for C5's 4096-row
     // outputs measured 3 us (4 %) faster per pass on MI355X than 16, and 6 alike, 4 or 32 slower.
@@ -906,7 +1128,7 @@ bool stream_part_of(const GemmArgs& g, StreamPart* p) {
     q.gx = (uint32_t)((N + 255) / 256);
     q.gy = (uint32_t)((M + 4 * q.arg - 1) / (4 * q.arg));
   } else if (sk.kind == SKINNY_DOT) {
-    if (M > 8 || !aligned(A) || !aligned(B)) return false;
+    if (M > 8) return false;
     const int kps = skinny_dot_kps(sk.m, sk.k), splits = (K + kps - 1) / kps;
     if (!split_ok(splits)) return false;
     q.kind = STREAM_DOT8;
@@ -915,7 +1137,7 @@ bool stream_part_of(const GemmArgs& g, StreamPart* p) {
     q.gx = (uint32_t)((N + 15) / 16);
     q.gy = (uint32_t)splits;
   } else if (sk.kind == SKINNY_ROWS) {
-    if (M > 8 || !aligned(B)) return false;
+    if (M > 8) return false;
     const int splits0 = skinny_rows_splits(sk.n, sk.k);
     const int kps = (K + splits0 - 1) / splits0, splits = (K + kps - 1) / kps;
     if (!split_ok(splits)) return false;
