@@ -109,6 +109,26 @@ __global__ void __launch_bounds__(64 * WM * WN, split_waves(BM, BN, U)) k_gemm_m
   if constexpr (N > 2) group_part<BM, BN, WM, WN, U, FLAGS, 2>(g.p[2], bid - g.p[1].blocks, smem);
 }
 
+// The same on 32x32 fp32 MFMA tiles: products too small to fill the chip alone (C3's input and weight
+// gradients, 256 to 512 blocks of 8-10 us, run side by side).
+template <int FLAGS, int I>
+__device__ __forceinline__ void small_part(const GroupPart& p, uint32_t bid, float* smem) {
+  constexpr bool TA = (FLAGS >> (2 * I + 1)) & 1, TB = (FLAGS >> (2 * I)) & 1;
+  StoreC epi{p.c, p.part, p.splits, (uint64_t)p.m * p.n};
+  gemm_f32_tile<32, 32, 32, 2, 2, TA, TB, LOAD_EVEN, 16>(p.a, p.b, p.m, p.n, p.k, nullptr, nullptr, 0, 0, p.splits, p.kps, p.bias, p.tm, p.tn, 1,
+                                                         epi, bid, p.blocks, smem);
+}
+
+template <int N, int FLAGS>
+__global__ void __launch_bounds__(256) k_gemm_f32_group(GroupParts g) {
+  __shared__ float smem[TileLds<32, 32, 32, false, true>::FLOATS];  // both operands K-contiguous: the largest
+  uint32_t bid = blockIdx.x;
+  if (bid < g.p[0].blocks) return small_part<FLAGS, 0>(g.p[0], bid, smem);
+  bid -= g.p[0].blocks;
+  if (N == 2 || bid < g.p[1].blocks) return small_part<FLAGS, 1>(g.p[1], bid, smem);
+  if constexpr (N > 2) small_part<FLAGS, 2>(g.p[2], bid - g.p[1].blocks, smem);
+}
+
 // Sums the K-split partial products in split order. Four outputs per thread (16-byte loads when
 // M N is a multiple of 4), all splits' loads issued before the adds.
 __global__ void __launch_bounds__(256) k_split_sum(const float* __restrict__ partial, float* __restrict__ C, uint64_t mn, int splits,
@@ -1172,10 +1192,13 @@ bool gemm_group(hipStream_t s, const GemmArgs* g, int count, bool launch) {
       return true;
     }
   }
-  // One split tile for all, 128x128: every split tile sums a K range's terms in the same order, so a
-  // product picked for a smaller one keeps its bits, and its K splits. K-split partials, if any, must
-  // be the deferred kind: a split sum after the grouped launch would be a second launch anyway.
-  const TileCfg t = SPLIT_128x128_2;
+  // One tile for all. Split tiles: 128x128, since every split tile sums a K range's terms in the same
+  // order, so a product picked for a smaller one keeps its bits, and its K splits. fp32 tiles: 32x32
+  // whole ones. K-split partials, if any, must be the deferred kind: a split sum after the grouped
+  // launch would be a second launch anyway.
+  const TileCfg first = pick_tile(g[0].m, g[0].n, g[0].k, 1);
+  const bool split = first.split;
+  const TileCfg t = split ? SPLIT_128x128_2 : TileCfg{32, 32, 32, 2, 2, 0};
   int mode;
   Launch l[GROUP_MAX];
   int flags = 0;
@@ -1184,7 +1207,7 @@ bool gemm_group(hipStream_t s, const GemmArgs* g, int count, bool launch) {
     if (!on_mfma_tiles(g[i]) || g[i].batch != 1 || g[i].m % t.bm || g[i].n % t.bn) return false;
     const TileCfg own = pick_tile(g[i].m, g[i].n, g[i].k, 1);
     const int own_splits = split_count(own, g[i].m, g[i].n, g[i].k, 1);
-    if (!own.split || (own_splits > 1 && !g[i].defer_split)) return false;
+    if ((own.split != 0) != split || (!split && (own.bm != 32 || own.bn != 32)) || (own_splits > 1 && !g[i].defer_split)) return false;
     mfma_launch(g[i], t, own_splits, &mode, &l[i]);
     if (mode != 0 || (i + 1 < count && l[i].grid.x % 8 != 0)) return false;
     flags |= ((g[i].ta ? 2 : 0) | (g[i].tb ? 1 : 0)) << (2 * i);
@@ -1194,9 +1217,8 @@ bool gemm_group(hipStream_t s, const GemmArgs* g, int count, bool launch) {
   // pair, with fc2's weight gradient ahead of them as a triple; and the attention projection's
   // weight gradient with the q, k, v projection's, which do not fill the chip alone (64 and 192
   // blocks) and so go together rather than each with its input gradient.
-  if (small && (large || flags != (2 | 2 << 2))) return false;
+  if (split && small && (large || flags != (2 | 2 << 2))) return false;
   constexpr int T = 2, N = 1;  // (ta, tb) = (true, false) and (false, true)
-  const dim3 block(64 * t.wm * t.wn);
   GroupParts parts{};
   uint32_t blocks = 0;
   for (int i = 0; i < count; i++) {
@@ -1204,10 +1226,11 @@ bool gemm_group(hipStream_t s, const GemmArgs* g, int count, bool launch) {
                            l[i].grid.x};
     blocks += l[i].grid.x;
   }
-#define RG_GROUP(COUNT_, FLAGS_)                                                                                      \
-  if (count == COUNT_ && flags == (FLAGS_)) {                                                                         \
-    if (launch) hipLaunchKernelGGL((k_gemm_mfma_group<128, 128, 2, 4, 2, COUNT_, FLAGS_>), dim3(blocks), block, 0, s, parts); \
-    return true;                                                                                                      \
+#define RG_GROUP(COUNT_, FLAGS_)                                                                                                   \
+  if (count == COUNT_ && flags == (FLAGS_)) {                                                                                      \
+    if (launch && split) hipLaunchKernelGGL((k_gemm_mfma_group<128, 128, 2, 4, 2, COUNT_, FLAGS_>), dim3(blocks), dim3(512), 0, s, parts); \
+    else if (launch) hipLaunchKernelGGL((k_gemm_f32_group<COUNT_, FLAGS_>), dim3(blocks), dim3(256), 0, s, parts);                  \
+    return true;                                                                                                                   \
   }
   RG_GROUP(2, N | T << 2)
   RG_GROUP(2, T | N << 2)
