@@ -254,7 +254,9 @@ class Tensor(Value):
         return self._t.dtype
 
     def numpy(self):
-        return np.frombuffer(self._t.tobytes(), dtype=self.dtype).reshape(self.shape).copy()
+        out = np.empty(self.shape, self.dtype)
+        self._t.copy_into(out)
+        return out
 
     def __array__(self, dtype=None, copy=None):
         out = self.numpy()

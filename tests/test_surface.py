@@ -449,3 +449,15 @@ def test_sampling_filters_keep_the_right_tokens():
     c = rg.compile(lambda k: random.categorical(k, nn.top_k_logits(rg.tensor(np.log([[0.5, 0.2, 0.3]] * 400), "float32"), 2)),
                    (random.key(0),))
     assert set(c(random.key(3)).tolist()) == {0, 2}
+
+
+def test_numpy_copies_every_size_whole():
+    """`Tensor.numpy` gives a new writable array, whether one thread or several copy it."""
+    import numpy as np
+    for shape in [(), (0, 3), (7,), (2, 1, 5), (1 << 20,), (3, 1 << 21)]:
+        a = np.arange(int(np.prod(shape)), dtype=np.float32).reshape(shape)
+        t = rg.tensor(a)
+        b = t.numpy()
+        assert b.shape == a.shape and b.dtype == a.dtype and np.array_equal(a, b) and b.flags.writeable
+        b += 1
+        assert np.array_equal(t.numpy(), a)
