@@ -886,6 +886,10 @@ int gemm_splits(int dtype, uint64_t m, uint64_t n, uint64_t k, uint64_t batch, b
   return (int)((k + kps - 1) / kps);
 }
 
+bool gemm_outer_product(uint64_t m, uint64_t n, uint64_t k, bool ta, bool tb) {
+  return skinny_plan(RG_F32, m, n, k, 1, ta, tb).kind == SKINNY_OUTER;
+}
+
 bool gemm_epilogue_tile(int dtype, uint64_t m, uint64_t n, uint64_t k, bool ta, bool tb, GemmTile* out) {
   if (m == 0 || n == 0 || m >= (1ull << 31) || n >= (1ull << 31) || k >= (1ull << 31)) return false;
   if (skinny_plan(dtype, m, n, k, 1, ta, tb).kind != SKINNY_NONE || !use_mfma(dtype, m, n, k)) return false;

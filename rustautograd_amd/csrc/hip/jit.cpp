@@ -58,6 +58,16 @@ std::string expr(int op, const std::vector<std::string>& a) {
 constexpr int EW_UNROLL = 1;
 constexpr uint64_t EW_BLOCKS = 16 * 256;
 
+// A group with outer products inside: a wave owns 256 columns and walks OUTER_ROWS rows,
+// OUTER_UNROLL at a time. It is bound by the group's own loads and stores, so what counts is many
+// short waves: a step of a matrix chain with SGD on its two 4096 x 4096 weights, their gradients
+// of K = 8 (256 MB read and written), takes 123 us at 8 rows by 2, 124 at 16 rows (by 1 or by 2),
+// 130 at 32 or 64 (by 2, 4 or 8), and 166 with the gradients stored and loaded; at K = 16 179, 184
+// to 187, 185 to 188 and 236. At 2048 and below all are within 2 % (66 against 77 us at 2048,
+// K = 4; 55 against 57 at 516, K = 3).
+constexpr int64_t OUTER_ROWS = 8;
+constexpr int OUTER_UNROLL = 2;
+
 std::string generate(const rgplan::Fused& f, const std::string& name, FusedKernel* k, bool device_fn) {
   const bool dbl = f.dtype == RG_F64;
   const char* T = dbl ? "double" : "float";
@@ -303,6 +313,106 @@ std::string generate_gemm(const rgplan::Fused& f, int64_t c_slot, bool store_c, 
   k->name = name;
   k->block = (uint32_t)nt;
   k->vec = 1;
+  return s.str();
+}
+
+std::string generate_outer(const rgplan::Fused& f, int64_t m, int64_t n, const std::vector<OuterProduct>& products, const std::string& name,
+                           FusedKernel* k) {
+  if (f.dtype != RG_F32 || n % 4 != 0 || m * n != f.n) throw std::runtime_error("outer products in a group: fp32 rows of a multiple of four");
+  const int64_t gx = (n / 4 + 63) / 64, rows = OUTER_ROWS;
+  const int U = OUTER_UNROLL;
+  const bool whole = m % U == 0;
+  k->name = name;
+  k->vec = 4 * U;
+  k->grid = (uint32_t)(gx * ((m + 4 * rows - 1) / (4 * rows)));
+  auto product_at = [&](int64_t slot) {
+    for (size_t p = 0; p < products.size(); p++)
+      if (products[p].slot == slot) return (int)p;
+    return -1;
+  };
+  bool alias = false;
+  for (auto& o : f.outputs)
+    for (auto& in : f.inputs) alias |= in.slot == o.second && product_at(in.slot) < 0;
+  const char* R = alias ? "" : "__restrict__ ";
+  std::ostringstream s;
+  s << "extern \"C\" __global__ void __launch_bounds__(" << TPB << ") " << name << "(";
+  for (size_t j = 0; j < f.inputs.size(); j++)
+    if (product_at(f.inputs[j].slot) < 0) s << "const float* " << R << "in" << j << ", ";
+  for (size_t j = 0; j < f.outputs.size(); j++) s << "float* " << R << "out" << j << ", ";
+  for (size_t p = 0; p < products.size(); p++)
+    s << (p ? ", " : "") << "const float* __restrict__ A" << p << ", const float* __restrict__ B" << p;
+  s << ") {\n  typedef const __attribute__((address_space(4))) float* Uniform;\n";
+  s << "  const unsigned int lane = threadIdx.x & 63u, col = (blockIdx.x % " << gx << "u * 64u + lane) * 4u;\n";
+  s << "  if (col >= " << n << "u) return;\n";
+  // Every op(B) row's four columns of the lane, kept for all its rows.
+  for (size_t p = 0; p < products.size(); p++) {
+    const auto& o = products[p];
+    s << "  float b" << p << "[" << o.k << "][4];\n";
+    s << "#pragma unroll\n  for (int k = 0; k < " << o.k << "; k++) {\n";
+    if (o.tb) s << "#pragma unroll\n    for (int v = 0; v < 4; v++) b" << p << "[k][v] = B" << p << "[(col + v) * " << o.k << "u + k];\n";
+    else s << "    const float4 t = *(const float4*)(B" << p << " + k * " << n << "u + col); b" << p << "[k][0] = t.x; b" << p << "[k][1] = t.y; b" << p
+           << "[k][2] = t.z; b" << p << "[k][3] = t.w;\n";
+    s << "  }\n";
+  }
+  std::vector<std::string> reg_expr((size_t)f.regs), in_expr(f.inputs.size());
+  for (size_t j = 0; j < f.inputs.size(); j++) {
+    const auto& in = f.inputs[j];
+    const int p = product_at(in.slot);
+    const std::string x = "x" + std::to_string(j);
+    if (p >= 0) in_expr[j] = "a" + std::to_string(p) + "[v]";
+    else if (in.kind == RG_ARG_SPLAT) s << "  const float " << x << "s = in" << j << "[0];\n", in_expr[j] = x + "s";
+    else if (in.kind == RG_ARG_FULL || in.kind == RG_ARG_ROW) in_expr[j] = x + "[u][v]";
+    else throw std::runtime_error("outer products in a group: broadcast inputs are not supported");
+    if (in.reg >= 0) reg_expr[(size_t)in.reg] = in_expr[j];
+  }
+  s << "  const int row0 = (int)(blockIdx.x / " << gx << "u * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * " << rows << ", row1 = row0 + " << rows
+    << " < " << m << " ? row0 + " << rows << " : " << m << ";\n";
+  s << "  for (int r = row0; r < row1; r += " << U << ") {\n";
+  // Loads of every row of the pass first.
+  for (size_t j = 0; j < f.inputs.size(); j++)
+    if (product_at(f.inputs[j].slot) < 0 && f.inputs[j].kind != RG_ARG_SPLAT) s << "    float x" << j << "[" << U << "][4];\n";
+  auto each_row = [&] {
+    s << "#pragma unroll\n    for (int u = 0; u < " << U << "; u++) {\n";
+    if (!whole) s << "      if (r + u >= row1) break;\n";
+    s << "      const unsigned int e = (unsigned int)(r + u) * " << n << "u + col;\n";
+  };
+  each_row();
+  for (size_t j = 0; j < f.inputs.size(); j++) {
+    const auto& in = f.inputs[j];
+    if (product_at(in.slot) >= 0 || in.kind == RG_ARG_SPLAT) continue;
+    const std::string at = in.kind == RG_ARG_FULL ? "e" : "e % " + std::to_string(in.row_len) + "u";
+    s << "      { const float4 t = *(const float4*)(in" << j << " + " << at << "); x" << j << "[u][0] = t.x; x" << j << "[u][1] = t.y; x" << j
+      << "[u][2] = t.z; x" << j << "[u][3] = t.w; }\n";
+  }
+  s << "    }\n";
+  each_row();
+  for (size_t p = 0; p < products.size(); p++) {
+    const auto& o = products[p];
+    s << "      float a" << p << "[4] = {0.f, 0.f, 0.f, 0.f};\n";
+    s << "#pragma unroll\n      for (int k = 0; k < " << o.k << "; k++) {\n        const float w = ((Uniform)A" << p << ")[";
+    if (o.ta) s << "k * " << m << "u + (unsigned int)(r + u)";
+    else s << "(unsigned int)(r + u) * " << o.k << "u + k";
+    s << "];\n#pragma unroll\n        for (int v = 0; v < 4; v++) a" << p << "[v] = __builtin_fmaf(w, b" << p << "[k][v], a" << p << "[v]);\n      }\n";
+  }
+  for (size_t j = 0; j < f.outputs.size(); j++) s << "      float o" << j << "[4];\n";
+  s << "#pragma unroll\n      for (int v = 0; v < 4; v++) {\n";
+  for (auto& op : f.ops) {
+    std::vector<std::string> args;
+    for (auto& [is_reg, idx] : op.args) {
+      if (is_reg) {
+        const std::string& e = reg_expr[(size_t)idx];
+        args.push_back(e.empty() ? "r" + std::to_string(idx) : e);
+      } else {
+        args.push_back(in_expr[(size_t)idx]);
+      }
+    }
+    s << "        const float r" << op.reg << " = " << expr(op.op, args) << ";\n";
+  }
+  for (size_t j = 0; j < f.outputs.size(); j++) s << "        o" << j << "[v] = r" << f.outputs[j].first << ";\n";
+  s << "      }\n";
+  for (size_t j = 0; j < f.outputs.size(); j++)
+    s << "      *(float4*)(out" << j << " + e) = make_float4(o" << j << "[0], o" << j << "[1], o" << j << "[2], o" << j << "[3]);\n";
+  s << "    }\n  }\n}\n";
   return s.str();
 }
 

@@ -73,6 +73,22 @@ struct ProductTile {
 std::string generate_gemm(const rgplan::Fused& f, int64_t c_slot, bool store_c, const ProductTile& t, const std::string& name,
                           FusedKernel* k, int col_sum = -1);
 
+// An outer product computed inside the group that reads it: op(A) (M x K) op(B) (K x N), K at most
+// 16, read by the group through `slot`.
+struct OuterProduct {
+  int64_t slot;
+  int k;
+  bool ta, tb;
+};
+
+// Source of one kernel computing fused group `f` (a plain group over M x N elements, N a multiple
+// of 4) with its inputs at `products`' slots computed from their operands instead of loaded: each
+// value is the outer-product kernel's sum (k in increasing order, by fma, from zero). The kernel's
+// parameters are the group's other inputs in order, its outputs in order, then each product's A and B.
+std::string generate_outer(const rgplan::Fused& f, int64_t m, int64_t n, const std::vector<OuterProduct>& products, const std::string& name,
+                           FusedKernel* k);
+
+
 // Compiles all sources into one code object for gfx950 and resolves each kernel. Modules are
 // cached by source text for the life of the process. Throws std::runtime_error with the log.
 void compile(const std::string& source, std::vector<FusedKernel*>& kernels);

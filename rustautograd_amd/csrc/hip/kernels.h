@@ -195,6 +195,9 @@ bool gemm_streamed(int dtype, uint64_t m, uint64_t n, uint64_t k, uint64_t batch
 int gemm_splits(int dtype, uint64_t m, uint64_t n, uint64_t k, uint64_t batch, bool ta, bool tb);
 uint64_t gemm_workspace(int dtype, uint64_t m, uint64_t n, uint64_t k, uint64_t batch, bool ta, bool tb);
 
+// Whether a single (unbatched) fp32 product runs on the outer-product kernel (K at most 16).
+bool gemm_outer_product(uint64_t m, uint64_t n, uint64_t k, bool ta, bool tb);
+
 // The split tile (gemm_split.h) of a single (unbatched) fp32 product with a multiple of four
 // columns, when it runs unsplit on that tile (the form an elementwise epilogue takes): its template
 // arguments. False for any other product. `whole`: M and N are multiples of the tile.

@@ -120,7 +120,8 @@ struct Program {
   // Per step: for a product launched with others at another step (group_products), that step;
   // -1 otherwise.
   std::vector<int64_t> pair_of;
-  // Per step: for a column sum computed by a product epilogue's kernel, the step it runs at; -1.
+  // Per step: for a column sum computed by a product epilogue's kernel, or an outer product
+  // computed by the group that reads it, the step it runs at; -1.
   std::vector<int64_t> absorbed_into;
   // Runs of consecutive small, independent fused groups launched as one kernel (merge_sets):
   // merged[m] replaces steps first..last when all of them run; merged_at[k] is the run starting
@@ -813,7 +814,63 @@ struct Epilogues {
   // computes this sum, or -1.
   std::vector<int64_t> sum_of, sum_in;
   std::vector<int> sum_out;  // per group step: which of the group's outputs the sum reads
+  // Per group step: the outer products computed inside the group's kernel; per step: the group
+  // whose kernel computes this product, or -1.
+  std::vector<std::vector<size_t>> outer_of;
+  std::vector<int64_t> outer_in;
 };
+
+constexpr uint64_t OUTER_MAX_K = 32;  // of one group's outer products together: 4 registers a lane each
+
+// The outer products each large elementwise group can compute itself (a weight gradient of at most
+// 16 rows in a parameter update): group j walks product k's M x N outputs, N a multiple of 4, with
+// Full, Row (length a multiple of 4) and Splat inputs; nothing else reads the product, and its
+// operands are not written between it and the group, nor by the group, so that they can be read
+// at step j. The product is then neither stored nor loaded: the group's kernel does at most
+// OUTER_MAX_K multiply-adds a value beside the group's own loads and stores. RG_HIP_PAIR=0, which
+// keeps every product in a launch without others, turns this off too.
+void find_outer_groups(const Plan& plan, const std::vector<std::vector<int64_t>>& writes, Epilogues* ep) {
+  const char* env = getenv("RG_HIP_PAIR");
+  if (env && env[0] == '0') return;
+  const auto& steps = plan.steps;
+  for (size_t j = 0; j < steps.size(); j++) {
+    const Step& sj = steps[j];
+    if (sj.kind != RG_STEP_FUSED || sj.fused.row_len != 0 || sj.fused.dtype != RG_F32 || fused_grid(sj.fused) <= MERGE_MAX_GRID) continue;
+    const rgplan::Fused& f = sj.fused;
+    bool kinds_ok = true;
+    for (auto& in : f.inputs)
+      kinds_ok = kinds_ok && (in.kind == RG_ARG_FULL || in.kind == RG_ARG_SPLAT || (in.kind == RG_ARG_ROW && in.row_len % 4 == 0));
+    if (!kinds_ok) continue;
+    uint64_t gm = 0, gn = 0, total_k = 0;
+    for (auto& in : f.inputs) {
+      if (in.kind != RG_ARG_FULL) continue;
+      size_t k = j;
+      while (k > 0 && !has_slot(writes[k - 1], in.slot)) k--;
+      if (k == 0) continue;
+      k--;
+      const Instr& p = steps[k].instr;
+      uint64_t m, n, kk;
+      bool ta, tb;
+      if (ep->outer_in[k] >= 0 || steps[k].kind != RG_STEP_INSTR || p.dtype != RG_F32 || p.dst != in.slot || p.args.size() != 2) continue;
+      if (!flat_product(p, &m, &n, &kk, &ta, &tb) || m * n != (uint64_t)f.n || n % 4 != 0 || !rgk::gemm_outer_product(m, n, kk, ta, tb)) continue;
+      if ((gm && (m != gm || n != gn)) || total_k + kk > OUTER_MAX_K || product_output_needed(plan, k, j)) continue;
+      bool ok = true;
+      for (auto& a : p.args) {
+        for (auto& o : f.outputs) ok = ok && o.second != a.slot;
+        for (size_t q = k + 1; q < j; q++) ok = ok && !has_slot(writes[q], a.slot);
+      }
+      // The group reads the slot once, as a Full input: the product's values have no other form here.
+      for (auto& other : f.inputs) ok = ok && (&other == &in || other.slot != in.slot);
+      for (size_t q = k + 1; q < j; q++) ok = ok && !(steps[q].kind == RG_STEP_INSTR && is_control(steps[q].instr.op));
+      if (!ok) continue;
+      gm = m;
+      gn = n;
+      total_k += kk;
+      ep->outer_of[j].push_back(k);
+      ep->outer_in[k] = (int64_t)j;
+    }
+  }
+}
 
 // Whether step s is an f32 sum over every axis but the last of the value in `slot`, shaped
 // [..., n] with `total` elements, into [1, ..., 1, n].
@@ -877,19 +934,23 @@ Epilogues find_epilogues(const Plan& plan) {
   const auto& steps = plan.steps;
   const size_t n = steps.size();
   Epilogues ep{std::vector<int64_t>(n, -1), std::vector<bool>(n, false), std::vector<int64_t>(n, -1), std::vector<int64_t>(n, -1),
-               std::vector<int>(n, -1)};
-  const char* env = getenv("RG_HIP_EPILOGUE");
-  if (env && env[0] == '0') return ep;
-  const bool every = env && std::string(env) == "all";
+               std::vector<int>(n, -1), std::vector<std::vector<size_t>>(n), std::vector<int64_t>(n, -1)};
   std::vector<std::vector<int64_t>> reads(n), writes(n);
   for (size_t q = 0; q < n; q++) {
     reads[q] = step_reads(steps[q]);
     writes[q] = step_writes(steps[q]);
   }
+  find_outer_groups(plan, writes, &ep);
+  for (size_t k = 0; k < n; k++)  // what moves with them is read at the group's step
+    if (ep.outer_in[k] >= 0)
+      for (auto& a : steps[k].instr.args) reads[(size_t)ep.outer_in[k]].push_back(a.slot);
+  const char* env = getenv("RG_HIP_EPILOGUE");
+  if (env && env[0] == '0') return ep;
+  const bool every = env && std::string(env) == "all";
   std::vector<bool> taken(n, false);
   for (size_t j = 0; j < n; j++) {
     const Step& sj = steps[j];
-    if (sj.kind != RG_STEP_FUSED || sj.fused.row_len != 0 || sj.fused.dtype != RG_F32) continue;
+    if (sj.kind != RG_STEP_FUSED || sj.fused.row_len != 0 || sj.fused.dtype != RG_F32 || !ep.outer_of[j].empty()) continue;
     const rgplan::Fused& f = sj.fused;
     if (fused_grid(f) <= MERGE_MAX_GRID) continue;
     bool kinds_ok = true;
@@ -977,6 +1038,18 @@ std::string epilogue_source(const Plan& plan, size_t j, int64_t pk, const std::s
     throw std::runtime_error("product epilogue: the product does not fit a single tile kernel");
   return rgjit::generate_gemm(plan.steps[j].fused, c, keep, rgjit::ProductTile{t.bm, t.bn, t.wm, t.wn, t.steps, t.tail, ta, tb},
                               prefix + "rge" + std::to_string(pk), fk, col_sum);
+}
+
+// Source of group j's kernel `name` with its outer products computed inside (find_outer_groups).
+std::string outer_source(const Plan& plan, size_t j, const std::vector<size_t>& ks, const std::string& name, rgjit::FusedKernel* fk) {
+  std::vector<rgjit::OuterProduct> products;
+  uint64_t m = 0, n = 0, kk;
+  for (size_t k : ks) {
+    bool ta, tb;
+    flat_product(plan.steps[k].instr, &m, &n, &kk, &ta, &tb);
+    products.push_back({plan.steps[k].instr.dst, (int)kk, ta, tb});
+  }
+  return rgjit::generate_outer(plan.steps[j].fused, (int64_t)m, (int64_t)n, products, name, fk);
 }
 
 // Independent products launched as one kernel (rgk::gemm_group): two adjacent plain products
@@ -1115,6 +1188,9 @@ void build_program(Program& prog) {
         bool keep = false;
         src << epilogue_source(prog.plan, k, pk, "", &keep, fk.get(), ep.sum_out[k]);
         store_c[(size_t)pk] = keep;
+      } else if (!ep.outer_of[k].empty()) {
+        src << outer_source(prog.plan, k, ep.outer_of[k], "rgf" + std::to_string(k), fk.get());
+        for (size_t p : ep.outer_of[k]) prog.absorbed_into[p] = (int64_t)k;
       } else if (st.kind == RG_STEP_ROWS) {
         src << rgjit::generate_rows(st.fused, "rgr" + std::to_string(k), fk.get());
       } else {
@@ -1191,16 +1267,20 @@ void build_program(Program& prog) {
       else prog.steps.push_back(combined(k, j));
       continue;
     }
-    if (st.kind == RG_STEP_INSTR && (ep.sum_in[k] >= 0 || attn_sum_in[k] >= 0)) {
+    if (st.kind == RG_STEP_INSTR && (ep.sum_in[k] >= 0 || attn_sum_in[k] >= 0 || ep.outer_in[k] >= 0)) {
       // A column sum computed by the combined kernel of the group it reads, or by the attention
-      // backward whose gradients it reads.
+      // backward whose gradients it reads; or an outer product its group computes.
       prog.steps.push_back([](hipStream_t, void* const*, void*) {});
       continue;
     }
     if (st.kind == RG_STEP_FUSED || st.kind == RG_STEP_ROWS) {
       rgjit::FusedKernel* fk = prog.fused[fi++].get();
       std::vector<int64_t> ins, outs;
-      for (auto& in : st.fused.inputs) ins.push_back(in.slot);
+      for (auto& in : st.fused.inputs) {
+        bool computed = false;
+        for (size_t p : ep.outer_of[k]) computed |= prog.plan.steps[p].instr.dst == in.slot;
+        if (!computed) ins.push_back(in.slot);
+      }
       for (auto& o : st.fused.outputs) outs.push_back(o.second);
       if (fk->grid == 0) {
         prog.steps.push_back([](hipStream_t, void* const*, void*) {});
@@ -1216,15 +1296,20 @@ void build_program(Program& prog) {
           fold_producer.push_back(k);
           prog.fold_bytes += ((uint64_t)fk->grid * fk->row_len * esize(dtype) + 255) / 256 * 256;
         }
-      if (ins.size() + outs.size() > 160) throw std::runtime_error("fused group with more than 160 operands");
+      // Then the operands of the outer products the group computes.
+      std::vector<int64_t> operands;
+      for (size_t p : ep.outer_of[k])
+        for (auto& a : prog.plan.steps[p].instr.args) operands.push_back(a.slot);
+      if (ins.size() + outs.size() + operands.size() > 160) throw std::runtime_error("fused group with more than 160 operands");
       const Program* pp = &prog;
-      prog.steps.push_back([fk, ins, outs, col_off, pp](hipStream_t s, void* const* sl, void* ws) {
+      prog.steps.push_back([fk, ins, outs, operands, col_off, pp](hipStream_t s, void* const* sl, void* ws) {
         void* ptrs[160];
         void* args[160];
         size_t q = 0;
         for (auto x : ins) ptrs[q++] = sl[x];
         for (size_t j = 0; j < outs.size(); j++)
           ptrs[q++] = col_off[j] == UINT64_MAX ? sl[outs[j]] : (char*)ws + pp->fold_base() + col_off[j];
+        for (auto x : operands) ptrs[q++] = sl[x];
         for (size_t j = 0; j < q; j++) args[j] = &ptrs[j];
         hipModuleLaunchKernel(fk->fn, fk->grid, 1, 1, fk->block, 1, 1, 0, s, args, nullptr);
       });
@@ -1279,7 +1364,12 @@ void build_program(Program& prog) {
     }
     const bool combined_here = (ep.at[j] >= 0 && ep.sunk[j]) || (epilogue_at[j] >= 0 && !ep.sunk[(size_t)epilogue_at[j]]);
     const bool moved_away = (ep.at[j] >= 0 && !ep.sunk[j]) || (epilogue_at[j] >= 0 && ep.sunk[(size_t)epilogue_at[j]]);
-    if (!moved_away && !combined_here) return step_reads(prog.plan.steps[j]);
+    if (!moved_away && !combined_here) {
+      r = step_reads(prog.plan.steps[j]);
+      for (size_t p : ep.outer_of[j])
+        for (auto& a : prog.plan.steps[p].instr.args) r.push_back(a.slot);
+      return r;
+    }
     if (combined_here) {
       const size_t g = ep.at[j] >= 0 ? j : (size_t)epilogue_at[j];
       const size_t pk = (size_t)ep.at[g];
@@ -1602,6 +1692,7 @@ std::string plan_source(const Plan& root, int* count) {
       rgjit::FusedKernel fk;
       bool keep;
       if (epi[k] >= 0) src << epilogue_source(plan, k, epi[k], prefix, &keep, &fk, eps.sum_out[k]);
+      else if (!eps.outer_of[k].empty()) src << outer_source(plan, k, eps.outer_of[k], prefix + "rgf" + std::to_string(k), &fk);
       else if (st.kind == RG_STEP_ROWS) src << rgjit::generate_rows(st.fused, prefix + "rgr" + std::to_string(k), &fk);
       else src << rgjit::generate(st.fused, prefix + "rgf" + std::to_string(k), &fk);
       (*count)++;
