@@ -991,6 +991,10 @@ Epilogues find_epilogues(const Plan& plan) {
       ep.at[j] = k;
       ep.sunk[j] = !hoist;
       taken[(size_t)k] = true;
+      // What moves counts where it runs, for the groups that follow.
+      const size_t from = hoist ? j : (size_t)k, to = hoist ? (size_t)k : j;
+      for (auto x : step_reads(steps[from])) reads[to].push_back(x);
+      for (auto x : step_writes(steps[from])) writes[to].push_back(x);
       // A column sum of one of the group's outputs a few steps later, with nothing between the
       // group and it overwriting that output: computed by the combined kernel from the values
       // it stores, summed in registers (a K-contiguous B, whole tiles: every output goes through
@@ -1063,9 +1067,25 @@ std::string outer_source(const Plan& plan, size_t j, const std::vector<size_t>& 
 // Step k launches them all, the others nothing; at run time a group whose operands turn out not
 // to fit (alignment) is launched as single kernels, at step k. The results are the single
 // launches'. RG_HIP_PAIR=0 turns this off.
-void group_products(Program& prog, const std::vector<GemmFill>& fills, const std::vector<rgk::GemmArgs>& base,
+void group_products(Program& prog, const Epilogues& ep, const std::vector<GemmFill>& fills, const std::vector<rgk::GemmArgs>& base,
                     std::vector<size_t>& fold_producer) {
   const size_t n = prog.plan.steps.size();
+  // What step q reads and writes when it runs: its own slots, those of an epilogue's group computed
+  // at the product's step, and those of products computed at a group's step.
+  std::vector<std::vector<int64_t>> reads(n), writes(n);
+  for (size_t q = 0; q < n; q++) {
+    reads[q] = step_reads(prog.plan.steps[q]);
+    writes[q] = step_writes(prog.plan.steps[q]);
+  }
+  auto runs_at = [&](size_t moved, size_t q) {
+    for (auto x : step_reads(prog.plan.steps[moved])) reads[q].push_back(x);
+    for (auto x : step_writes(prog.plan.steps[moved])) writes[q].push_back(x);
+  };
+  for (size_t q = 0; q < n; q++) {
+    if (ep.at[q] >= 0 && ep.sunk[q]) runs_at((size_t)ep.at[q], q);
+    else if (ep.at[q] >= 0) runs_at(q, (size_t)ep.at[q]);
+    if (ep.outer_in[q] >= 0) runs_at(q, (size_t)ep.outer_in[q]);
+  }
   prog.pair_of.assign(n, -1);
   const char* env = getenv("RG_HIP_PAIR");
   if (env && env[0] == '0') return;
@@ -1093,10 +1113,9 @@ void group_products(Program& prog, const std::vector<GemmFill>& fills, const std
     for (size_t q = j + 1; q < k; q++) {
       const Step& sq = prog.plan.steps[q];
       if (sq.kind == RG_STEP_INSTR && is_control(sq.instr.op)) return false;
-      const auto w = step_writes(sq), r = step_reads(sq);
       for (auto& arg : pj.args)
-        if (has_slot(w, arg.slot)) return false;
-      if (has_slot(w, pj.dst) || has_slot(r, pj.dst)) return false;
+        if (has_slot(writes[q], arg.slot)) return false;
+      if (has_slot(writes[q], pj.dst) || has_slot(reads[q], pj.dst)) return false;
     }
     return true;
   };
@@ -1339,7 +1358,7 @@ void build_program(Program& prog) {
       while (fold_producer.size() < prog.folds.size()) fold_producer.push_back(k);
     }
   }
-  group_products(prog, gemm_fills, gemm_base, fold_producer);
+  group_products(prog, ep, gemm_fills, gemm_base, fold_producer);
   for (auto& s : prog.plan.slots) prog.slot_bytes.push_back(std::max<uint64_t>((uint64_t)s.cap * esize(s.dtype), 4));
   place_bodies(prog);
   // Each fold runs before the first later step reading its output, or right after its producer.
