@@ -228,8 +228,12 @@ std::vector<bool> tails(const Graph& g, const std::vector<bool>& keep, const std
   return tail;
 }
 
-// Longest rows a row-group kernel keeps in one wavefront's registers.
-constexpr size_t ROW_MAX = 1024;
+// Longest rows a row-group kernel keeps in registers: a wavefront's to COL_MAX, above that those of
+// a block of a wave per 1024 elements (16 a lane either way). Column reductions, whose waves each
+// keep a whole row's accumulators, join groups of a wavefront's rows only. The softmax and cross
+// entropy of 4096 rows of 5000 take LONGROWS.
+constexpr size_t ROW_MAX = 8192;
+constexpr size_t COL_MAX = 1024;
 
 // A last-axis reduction with kept dimensions, the seed of a row group: [rows..., L] -> [rows..., 1].
 bool row_reduce(const Graph& g, size_t i) {
@@ -352,7 +356,7 @@ std::vector<std::vector<size_t>> row_groups(const Graph& g, const std::vector<bo
     const Node& n = g.nodes[i];
     if (n.op.kind != RG_OP_REDUCE || n.dtype == DType::I32) return false;
     const Shape& s = g.shape(n.inputs[0]);
-    if (s.size() < 2 || s.back() > (int64_t)ROW_MAX || n.op.v.size() + 1 != s.size()) return false;
+    if (s.size() < 2 || s.back() > (int64_t)COL_MAX || n.op.v.size() + 1 != s.size()) return false;
     Shape ax = n.op.v;
     std::sort(ax.begin(), ax.end());
     for (size_t q = 0; q < ax.size(); q++)

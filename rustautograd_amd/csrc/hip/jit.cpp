@@ -481,19 +481,23 @@ std::string generate_rows(const rgplan::Fused& f, const std::string& name, Fused
   const char* T = dbl ? "double" : "float";
   const int64_t L = f.row_len, rows = f.n / f.row_len;
   const int maxv = dbl ? 2 : 4;
+  // Rows of at most ROW_WAVE elements take a wave each; longer ones a block, a wave per ROW_WAVE
+  // elements, so that a lane never holds more than 16 elements of a value.
+  const int64_t RW = (L + ROW_WAVE - 1) / ROW_WAVE, LN = 64 * RW;
   int V = 1;
   for (int v = maxv; v > 1; v /= 2)
-    if (L % (64 * v) == 0) {
+    if (L % (RW > 1 ? v : 64 * v) == 0) {
       V = v;
       break;
     }
-  const int64_t E = (L + 64 * V - 1) / (64 * V) * V;
-  const bool exact = L % (64 * V) == 0;
+  const int64_t E = (L + LN * V - 1) / (LN * V) * V;
+  const bool exact = L % (LN * V) == 0;
   const char* VT = dbl ? (V == 2 ? "double2" : "double") : (V == 4 ? "float4" : V == 2 ? "float2" : "float");
   const char* lanes[4] = {"x", "y", "z", "w"};
   k->name = name;
   k->vec = 1;
-  k->grid = (uint32_t)((rows + 3) / 4);
+  k->grid = (uint32_t)(RW > 1 ? rows : (rows + 3) / 4);
+  if (RW > 1) k->block = (uint32_t)LN;
   // Column reductions (RG_ROWS_COLUMN): the waves walk rows grid-stride, accumulating them.
   std::vector<bool> col_reg((size_t)f.regs, false);
   bool has_col = false;
@@ -501,6 +505,7 @@ std::string generate_rows(const rgplan::Fused& f, const std::string& name, Fused
     if (m.op == RG_OP_REDUCE && (m.aux & RG_ROWS_COLUMN)) col_reg[(size_t)m.reg] = has_col = true;
   k->col_kind.assign(f.outputs.size(), -1);
   k->row_len = (uint32_t)L;
+  if (has_col && RW > 1) throw std::runtime_error("row group with column reductions over rows longer than a wave's");
   if (has_col) {
     k->grid = (uint32_t)std::min<int64_t>((rows + COL_WAVES - 1) / COL_WAVES, COL_BLOCKS);
     k->block = 64 * COL_WAVES;
@@ -529,12 +534,12 @@ std::string generate_rows(const rgplan::Fused& f, const std::string& name, Fused
   for (auto& o : f.outputs)
     for (auto& in : f.inputs) alias |= in.slot == o.second;
   const char* R = alias ? "" : "__restrict__ ";
-  const int waves = has_col ? COL_WAVES : TPB / 64;
+  const int waves = has_col ? COL_WAVES : RW > 1 ? (int)RW : TPB / 64;
   s << "extern \"C\" __global__ void __launch_bounds__(" << 64 * waves << ") " << name << "(";
   for (size_t j = 0; j < f.inputs.size(); j++) s << (j ? ", " : "") << "const " << T << "* " << R << "in" << j;
   for (size_t j = 0; j < f.outputs.size(); j++) s << ", " << T << "* " << R << "out" << j;
   s << ") {\n";
-  s << "  const unsigned lane = threadIdx.x & 63u;\n";
+  s << "  const unsigned lane = threadIdx.x" << (RW > 1 ? "" : " & 63u") << ";\n";
   auto col_init = [&](int64_t aux) {
     const int64_t kind = aux & ~(int64_t)RG_ROWS_COLUMN;
     return kind == RG_REDUCE_SUM ? std::string("0") : kind == RG_REDUCE_MAX ? std::string("-__builtin_huge_val()") : std::string("__builtin_huge_val()");
@@ -550,13 +555,15 @@ std::string generate_rows(const rgplan::Fused& f, const std::string& name, Fused
           << col_init(m.aux) << ";\n";
     s << "  for (unsigned long long row = (unsigned long long)blockIdx.x * " << waves << "ull + (threadIdx.x >> 6); row < " << rows
       << "ull; row += (unsigned long long)gridDim.x * " << waves << "ull) {\n";
+  } else if (RW > 1) {
+    s << "  const unsigned long long row = blockIdx.x;\n";
   } else {
     s << "  const unsigned long long row = (unsigned long long)blockIdx.x * 4ull + (threadIdx.x >> 6);\n";
     s << "  if (row >= " << rows << "ull) return;\n";
   }
   // Element e of this lane sits at column J(e) of the row.
   auto col = [&](int64_t e) {
-    return std::to_string((e / V) * 64 * V + e % V) + "u + lane * " + std::to_string(V) + "u";
+    return std::to_string((e / V) * LN * V + e % V) + "u + lane * " + std::to_string(V) + "u";
   };
   auto valid = [&](int64_t e) { return exact ? std::string("true") : "(" + col(e) + " < " + std::to_string(L) + "u)"; };
   // Offset of a broadcast input's row: coordinates of `row` over the leading dimensions.
@@ -586,6 +593,14 @@ std::string generate_rows(const rgplan::Fused& f, const std::string& name, Fused
     s << "  " << T << " " << x << "[" << E << "];\n";
     if (V > 1) {
       for (int64_t c = 0; c < E / V; c++) {
+        if (!exact) {  // whole vectors: the row's length is a multiple of V
+          s << "  if (" << valid(c * V) << ") { const " << VT << " t = *(const " << VT << "*)(" << base << " + " << col(c * V) << ");";
+          for (int v = 0; v < V; v++) s << " " << x << "[" << c * V + v << "] = t." << lanes[v] << ";";
+          s << " } else {";
+          for (int v = 0; v < V; v++) s << " " << x << "[" << c * V + v << "] = (" << T << ")0;";
+          s << " }\n";
+          continue;
+        }
         s << "  { const " << VT << " t = *(const " << VT << "*)(" << base << " + " << col(c * V) << ");";
         for (int v = 0; v < V; v++) s << " " << x << "[" << c * V + v << "] = t." << lanes[v] << ";";
         s << " }\n";
@@ -662,6 +677,13 @@ std::string generate_rows(const rgplan::Fused& f, const std::string& name, Fused
       // The 64 lanes' partial values combined without LDS (rg_wave_sum and its kin, ops.h).
       s << "  " << rn << " = " << (m.aux == RG_REDUCE_SUM ? "rg_wave_sum(" : m.aux == RG_REDUCE_MAX ? "rg_wave_max(" : "rg_wave_min(") << rn
         << ");\n";
+      if (RW > 1) {
+        // The waves' values in wave order, through LDS of the reduction's own: every wave gets them.
+        s << "  __shared__ " << T << " w" << m.reg << "[" << RW << "];\n";
+        s << "  if ((lane & 63u) == 0) w" << m.reg << "[lane >> 6] = " << rn << ";\n  __syncthreads();\n";
+        s << "  " << rn << " = w" << m.reg << "[0];\n";
+        for (int64_t q = 1; q < RW; q++) s << "  " << rn << " = " << comb(rn, "w" + std::to_string(m.reg) + "[" + std::to_string(q) + "]") << ";\n";
+      }
       continue;
     }
     if (level[(size_t)m.reg]) {
@@ -701,7 +723,7 @@ std::string generate_rows(const rgplan::Fused& f, const std::string& name, Fused
     std::string base = "(" + o + " + row * " + std::to_string(L) + "ull)";
     if (V > 1) {
       for (int64_t c = 0; c < E / V; c++) {
-        s << "  { " << VT << " t;";
+        s << "  " << (exact ? "" : "if (" + valid(c * V) + ") ") << "{ " << VT << " t;";
         for (int v = 0; v < V; v++) s << " t." << lanes[v] << " = " << rn << "[" << c * V + v << "];";
         s << " *(" << VT << "*)(" << base << " + " << col(c * V) << ") = t; }\n";
       }

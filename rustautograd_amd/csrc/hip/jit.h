@@ -26,6 +26,11 @@ struct FusedKernel {
   uint32_t block = TPB;  // threads per block
 };
 
+// Elements of a row that one wave of a row group's kernel holds; a longer row takes a block, which
+// is bound by its loads and stores: 4096 rows of 5000 (five waves), two values read, one written
+// and two reductions between, 38.5 us, 6.4 TB/s.
+constexpr int64_t ROW_WAVE = 1024;
+
 // A row group with column reductions: COL_BLOCKS blocks of COL_WAVES waves (one block per CU,
 // four waves per SIMD), each folding the rows it walks into one partial row. (Two blocks per CU
 // at 64 registers, one row per wave, measured no faster on C4's layer norms.)
@@ -48,9 +53,10 @@ std::string generate(const rgplan::Fused& f, const std::string& name, FusedKerne
 std::string generate_merged(const std::vector<const rgplan::Fused*>& parts, const std::string& name, FusedKernel* k);
 std::vector<int64_t> merged_slots(const std::vector<const rgplan::Fused*>& parts);
 
-// Source of one row-group kernel (RG_STEP_ROWS): `k->grid` blocks of four rows each, or, with
-// column reductions, COL_BLOCKS blocks of COL_WAVES waves walking the rows grid-stride and writing
-// one partial row per block for each column output (see col_kind).
+// Source of one row-group kernel (RG_STEP_ROWS): `k->grid` blocks of four rows each (of one
+// row longer than ROW_WAVE each), or, with column reductions, COL_BLOCKS blocks of COL_WAVES waves
+// walking the rows grid-stride and writing one partial row per block for each column output (see
+// col_kind).
 std::string generate_rows(const rgplan::Fused& f, const std::string& name, FusedKernel* k);
 
 // A product's tile for generate_gemm (the template arguments of rgg::gemm_mfma_block).
