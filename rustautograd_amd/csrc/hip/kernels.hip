@@ -297,17 +297,29 @@ __global__ void __launch_bounds__(TPB) k_take_grad(const T* __restrict__ ct, con
   if (q < block) dst[((uint64_t)o * dim + d) * block + q] = acc;
 }
 
-template <class T>
+// W elements of a row per thread, stored at once: the output (a row of zeros but for the taken
+// elements) is all the traffic there is, and 4-byte stores do not fill it: 4096 rows of 5000
+// take 19.5 us, 29.8 with an element a thread.
+// W is 16 bytes of a row whose length W divides, else 1.
+template <class T, int W>
+struct alignas(W * sizeof(T)) Run {
+  T v[W];
+};
+
+template <class T, int W>
 __global__ void __launch_bounds__(TPB) k_take_along_grad(const T* __restrict__ ct, const int* __restrict__ idx, T* __restrict__ dst,
                                                          uint32_t n, FastDiv v, uint32_t k) {
-  uint32_t t = blockIdx.x * TPB + threadIdx.x;
-  if (t >= n) return;
-  uint32_t r = v.div(t);
-  uint32_t c = t - r * v.d;
-  T acc = (T)0;
-  for (uint32_t x = 0; x < k; x++)
-    if (clamp_index(idx[r * k + x], v.d) == c) acc = acc + ct[r * k + x];
-  dst[t] = acc;
+  const uint32_t t = blockIdx.x * TPB + threadIdx.x;
+  if (t >= n / W) return;
+  const uint32_t r = v.div(t * W), c = t * W - r * v.d;
+  Run<T, W> acc{};
+  for (uint32_t x = 0; x < k; x++) {
+    const uint32_t at = clamp_index(idx[r * k + x], v.d);
+#pragma unroll
+    for (int e = 0; e < W; e++)
+      if (at == c + e) acc.v[e] = acc.v[e] + ct[r * k + x];
+  }
+  *(Run<T, W>*)(dst + (uint64_t)t * W) = acc;
 }
 
 // ---- random streams (SplitMix64 of key and index, src/plan.rs:1391-1435) ----------------
@@ -820,8 +832,12 @@ void take_grad(hipStream_t s, int dtype, const void* ct, const int32_t* idx, voi
 
 void take_along_grad(hipStream_t s, int dtype, const void* ct, const int32_t* idx, void* dst, uint64_t n, uint64_t k, uint64_t v) {
   FastDiv fv((uint32_t)v);
-  if (dtype == RG_F32) RG_LAUNCH(k_take_along_grad<float>, n, (const float*)ct, idx, (float*)dst, (uint32_t)n, fv, (uint32_t)k);
-  else RG_LAUNCH(k_take_along_grad<double>, n, (const double*)ct, idx, (double*)dst, (uint32_t)n, fv, (uint32_t)k);
+#define RG_TAKE(T, W) RG_LAUNCH((k_take_along_grad<T, W>), n / W, (const T*)ct, idx, (T*)dst, (uint32_t)n, fv, (uint32_t)k)
+  if (dtype == RG_F32 && v % 4 == 0) RG_TAKE(float, 4);
+  else if (dtype == RG_F32) RG_TAKE(float, 1);
+  else if (v % 2 == 0) RG_TAKE(double, 2);
+  else RG_TAKE(double, 1);
+#undef RG_TAKE
 }
 
 void rand_uniform(hipStream_t s, int dtype, const int32_t* key, void* dst, uint64_t n) {

@@ -460,3 +460,13 @@ def test_streamed_products_launched_together_match_single_launches(monkeypatch):
         want = (a.T if ta else a).astype(np.float64) @ (b.T if tb else b).astype(np.float64)
         assert np.array_equal(out0[q].view(np.uint32), out1[q].view(np.uint32)), (m, k, n, ta, tb)
         assert np.abs(out1[q] - want).max() <= 1e-4 * np.abs(want).max(), (m, k, n, ta, tb)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+@pytest.mark.parametrize("rows,k,v", [(3, 1, 1), (7, 2, 4), (5, 3, 5), (130, 1, 6), (77, 1, 1023), (33, 5, 1024), (4, 1, 5000)])
+def test_taken_elements_gradients_of_every_width(rows, k, v, dtype):
+    """Rows written 16 bytes at a time when their length allows it; repeated and clamped indices add in order."""
+    gen = np.random.default_rng(v)
+    idx = t(gen.integers(-1, v + 2, size=(rows, k)).tolist(), "int32")
+    ct = t(gen.normal(size=(rows, k)).tolist(), dtype)
+    agree(lambda g, i: op(g, "take_along_grad", [i[0], i[1]], shape=[rows, v]), [ct, idx], what=f"{rows} x {v}, {k} taken", ulps=0)
