@@ -774,7 +774,7 @@ bool flat_product(const Instr& i, uint64_t* m, uint64_t* n, uint64_t* k, bool* t
 
 // Elementwise groups computed in the epilogue of the product they read (at[j] = k: plain fused
 // group j reads product k's output and runs inside product k's kernel). Taken when product k is
-// one unsplit fp32 MFMA tile product (gemm_epilogue_tile), group j walks its M x N outputs with
+// one unsplit product on a split tile (gemm_epilogue_tile), group j walks its M x N outputs with
 // Full, Row (length a multiple of 4) and Splat inputs and writes none of the product's operands
 // (other blocks of the product still read them while the epilogue stores), and the combined
 // kernel can run at one of the two steps without changing any value, with no control flow
