@@ -818,6 +818,28 @@ struct Epilogues {
   // whose kernel computes this product, or -1.
   std::vector<std::vector<size_t>> outer_of;
   std::vector<int64_t> outer_in;
+  // The column sums the attention backward computes (attention_column_sum): per attention step,
+  // the sum step; per sum step, the attention step; or -1.
+  std::vector<int64_t> attn_sum_of, attn_sum_in;
+  // What each step reads and writes: its own slots, and those of what was moved to it.
+  std::vector<std::vector<int64_t>> reads, writes;
+
+  // Whether the column sum at step q of what step j writes to slot `summed` can be written by the
+  // kernel that computes j at step c <= j < q: no step between c and q reads or writes the sum's
+  // slot (its fold is due from c on), and none between j and q overwrites what is summed.
+  bool sum_moves(const Plan& plan, size_t c, size_t j, size_t q, int64_t summed) const {
+    const int64_t dst = plan.steps[q].instr.dst;
+    for (size_t r = c + 1; r < q; r++) {
+      if (r != j && (has_slot(writes[r], dst) || has_slot(reads[r], dst))) return false;
+      if (r > j && has_slot(writes[r], summed)) return false;
+    }
+    return true;
+  }
+  // Step `from` runs at step `to`.
+  void moves(const Plan& plan, size_t from, size_t to) {
+    for (auto x : step_reads(plan.steps[from])) reads[to].push_back(x);
+    for (auto x : step_writes(plan.steps[from])) writes[to].push_back(x);
+  }
 };
 
 constexpr uint64_t OUTER_MAX_K = 32;  // of one group's outer products together: 4 registers a lane each
@@ -829,7 +851,8 @@ constexpr uint64_t OUTER_MAX_K = 32;  // of one group's outer products together:
 // at step j. The product is then neither stored nor loaded: the group's kernel does at most
 // OUTER_MAX_K multiply-adds a value beside the group's own loads and stores. RG_HIP_PAIR=0, which
 // keeps every product in a launch without others, turns this off too.
-void find_outer_groups(const Plan& plan, const std::vector<std::vector<int64_t>>& writes, Epilogues* ep) {
+void find_outer_groups(const Plan& plan, Epilogues* ep) {
+  const auto& writes = ep->writes;
   const char* env = getenv("RG_HIP_PAIR");
   if (env && env[0] == '0') return;
   const auto& steps = plan.steps;
@@ -892,7 +915,7 @@ bool column_sum_of(const Step& st, int64_t slot, uint64_t total, uint64_t n) {
 // backward can write those sums itself: dq, dk and dv rows of one slot, L columns a row, the
 // views' heads covering every column once, and shapes for which the backward writes column sums
 // (rgk::attention_backward_column_sums). -1 otherwise, or with RG_HIP_EPILOGUE_SUMS=0.
-int64_t attention_column_sum(const Plan& plan, size_t j) {
+int64_t attention_column_sum(const Plan& plan, const Epilogues& ep, size_t j) {
   const Step& sj = plan.steps[j];
   if (sj.kind != RG_STEP_ATTN || !sj.attn.backward || sj.attn.out.size() != 3 || sj.attn.dtype != RG_F32) return -1;
   const char* sums = getenv("RG_HIP_EPILOGUE_SUMS");
@@ -920,32 +943,19 @@ int64_t attention_column_sum(const Plan& plan, size_t j) {
   for (size_t q = j + 1; q < plan.steps.size() && q <= j + 4; q++) {
     const Step& sq = plan.steps[q];
     if (sq.kind == RG_STEP_INSTR && is_control(sq.instr.op)) return -1;
-    if (column_sum_of(sq, slot, (uint64_t)(B * at.tq * L), (uint64_t)L)) {
-      for (size_t r = j + 1; r < q; r++)
-        if (has_slot(step_writes(plan.steps[r]), slot)) return -1;
-      return (int64_t)q;
-    }
+    if (column_sum_of(sq, slot, (uint64_t)(B * at.tq * L), (uint64_t)L))
+      return ep.sum_in[q] < 0 && ep.sum_moves(plan, j, j, q, slot) ? (int64_t)q : -1;
   }
   return -1;
 }
 
-
-Epilogues find_epilogues(const Plan& plan) {
+void find_product_epilogues(const Plan& plan, Epilogues* found) {
+  Epilogues& ep = *found;
   const auto& steps = plan.steps;
   const size_t n = steps.size();
-  Epilogues ep{std::vector<int64_t>(n, -1), std::vector<bool>(n, false), std::vector<int64_t>(n, -1), std::vector<int64_t>(n, -1),
-               std::vector<int>(n, -1), std::vector<std::vector<size_t>>(n), std::vector<int64_t>(n, -1)};
-  std::vector<std::vector<int64_t>> reads(n), writes(n);
-  for (size_t q = 0; q < n; q++) {
-    reads[q] = step_reads(steps[q]);
-    writes[q] = step_writes(steps[q]);
-  }
-  find_outer_groups(plan, writes, &ep);
-  for (size_t k = 0; k < n; k++)  // what moves with them is read at the group's step
-    if (ep.outer_in[k] >= 0)
-      for (auto& a : steps[k].instr.args) reads[(size_t)ep.outer_in[k]].push_back(a.slot);
+  auto &reads = ep.reads, &writes = ep.writes;
   const char* env = getenv("RG_HIP_EPILOGUE");
-  if (env && env[0] == '0') return ep;
+  if (env && env[0] == '0') return;
   const bool every = env && std::string(env) == "all";
   std::vector<bool> taken(n, false);
   for (size_t j = 0; j < n; j++) {
@@ -993,12 +1003,11 @@ Epilogues find_epilogues(const Plan& plan) {
       taken[(size_t)k] = true;
       // What moves counts where it runs, for the groups that follow.
       const size_t from = hoist ? j : (size_t)k, to = hoist ? (size_t)k : j;
-      for (auto x : step_reads(steps[from])) reads[to].push_back(x);
-      for (auto x : step_writes(steps[from])) writes[to].push_back(x);
-      // A column sum of one of the group's outputs a few steps later, with nothing between the
-      // group and it overwriting that output: computed by the combined kernel from the values
-      // it stores, summed in registers (a K-contiguous B, whole tiles: every output goes through
-      // put4). RG_HIP_EPILOGUE_SUMS=0 leaves it to its own kernel.
+      ep.moves(plan, from, to);
+      // A column sum of one of the group's outputs a few steps later, with nothing between that
+      // overwrites the output or needs the sum's slot (sum_moves): computed by the combined kernel
+      // from the values it stores, summed in registers (a K-contiguous B, whole tiles: every output
+      // goes through put4). RG_HIP_EPILOGUE_SUMS=0 leaves it to its own kernel.
       const char* sums = getenv("RG_HIP_EPILOGUE_SUMS");
       if ((sums && sums[0] == '0') || !tb || !tile.whole) break;
       for (size_t q = j + 1; q < n && q <= j + 4; q++) {
@@ -1007,9 +1016,8 @@ Epilogues find_epilogues(const Plan& plan) {
         for (size_t o = 0; o < f.outputs.size(); o++)
           if (column_sum_of(steps[q], f.outputs[o].second, m * nn, nn)) out = (int)o;
         if (out >= 0) {
-          bool clear = true;
-          for (size_t r = j + 1; r < q; r++) clear = clear && !has_slot(writes[r], f.outputs[(size_t)out].second);
-          if (clear) {
+          if (ep.sum_moves(plan, to, j, q, f.outputs[(size_t)out].second)) {
+            ep.moves(plan, q, to);
             ep.sum_of[j] = (int64_t)q;
             ep.sum_in[q] = (int64_t)j;
             ep.sum_out[j] = out;
@@ -1019,6 +1027,28 @@ Epilogues find_epilogues(const Plan& plan) {
       }
       break;
     }
+  }
+}
+
+// What the plan's steps compute in other steps' kernels.
+Epilogues find_epilogues(const Plan& plan) {
+  const size_t n = plan.steps.size();
+  const std::vector<int64_t> none(n, -1);
+  Epilogues ep{none, std::vector<bool>(n, false), none, none, std::vector<int>(n, -1), std::vector<std::vector<size_t>>(n), none, none, none, {}, {}};
+  for (auto& st : plan.steps) {
+    ep.reads.push_back(step_reads(st));
+    ep.writes.push_back(step_writes(st));
+  }
+  find_outer_groups(plan, &ep);
+  for (size_t k = 0; k < n; k++)
+    if (ep.outer_in[k] >= 0) ep.moves(plan, k, (size_t)ep.outer_in[k]);
+  find_product_epilogues(plan, &ep);
+  for (size_t j = 0; j < n; j++) {
+    const int64_t q = attention_column_sum(plan, ep, j);
+    if (q < 0) continue;
+    ep.attn_sum_of[j] = q;
+    ep.attn_sum_in[(size_t)q] = (int64_t)j;
+    ep.moves(plan, (size_t)q, j);
   }
   return ep;
 }
@@ -1070,22 +1100,7 @@ std::string outer_source(const Plan& plan, size_t j, const std::vector<size_t>& 
 void group_products(Program& prog, const Epilogues& ep, const std::vector<GemmFill>& fills, const std::vector<rgk::GemmArgs>& base,
                     std::vector<size_t>& fold_producer) {
   const size_t n = prog.plan.steps.size();
-  // What step q reads and writes when it runs: its own slots, those of an epilogue's group computed
-  // at the product's step, and those of products computed at a group's step.
-  std::vector<std::vector<int64_t>> reads(n), writes(n);
-  for (size_t q = 0; q < n; q++) {
-    reads[q] = step_reads(prog.plan.steps[q]);
-    writes[q] = step_writes(prog.plan.steps[q]);
-  }
-  auto runs_at = [&](size_t moved, size_t q) {
-    for (auto x : step_reads(prog.plan.steps[moved])) reads[q].push_back(x);
-    for (auto x : step_writes(prog.plan.steps[moved])) writes[q].push_back(x);
-  };
-  for (size_t q = 0; q < n; q++) {
-    if (ep.at[q] >= 0 && ep.sunk[q]) runs_at((size_t)ep.at[q], q);
-    else if (ep.at[q] >= 0) runs_at(q, (size_t)ep.at[q]);
-    if (ep.outer_in[q] >= 0) runs_at(q, (size_t)ep.outer_in[q]);
-  }
+  const auto &reads = ep.reads, &writes = ep.writes;
   prog.pair_of.assign(n, -1);
   const char* env = getenv("RG_HIP_PAIR");
   if (env && env[0] == '0') return;
@@ -1181,16 +1196,7 @@ void build_program(Program& prog) {
   prog.epilogue_of = ep.at;
   prog.epilogue_sunk = ep.sunk;
   prog.absorbed_into.assign(n_steps, -1);
-  // Column sums the attention backward computes (attention_column_sum): per attention step, the
-  // sum step; per sum step, the attention step.
-  std::vector<int64_t> attn_sum_of(n_steps, -1), attn_sum_in(n_steps, -1);
-  for (size_t j = 0; j < n_steps; j++) {
-    const int64_t q = attention_column_sum(prog.plan, j);
-    if (q >= 0 && ep.sum_in[(size_t)q] < 0) {
-      attn_sum_of[j] = q;
-      attn_sum_in[(size_t)q] = (int64_t)j;
-    }
-  }
+  const std::vector<int64_t>&attn_sum_of = ep.attn_sum_of, &attn_sum_in = ep.attn_sum_in;
   std::vector<int64_t> epilogue_at(n_steps, -1);  // product step -> the group it computes
   for (size_t j = 0; j < n_steps; j++)
     if (ep.at[j] >= 0) epilogue_at[(size_t)ep.at[j]] = (int64_t)j;
