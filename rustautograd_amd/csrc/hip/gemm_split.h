@@ -14,11 +14,10 @@
 // steps form the sum of a (-b) and subtract it, which turns their bias the other way (without that
 // it made up a quarter of the error at K = 5000 and showed in sums over a gradient's rows). Against
 // 64-bit sums the relative error is 0.25-0.3 of the fp32 MFMA tile's for K = 256 to 8192 (normal
-// operands, 2048: 1.8e-7 against 7.9e-7). bf16 has fp32's exponent range; only operand values below
-// 2^-109 lose low bits of x3 (or x2) to its underflow.
-// A value that is not finite, or that rounds past the largest bf16 value, leaves NaN in every sum
-// it enters, so a wave that ends with a sum that is not finite forms its outputs again with fp32
-// MFMAs straight from memory: such outputs are the fp32 tile's.
+// operands, 2048: 1.8e-7 against 7.9e-7).
+// A value that is not finite, or that rounds past the largest bf16 value (scaled: see SPLIT_SCALE),
+// leaves NaN in every sum it enters, so a wave that ends with a sum that is not finite forms its
+// outputs again with fp32 MFMAs straight from memory: such outputs are the fp32 tile's.
 //
 // What bounds it: six bf16 terms at 2.5 PFLOP/s are 417 TFLOP/s of fp32 products against 157 on the
 // fp32 MFMA; a large bf16 product of the vendor library reaches 1.2 PFLOP/s on this chip, a sixth of
@@ -108,6 +107,14 @@ __device__ __forceinline__ void split_bf16(float x0, float x1, uint32_t& p1, uin
 
 constexpr int SPLIT_BK = 32;  // K step
 
+// Operands are split after multiplication by 2^23, and a step's sums, 2^46 too large, are multiplied
+// by 2^-46 as they are added: both are exact. So any fp32 value, 2^-149 at the least, has a first part
+// in bf16's normal range and loses none of the others (unscaled, values of 2^-120 kept 15 bits and
+// those below 2^-134 none; with 2^16 a part below 2^-126 is held, but the MFMA cuts off what it is
+// added to on the scale of 2^-126: 8.5e-7 for values of a few 2^-149). The price is at the other end:
+// outputs of values from 2^104 or step sums from 2^82 on are formed by the fp32 MFMAs.
+constexpr float SPLIT_SCALE = 8388608.0f, SPLIT_UNSCALE = 1.0f / (8388608.0f * 8388608.0f);
+
 // Layout of R rows (or columns) x 32 k of one operand in LDS: three planes of cells (16 bytes,
 // eight consecutive k), [k / 8][row], the k / 8 groups two cells further apart than R so that the
 // stores of a K-contiguous operand (four lanes per row) spread over all banks; the MFMA's reads are
@@ -182,9 +189,8 @@ struct SplitStage {
       }
     }
   }
-  // `sign` (1 or -1) times the staged values, split, into LDS.
-  template <bool SIGNED>
-  __device__ __forceinline__ void store(cell* lds, int tid, float sign) const {
+  // `factor` times the staged values, split, into LDS.
+  __device__ __forceinline__ void store(cell* lds, int tid, float factor) const {
 #pragma unroll
     for (int q = 0; q < G::PER; q++) {
       const int u = q * NT + tid;
@@ -196,8 +202,7 @@ struct SplitStage {
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           uint32_t x1, x2, x3;
-          const float x = v[q][j][2 * e], y = v[q][j][2 * e + 1];
-          split_bf16(SIGNED ? x * sign : x, SIGNED ? y * sign : y, x1, x2, x3);
+          split_bf16(v[q][j][2 * e] * factor, v[q][j][2 * e + 1] * factor, x1, x2, x3);
           p1[e] = x1, p2[e] = x2, p3[e] = x3;
         }
         cell* d = lds + g * G::GROUP + G::place(r + j);
@@ -268,10 +273,8 @@ __device__ __forceinline__ void gemm_split_tile(const float* __restrict__ A, con
   auto store = [&](float sign) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      sa[u].template store<false>(smem + u * STEP, tid, 1.0f);
-      if constexpr (U % 2 == 1) sb[u].template store<true>(smem + u * STEP + GA::CELLS, tid, u % 2 ? -sign : sign);
-      else if (u % 2) sb[u].template store<true>(smem + u * STEP + GA::CELLS, tid, -1.0f);
-      else sb[u].template store<false>(smem + u * STEP + GA::CELLS, tid, 1.0f);
+      sa[u].store(smem + u * STEP, tid, SPLIT_SCALE);
+      sb[u].store(smem + u * STEP + GA::CELLS, tid, u % 2 ? -sign * SPLIT_SCALE : sign * SPLIT_SCALE);
     }
   };
   floatx4 acc[TM][TN];
@@ -303,7 +306,7 @@ __device__ __forceinline__ void gemm_split_tile(const float* __restrict__ A, con
 #pragma unroll
       for (int n = 0; n < TN; n++)
 #pragma unroll
-        for (int r = 0; r < 4; r++) acc[i][n][r] = __builtin_fmaf(step[n][r], sign, acc[i][n][r]);
+        for (int r = 0; r < 4; r++) acc[i][n][r] = __builtin_fmaf(step[n][r], sign * SPLIT_UNSCALE, acc[i][n][r]);
     }
   };
   auto multiply = [&](float sign, int t, bool last) __attribute__((always_inline)) {

@@ -116,6 +116,23 @@ def test_small_values_keep_their_precision():
     assert np.linalg.norm(_product(a, b) - want) <= 3e-7 * np.linalg.norm(want)
 
 
+@pytest.mark.parametrize("exponent", [-108, -112, -120, -126, -133, -140, -146])
+@pytest.mark.parametrize("small", ["left", "right", "both"])
+def test_the_smallest_values_keep_their_precision(exponent, small):
+    """Down to the denormal values next to 0, on either side, every bit an operand has counts: the
+    bounds are those of ordinary operands. Both sides small: their products are denormal or near it,
+    and each K step's sum and each addition may round to a multiple of 2^-149."""
+    a, b = _operands(1024, 1024, 64, False, False)
+    low, high = (exponent // 2, exponent - exponent // 2) if small == "both" else (exponent, 100)
+    a, b = (np.ldexp(x, e).astype(np.float32) for x, e in zip((a, b), (high, low) if small == "right" else (low, high)))
+    print(f"operands of 2^{exponent}, {small}", flush=True)
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    err = _product(a, b).astype(np.float64) - want
+    floor = 4 * 2.0 ** -149 if small == "both" else 0.0
+    assert np.all(np.abs(err) <= 50 * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)) + floor)
+    assert np.linalg.norm(err) <= 3e-7 * np.linalg.norm(want) + floor * 1024
+
+
 def test_an_error_has_no_direction():
     """Sums over many rows of a result do not collect a bias: their error is that of as many
     independent errors (twice allowed; the MFMA's own roundings, all one way, would give 15 times)."""
