@@ -16,8 +16,8 @@
 // 64-bit sums the relative error is 0.25-0.3 of the fp32 MFMA tile's for K = 256 to 8192 (normal
 // operands, 2048: 1.8e-7 against 7.9e-7).
 // A value that is not finite, or that rounds past the largest bf16 value (scaled: see SPLIT_SCALE),
-// leaves NaN in every sum it enters, so a wave that ends with a sum that is not finite forms its
-// outputs again with fp32 MFMAs straight from memory: such outputs are the fp32 tile's.
+// leaves NaN in every sum it enters. Sums that end not finite are formed again with fp32 MFMAs
+// straight from memory: such outputs are the fp32 tile's, all others are not touched.
 //
 // What bounds it: six bf16 terms at 2.5 PFLOP/s are 417 TFLOP/s of fp32 products against 157 on the
 // fp32 MFMA; a large bf16 product of the vendor library reaches 1.2 PFLOP/s on this chip, a sixth of
@@ -331,39 +331,37 @@ __device__ __forceinline__ void gemm_split_tile(const float* __restrict__ A, con
   }
   multiply(sign, rounds - 1, true);
   // Lane l of the wave's tile (i, n) holds output row 16 i + l % 16, columns 16 n + 4 (l / 16) .. + 3.
-  // A sum that is not finite: this wave's outputs again, in fp32.
-  float finite = 0.0f;  // NaN once any sum is infinite or NaN
+  // Sums that are not finite again, in fp32: those alone, so that an output depends on its own row and
+  // column and on no neighbour, whatever the tile.
 #pragma unroll
-  for (int i = 0; i < TM; i++)
+  for (int i = 0; i < TM; i++) {
+    float finite = 0.0f;  // NaN once any sum of these 16 rows is infinite or NaN
 #pragma unroll
     for (int n = 0; n < TN; n++)
 #pragma unroll
       for (int r = 0; r < 4; r++) finite = __builtin_fmaf(acc[i][n][r], 0.0f, finite);
-  if (__ballot(!(finite == 0.0f)) != 0) {
+    if (__ballot(!(finite == 0.0f)) == 0) continue;
+    floatx4 again[TN];
 #pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-      for (int n = 0; n < TN; n++) acc[i][n] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int n = 0; n < TN; n++) again[n] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 1
     for (int k0 = kbeg; k0 < kend; k0 += 4) {
       const int k = min(k0 + lo, kend - 1);
       const bool live = k0 + lo < kend;
-      float y[TN];
+      const int64_t r = wm * WTM + i * 16 + li;
+      const float v = Ab[TA ? (int64_t)k * M + r : r * K + k];
+      const float x = live ? v : 0.0f;
 #pragma unroll
       for (int n = 0; n < TN; n++) {
         const int64_t c = wn * WTN + n * 16 + li;
-        const float v = Bb[TB ? c * K + k : (int64_t)k * N + c];
-        y[n] = live ? v : 0.0f;
-      }
-#pragma unroll
-      for (int i = 0; i < TM; i++) {
-        const int64_t r = wm * WTM + i * 16 + li;
-        const float v = Ab[TA ? (int64_t)k * M + r : r * K + k];
-        const float x = live ? v : 0.0f;
-#pragma unroll
-        for (int n = 0; n < TN; n++) acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[n], x, acc[i][n], 0, 0, 0);
+        const float w = Bb[TB ? c * K + k : (int64_t)k * N + c];
+        again[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(live ? w : 0.0f, x, again[n], 0, 0, 0);
       }
     }
+#pragma unroll
+    for (int n = 0; n < TN; n++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) acc[i][n][r] = acc[i][n][r] * 0.0f == 0.0f ? acc[i][n][r] : again[n][r];
   }
   // The outputs leave through LDS, 32 rows x 32 columns of a wave at a time, so that a lane stores
   // the same four columns of every eighth row and a store covers whole 128-byte runs of eight rows

@@ -108,6 +108,31 @@ def test_values_that_are_not_finite_spread_as_in_fp32(k):
     assert np.allclose(got[1000][row], want[1000][row], rtol=1e-5)
 
 
+@pytest.mark.parametrize("m,n,k", [(1024, 1024, 96), (4096, 1536, 64), (4096, 2048, 288), (256, 1024, 4096)])
+@pytest.mark.parametrize("ta,tb", [(False, True), (True, False)])
+def test_outputs_beside_others_that_are_not_finite_keep_their_bits(m, n, k, ta, tb):
+    """Infinities, NaN and huge values in some rows and columns change no bit of the others, on any
+    tile and wherever their row lies in a wave's."""
+    a, b = _operands(m, n, k, ta, tb)
+    print(f"values that are not finite in {m} x {n} x {k}, ta {ta}, tb {tb}", flush=True)
+    clean = _product(a, b, ta, tb)
+    rows, cols = np.zeros(m, bool), np.zeros(n, bool)
+    x, y = (a.T if ta else a), (b.T if tb else b)
+    for at, value in [(3, np.inf), (20, np.nan), (100, np.float32(3.4e38)), (m - 1, -np.inf)]:
+        x[at, at % k] = value
+        rows[at] = True
+    y[k - 1, 77] = np.nan
+    cols[77] = True
+    got = _product(a, b, ta, tb)
+    keep = ~rows[:, None] & ~cols[None, :]
+    assert np.array_equal(got[keep].view(np.uint32), clean[keep].view(np.uint32))
+    assert np.all(~np.isfinite(got[[3, 20, m - 1]])) and np.all(np.isnan(got[:, 77]))
+    other = np.arange(n) != 77
+    want = x[100].astype(np.float64) @ y[:, other].astype(np.float64)
+    fits = np.abs(want) < 3e38  # 3.4e38 times a value above 1 overflows
+    assert np.any(fits) and np.allclose(got[100, other][fits], want[fits], rtol=1e-5)
+
+
 def test_small_values_keep_their_precision():
     """Values down to 2^-100 (with factors that bring the products back into range) lose nothing."""
     a, b = _operands(1024, 1024, 256, False, False)
