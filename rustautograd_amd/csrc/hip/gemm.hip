@@ -358,11 +358,14 @@ __global__ void __launch_bounds__(256) k_gemm_f64(const double* __restrict__ A, 
 
 // C (M <= MR rows) = op(A) B with B row-major K x N (N >= 4). A block of
 // four waves owns 256 columns (a float4 per lane) and one K split; its waves take consecutive
-// quarters of the split, sum their k in increasing order, and combine in wave order through
-// LDS. With several splits, split s writes partials [s][M N], summed in split order afterwards.
-// The loop has no branches: a wave's K range is made uniform (readfirstlane), so op(A) values are
-// scalar loads that never wait on the B rows in flight; rows m >= M read row M - 1 and are not
-// stored.
+// quarters of the split and combine in wave order through LDS. With several splits, split s writes
+// partials [s][M N], summed in split order afterwards. Rows m >= M read row M - 1 and are not stored.
+// Bound by the latency of its loads (a wave or two per SIMD): B's next eight rows are loaded while
+// these are multiplied, and op(A)'s values of 64 k go through the wave's own part of LDS. (Read as
+// scalars, one load each, they took longer than B: 16 x 4096 x 4096 35 us, 25.6 here; 8 x 1024 x 4096
+// 16.8 and 14.6.) The products of 16 k are summed by themselves and then added, so that a wave's sum
+// meets one rounding of its own size per 16 k: 1.2e-7 against 64-bit sums at K = 4096, 1.7e-7 when
+// each was added to it.
 __device__ __forceinline__ float4 row4(const float* p) {
   const rowx4 x = *(const rowx4*)p;
   return make_float4(x[0], x[1], x[2], x[3]);
@@ -375,7 +378,9 @@ __device__ __forceinline__ float4 row4(const float* p, int left) {
 
 template <int MR>
 struct RowsLds {
-  static constexpr int FLOAT4S = 3 * MR * 64;  // the sums of waves 1..3; wave 0 keeps its own
+  static constexpr int SUMS = 3 * MR * 64;  // float4s: the sums of waves 1..3; wave 0 keeps its own
+  static constexpr int PANEL = 64 * MR / 4;  // a wave's op(A) values of 64 k; waves 1..3 have theirs where their sums go
+  static constexpr int FLOAT4S = SUMS + PANEL;
 };
 
 // op(A) of the streaming kernels, read through the constant address space: the launch never
@@ -384,41 +389,80 @@ struct RowsLds {
 typedef const __attribute__((address_space(4))) float* ConstOperand;
 
 // Block (bx, by) of k_gemm_skinny_rows, its wave sums combined through `lds`.
-template <int MR, int UNROLL = 8>
+template <int MR>
 __device__ __forceinline__ void skinny_rows_block(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ out, int M,
                                                   int N, int K, bool ta, int kps, uint32_t bx, uint32_t by, float4* lds) {
   float4(*red)[MR][64] = (float4(*)[MR][64])lds;
-  const ConstOperand Ac = (ConstOperand)A;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  float4(*panel)[MR / 4] = (float4(*)[MR / 4])(wave == 0 ? lds + RowsLds<MR>::SUMS : &red[wave - 1][0][0]);
   const int col = (bx * 64 + lane) * 4;
   const int colr = min(col, N - 4);
   const int k0 = by * kps, k1 = min(K, k0 + kps);
   const int quarter = (k1 - k0 + 3) / 4;
   const int kw0 = min(k1, k0 + wave * quarter), kw1 = min(k1, kw0 + quarter);
   const uint64_t sm = ta ? 1 : (uint64_t)K, sk = ta ? (uint64_t)M : 1;  // op(A)[m][k] = A[m * sm + k * sk]
-  float4 acc[MR];
+  float4 acc[MR], run[MR];
 #pragma unroll
-  for (int m = 0; m < MR; m++) acc[m] = make_float4(0.f, 0.f, 0.f, 0.f);
-  int k = kw0;
-  for (; k + UNROLL <= kw1; k += UNROLL) {
-    float4 b[UNROLL];
+  for (int m = 0; m < MR; m++) acc[m] = run[m] = make_float4(0.f, 0.f, 0.f, 0.f);
+  // The wave's op(A) values of 64 k from kc on, a k to a lane.
+  auto stage = [&](int kc) __attribute__((always_inline)) {
+    const int k = min(kc + lane, kw1 - 1);
+    float a[MR];
 #pragma unroll
-    for (int u = 0; u < UNROLL; u++) b[u] = row4(B + (uint64_t)(k + u) * N + colr);
+    for (int m = 0; m < MR; m++) a[m] = A[(uint64_t)min(m, M - 1) * sm + (uint64_t)k * sk];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int u = 0; u < UNROLL; u++)
+    for (int q = 0; q < MR / 4; q++) panel[lane][q] = make_float4(a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  auto load = [&](float4 (&b)[8], int k) __attribute__((always_inline)) {
 #pragma unroll
-      for (int m = 0; m < MR; m++) {
-        const float a = Ac[(uint64_t)min(m, M - 1) * sm + (uint64_t)(k + u) * sk];
-        acc[m] = make_float4(fmaf(a, b[u].x, acc[m].x), fmaf(a, b[u].y, acc[m].y), fmaf(a, b[u].z, acc[m].z), fmaf(a, b[u].w, acc[m].w));
+    for (int u = 0; u < 8; u++) b[u] = row4(B + (uint64_t)(k + u) * N + colr);
+  };
+  auto row = [&](int i, const float4& b) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < MR / 4; q++) {
+      const float4 t = panel[i][q];
+      const float a[4] = {t.x, t.y, t.z, t.w};
+#pragma unroll
+      for (int m = 0; m < 4; m++) {
+        float4& r = run[4 * q + m];
+        r = make_float4(fmaf(a[m], b.x, r.x), fmaf(a[m], b.y, r.y), fmaf(a[m], b.z, r.z), fmaf(a[m], b.w, r.w));
       }
-  }
-  for (; k < kw1; k++) {
-    const float4 b = row4(B + (uint64_t)k * N + colr);
+    }
+  };
+  auto add = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int m = 0; m < MR; m++) {
-      const float a = Ac[(uint64_t)min(m, M - 1) * sm + (uint64_t)k * sk];
-      acc[m] = make_float4(fmaf(a, b.x, acc[m].x), fmaf(a, b.y, acc[m].y), fmaf(a, b.z, acc[m].z), fmaf(a, b.w, acc[m].w));
+      acc[m] = make_float4(acc[m].x + run[m].x, acc[m].y + run[m].y, acc[m].z + run[m].z, acc[m].w + run[m].w);
+      run[m] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
+  };
+  const int whole = kw0 + (kw1 - kw0) / 8 * 8;
+  float4 b0[8], b1[8];
+  if (kw0 < whole) load(b0, kw0);
+  int kc = kw0;
+  if (kw0 < kw1) stage(kw0);
+#pragma unroll 1
+  for (int k = kw0; k < whole; k += 16) {
+    if (k - kc == 64) stage(kc = k);
+    const bool second = k + 8 < whole;
+    if (second) load(b1, k + 8);
+#pragma unroll
+    for (int u = 0; u < 8; u++) row(k - kc + u, b0[u]);
+    if (second) {
+      if (k + 16 < whole) load(b0, k + 16);
+#pragma unroll
+      for (int u = 0; u < 8; u++) row(k - kc + 8 + u, b1[u]);
+    }
+    add();
+  }
+  if (whole < kw1) {
+    if (whole - kc == 64) stage(kc = whole);
+    for (int k = whole; k < kw1; k++) row(k - kc, row4(B + (uint64_t)k * N + colr));
+    add();
   }
   if (wave > 0)
 #pragma unroll
@@ -443,7 +487,7 @@ __device__ __forceinline__ void skinny_rows_block(const float* __restrict__ A, c
 // 4 NC consecutive columns of C (NC per wave) and one K split of `kps` (a multiple of 256, at
 // most DOT_KPS); it copies its A panel to LDS while its first B rows load, so the loop's only
 // global loads are the B rows, four float4 steps deep. Lanes take k in float4 steps 256 apart, each lane summing its
-// share in increasing k; the 64 lane sums combine by a fixed xor butterfly, and with several
+// share in increasing k, four at a time; the 64 lane sums combine by a fixed xor butterfly, and with several
 // splits, split s writes partials [s][M N], summed in split order afterwards. Rows m >= M read
 // row M - 1 and are not stored. (For 16 rows the split is at most DOT_KPS / 2.)
 constexpr int DOT_KPS = 1024;
@@ -498,7 +542,7 @@ __device__ __forceinline__ void skinny_dot_block(const float* __restrict__ A, co
           const float4 a = panel[m][(kk + h * 256) / 4];
 #pragma unroll
           for (int c = 0; c < NC; c++)
-            acc[m][c] = fmaf(a.w, b[h][c].w, fmaf(a.z, b[h][c].z, fmaf(a.y, b[h][c].y, fmaf(a.x, b[h][c].x, acc[m][c]))));
+            acc[m][c] += fmaf(a.w, b[h][c].w, fmaf(a.z, b[h][c].z, fmaf(a.y, b[h][c].y, a.x * b[h][c].x)));
         }
     if (kk + 1024 < len) load(b, kk + 1024);
   }
@@ -549,11 +593,11 @@ __device__ __forceinline__ void outer_block(const float* __restrict__ A, const f
   }
 }
 
-template <int MR, int UNROLL = 8>
+template <int MR>
 __global__ void __launch_bounds__(256) k_gemm_skinny_rows(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ out,
                                                           int M, int N, int K, bool ta, int kps) {
   __shared__ float4 lds[RowsLds<MR>::FLOAT4S];
-  skinny_rows_block<MR, UNROLL>(A, B, out, M, N, K, ta, kps, blockIdx.x, blockIdx.y, lds);
+  skinny_rows_block<MR>(A, B, out, M, N, K, ta, kps, blockIdx.x, blockIdx.y, lds);
 }
 
 template <int MR, int NC>
@@ -691,6 +735,18 @@ bool use_mfma(int dtype, uint64_t m, uint64_t n, uint64_t k) {
   return dtype == RG_F32 && m >= side && n >= side && k >= 8 && m * n * k >= (1u << 18);
 }
 
+// Products up to which a block per output (k_gemm_tiny_out) is faster than the row kernel, or than
+// the dot kernel where each output is a product of two contiguous rows. Its time grows with their
+// number, the others' hardly does (us, M x N x K): rows 1x66x513 6 against 15, 8x66x2050 10 and 14,
+// 3x515x2050 19 and 18; 16x66x513 6 and 20, 16x515x513 21 and 20; dots 1x2050x4096 9 and 18,
+// 3x1001x4096 12 and 14, 8x1001x1000 11 and 10; 16x1001x513 11 and 15, 16x1024x2050 28 and 16. Its sums are also the more
+// exact, the lanes each taking a few k (1x1001x1000: 0.9e-7 against 64-bit sums, rows 1.0e-7).
+// A dot product of more than DOT_KPS takes a second launch.
+uint64_t tiny_products(uint64_t rows, uint64_t k, bool dots) {
+  if (dots) return rows <= 8 && k <= DOT_KPS ? 8u << 20 : 12u << 20;
+  return rows <= 8 ? 2u << 20 : 4u << 20;
+}
+
 // Which skinny kernel a product takes, from shapes and flags alone. Every size goes: a chain of
 // 8 x 2050 x 2050 products on the plain kernel instead took 10 times as long.
 Skinny skinny_plan(int dtype, uint64_t m, uint64_t n, uint64_t k, uint64_t batch, bool ta, bool tb) {
@@ -704,12 +760,15 @@ Skinny skinny_plan(int dtype, uint64_t m, uint64_t n, uint64_t k, uint64_t batch
     sk.kind = SKINNY_OUTER;
     return sk;
   }
-  if (m <= 16 && k >= 512 && n >= 64) {
+  // Few enough products for a block per output (skinny_plan's last rule) to take them all in the
+  // time the row and dot kernels take to start up (us on MI355X).
+  const bool tiny = m * n <= 16384 && k >= 512 && m * n * k <= tiny_products(std::min(m, n), k, n == 1 ? !ta : tb);
+  if (m <= 16 && k >= 512 && n >= 64 && !tiny) {
     if (!tb) sk.kind = SKINNY_ROWS;
     else if (!ta) sk.kind = SKINNY_DOT;
     if (sk.kind != SKINNY_NONE) return sk;
   }
-  if (n == 1 && k >= 512 && m >= 64) {
+  if (n == 1 && k >= 512 && m >= 64 && !tiny) {
     // op(A) x with A stored K x M (ta): rows kernel over A; stored M x K: dot kernel over A's rows.
     sk.swapped = true;
     sk.m = 1;
@@ -976,8 +1035,8 @@ bool gemm_skinny(hipStream_t s, const GemmArgs& g, const Skinny& sk) {
   const int splits = (K + kps - 1) / kps;
   float* out = splits > 1 ? (float*)g.workspace : C;
   dim3 grid((uint32_t)((N + 255) / 256), (uint32_t)splits);
-  if (M <= 8) hipLaunchKernelGGL((k_gemm_skinny_rows<8, 8>), grid, dim3(256), 0, s, A, B, out, M, N, K, sk.ta, kps);
-  else hipLaunchKernelGGL((k_gemm_skinny_rows<16, 8>), grid, dim3(256), 0, s, A, B, out, M, N, K, sk.ta, kps);
+  if (M <= 8) hipLaunchKernelGGL((k_gemm_skinny_rows<8>), grid, dim3(256), 0, s, A, B, out, M, N, K, sk.ta, kps);
+  else hipLaunchKernelGGL((k_gemm_skinny_rows<16>), grid, dim3(256), 0, s, A, B, out, M, N, K, sk.ta, kps);
   sum_splits(out, splits);
   return true;
 }
