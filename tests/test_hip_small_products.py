@@ -63,3 +63,9 @@ def test_float32_products_of_odd_sizes(m, n, k, ta, tb):
 @pytest.mark.parametrize("m,n,k", [(40, 24, 40), (33, 16, 50), (24, 24, 24), (5, 7, 60)])
 def test_batched_float32_products_of_odd_sizes(m, n, k):
     _check(m, n, k, False, False, "float32", (4, 6))
+
+
+def test_many_small_float64_products():
+    """Sides under a 64x64 and a 32x32 tile, in batches that would fill the chip with such tiles."""
+    _check(20, 20, 8, False, True, "float64", (2048,))
+    _check(16, 40, 9, False, False, "float64", (1024,))
