@@ -1127,7 +1127,8 @@ void gemm_small(hipStream_t s, const GemmArgs& g) {
   const uint64_t outputs = g.m * g.n;
   const bool rows = g.n == 1 && !g.ta;  // every output a contiguous row against one vector
   // A wave per output where K gives its lanes work and the outputs alone do not fill the chip.
-  if (g.k >= 32 && (outputs * g.batch <= 16384 || rows) && outputs < (1ull << 31)) {
+  // (A launch has fewer than 2^32 threads in x: fewer than 2^24 blocks of four outputs.)
+  if (g.k >= 32 && (outputs * g.batch <= 16384 || rows) && (outputs + 3) / 4 < (1ull << 24)) {
     const int w = outputs * g.batch >= 2048 ? 1 : g.k <= 512 ? 1 : g.k <= 2048 ? 4 : 16;
     const dim3 grid((uint32_t)(w == 1 ? (outputs + 3) / 4 : outputs), (uint32_t)g.batch);
 #define RG_DOTS(W_)                                                                                                                        \

@@ -69,3 +69,18 @@ def test_many_small_float64_products():
     """Sides under a 64x64 and a 32x32 tile, in batches that would fill the chip with such tiles."""
     _check(20, 20, 8, False, True, "float64", (2048,))
     _check(16, 40, 9, False, False, "float64", (1024,))
+
+
+def test_the_tallest_matrix_against_a_vector():
+    """2^26 - 1 rows of 32, just under the largest buffer: a wave per output would be a launch of 2^32
+    threads, one more than there may be. Every value is checked on a sample of rows and at both ends."""
+    rows, k = 2 ** 26 - 1, 32
+    gen = np.random.default_rng(1)
+    x, y, z = gen.standard_normal((rows, 1), dtype=np.float32), gen.standard_normal((1, k), dtype=np.float32), gen.standard_normal((k, 1), dtype=np.float32)
+    print(f"{rows} x 1 x {k}", flush=True)
+    args = tuple(rg.tensor(v) for v in (x, y, z))
+    got = rg.compile(lambda x, y, z: rg.maximum(x, y) @ z, args, validate="none", device="hip")(*args).numpy()
+    at = np.r_[0:1000, rows - 1000:rows, gen.integers(0, rows, 100000)]
+    a = np.maximum(x[at], y).astype(np.float64)
+    assert got.shape == (rows, 1)
+    assert np.all(np.abs(got[at] - a @ z) <= (k + 1) * 2.0 ** -24 * (np.abs(a) @ np.abs(z)))
