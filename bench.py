@@ -22,7 +22,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0       # MI355X HBM3E
-FP32_MFMA_PEAK_TFLOPS = 157.3
+FP32_MFMA_PEAK_TFLOPS = 157.3  # products on the bf16 cores, in six terms each, 16/6 of it (a step's peak_factor)
 
 
 def _numel(s):
@@ -53,10 +53,11 @@ def classify(plan, runs_in=None):
         members.setdefault(r, []).append(k)
 
     def add(name, k, st, launch=True):
-        c = classes.setdefault(name, {"steps": [], "flops": 0.0, "executed_flops": 0.0, "bytes": 0.0, "launches": 0})
+        c = classes.setdefault(name, {"steps": [], "flops": 0.0, "executed_flops": 0.0, "bytes": 0.0, "launches": 0, "at_peak": 0.0})
         c["steps"].append(k)
         if st["bound"] == "mfma":
             c["flops"] += st["flops"]
+            c["at_peak"] += st["flops"] / st.get("peak_factor", 1.0)  # flops at the fp32 peak that take as long at the step's own
             c["executed_flops"] += st.get("executed_flops", st["flops"])
         c["bytes"] += st["bytes"]
         c["launches"] += 1 if launch else 0
@@ -92,6 +93,11 @@ def classify(plan, runs_in=None):
         else:
             add("structural_other", k, st)
     return classes
+
+
+def peak_tflops(c):
+    """The rate a class of products would reach with every product at the peak of its units."""
+    return FP32_MFMA_PEAK_TFLOPS * c["flops"] / c["at_peak"]
 
 
 def time_classes(compiled, inputs, classes, repeats, trials=15):
@@ -214,8 +220,8 @@ def roofline_of(compiled, inputs, reps, workload):
     avg_s = dom["isolated_seconds"] / dom["launches"]
     achieved = per_launch / avg_s / (1e12 if dom["flops"] else 1e9)
     if dom["flops"]:
-        roof = {"bound": "mfma", "achieved": round(achieved, 2), "peak": FP32_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
-                "frac": round(achieved / FP32_MFMA_PEAK_TFLOPS, 4)}
+        peak = peak_tflops(dom)
+        roof = {"bound": "mfma", "achieved": round(achieved, 2), "peak": round(peak, 1), "unit": "TFLOP/s", "frac": round(achieved / peak, 4)}
     else:
         roof = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 4)}
@@ -224,7 +230,7 @@ def roofline_of(compiled, inputs, reps, workload):
                  "algorithmic_bytes_per_launch": round(dom["bytes"] / dom["launches"]), "avg_launch_us": round(avg_s * 1e6, 2),
                  "in_pass_avg_launch_us": round(dom["seconds"] / dom["launches"] * 1e6, 2)})
     kernels = {k: {"ms_per_step": round(v["seconds"] * 1e3, 3), "launches": v["launches"], "achieved": round(v["achieved"], 2),
-                   "unit": v["unit"], "frac": round(v["achieved"] / (FP32_MFMA_PEAK_TFLOPS if v["unit"] == "TFLOP/s" else HBM_PEAK_GBS), 4),
+                   "unit": v["unit"], "frac": round(v["achieved"] / (peak_tflops(v) if v["unit"] == "TFLOP/s" else HBM_PEAK_GBS), 4),
                    "isolated_ms_per_step": round(v["isolated_seconds"] * 1e3, 3), "timing": v["timing"]}
                for k, v in sorted(classes.items(), key=lambda kv: -kv[1]["seconds"])}
     for k, v in classes.items():
@@ -233,7 +239,7 @@ def roofline_of(compiled, inputs, reps, workload):
         if v["flops"] and v["executed_flops"] != v["flops"]:
             ex = v["executed_flops"] / v["seconds"] / 1e12
             kernels[k].update({"executed_share": round(v["executed_flops"] / v["flops"], 5), "executed_achieved": round(ex, 2),
-                               "executed_frac": round(ex / FP32_MFMA_PEAK_TFLOPS, 4)})
+                               "executed_frac": round(ex / peak_tflops(v), 4)})
     return roof, kernels, total_s
 
 

@@ -123,11 +123,16 @@ int rg_hip_exec_time_steps(void* exec, const int64_t* steps, int64_t n_steps, in
  * source is cut), or -1 with the message in `buf`. No reference counterpart. */
 int rg_hip_kernel_source(const int64_t* words, size_t n_words, char* buf, size_t len);
 /* Roofline support for `Compiled::profile` (validate.rs:875-919 times operations; this adds the
- * ceiling they are measured against), with no reference counterpart. Whether the backend runs
- * a product of op(A) m x k by op(B) k x n over `batch` problems through its bandwidth-bound
- * streaming kernels (1) or its matrix-core kernels (0): a pure function of the arguments that
- * touches no device. */
+ * ceiling they are measured against), with no reference counterpart. Whether a product of op(A)
+ * m x k by op(B) k x n over `batch` problems is priced by its bytes (1) or its operations (0): by
+ * bytes where the backend runs it through its bandwidth-bound streaming kernels, but for dot
+ * products (B transposed, or n = 1) over a K that 256 does not divide, which stream as well and are
+ * priced by their operations. A pure function of the arguments that touches no device. */
 int rg_hip_gemm_streamed(int32_t dtype, int64_t m, int64_t n, int64_t k, int64_t batch, int32_t ta, int32_t tb);
+/* The rate such a product could reach on the units that it runs on, as a multiple of the device's
+ * peak of its type (peaks[1] or peaks[2] below): 16 / 6 for fp32 products on the bf16 matrix cores,
+ * 16 times as fast and six terms a product; 1 otherwise. Pure, as above. */
+double rg_hip_gemm_peak_factor(int32_t dtype, int64_t m, int64_t n, int64_t k, int64_t batch, int32_t ta, int32_t tb);
 /* The current device's published peaks: peaks[0] HBM bandwidth in GB/s, peaks[1] dense fp32
  * matrix-core TFLOP/s, peaks[2] dense fp64 matrix-core TFLOP/s, and its name in `name`.
  * Returns 0, or 1 (message in `name`) when no device is visible or it has no published figures. */

@@ -1343,6 +1343,7 @@ int rg_cpu_exec_step_timed(void* exec, double* seconds) {
   return 0;
 }
 
+double rg_cpu_gemm_peak_factor(int32_t, int64_t, int64_t, int64_t, int64_t, int32_t, int32_t) { return 1.0; }
 int rg_cpu_threads(void) { return omp_get_max_threads(); }
 void rg_cpu_set_threads(int n) { omp_set_num_threads(n); }
 void rg_cpu_set_row_parallel_gemm(int on) { g_row_parallel_gemm = on != 0; }

@@ -60,6 +60,7 @@ void register_backend(const std::string& name, const std::string& path, const st
   bind(*b, b->exec_time_steps, "exec_time_steps", false);
   bind(*b, b->exec_run, "exec_run", false);
   bind(*b, b->gemm_streamed, "gemm_streamed", false);
+  bind(*b, b->gemm_peak_factor, "gemm_peak_factor", false);
   bind(*b, b->device_peaks, "device_peaks", false);
   g_backends.push_back(std::move(b));
 }

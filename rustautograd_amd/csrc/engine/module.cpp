@@ -327,16 +327,17 @@ PYBIND11_MODULE(_rg, m) {
            [](const PyCompiled& c) {
              // Per-step description for measurement tools: kind, op, dtype, n, shapes.
              py::list out;
-             const StreamedFn streamed = c.c->streamed_products();
+             const PriceFn price = c.c->product_prices();
              for (auto& s : c.c->plan.steps) {
                py::dict d;
-               // Algorithmic work: flops priced against the matrix-core peak ("mfma"), or bytes
-               // against HBM bandwidth ("hbm").
-               const StepWork w = step_work(s, streamed);
+               // Algorithmic work: flops priced against `peak_factor` times the matrix-core peak
+               // ("mfma"), or bytes against HBM bandwidth ("hbm").
+               const StepWork w = step_work(s, price);
                d["flops"] = w.flops;
                d["executed_flops"] = w.executed_flops;
                d["bytes"] = w.bytes;
                d["bound"] = w.compute ? "mfma" : "hbm";
+               d["peak_factor"] = w.peak_factor;
                if (s.attn) {
                  const Attn& a = s.att;
                  d["kind"] = "attention";

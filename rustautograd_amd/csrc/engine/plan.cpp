@@ -1245,7 +1245,7 @@ size_t Plan::n_fused_ops() const {
   return k;
 }
 
-StepWork step_work(const Step& s, const StreamedFn& streamed) {
+StepWork step_work(const Step& s, const PriceFn& price) {
   StepWork w;
   if (s.attn) {
     const AttnShape& a = s.att.shape;
@@ -1330,7 +1330,9 @@ StepWork step_work(const Step& s, const StreamedFn& streamed) {
       w.flops = 2.0 * (double)m * (double)n * (double)k * (double)batch;
       w.executed_flops = w.flops;
       w.bytes = (in_elems + (double)i.n) * ds;
-      w.compute = i.dtype != DType::I32 && !(streamed && streamed(i.dtype, m, n, k, batch, ta, tb));
+      const double factor = price ? price(i.dtype, m, n, k, batch, ta, tb) : 1.0;
+      w.compute = i.dtype != DType::I32 && factor > 0;
+      if (w.compute) w.peak_factor = factor;
       return w;
     }
     case RG_OP_TAKE:

@@ -199,16 +199,17 @@ struct Plan {
 // Algorithmic work of one step, the figure a roofline divides by its time: the flops of products
 // (fused attention, and matrix products on matrix cores) priced against the matrix-core peak, and
 // for every other step the bytes it must move at least (each distinct input read once, each output
-// written once) priced against HBM bandwidth. `streamed` says whether the device runs a product
-// of these dimensions through bandwidth-bound kernels (then it is priced by its bytes); when it is
-// empty every floating-point product is priced by its flops.
+// written once) priced against HBM bandwidth. `price` says how the device prices a product of these
+// dimensions: 0 by its bytes (it streams), else by its flops against that multiple of the matrix-core
+// peak; when it is empty every floating-point product is priced by its flops against the peak.
 struct StepWork {
   double flops = 0, bytes = 0;
   double executed_flops = 0;  // the flops the device executes: attention skips hidden tiles
   bool compute = false;       // priced by flops
+  double peak_factor = 1;     // against this multiple of the matrix-core peak
 };
-using StreamedFn = std::function<bool(DType, uint64_t m, uint64_t n, uint64_t k, uint64_t batch, bool ta, bool tb)>;
-StepWork step_work(const Step& s, const StreamedFn& streamed);
+using PriceFn = std::function<double(DType, uint64_t m, uint64_t n, uint64_t k, uint64_t batch, bool ta, bool tb)>;
+StepWork step_work(const Step& s, const PriceFn& price);
 
 // Buffer assignment by last use, scanning steps in order; with reuse=false no buffer is shared (plan.rs:462-465).
 Plan build_plan(const Graph& g, const std::vector<uint32_t>& outputs, bool reuse);

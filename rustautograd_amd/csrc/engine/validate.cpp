@@ -805,10 +805,11 @@ Json Compiled::validate(const std::vector<Tensor>& examples) {
   return r;
 }
 
-StreamedFn Compiled::streamed_products() const {
-  if (!device->gemm_streamed) return {};
+PriceFn Compiled::product_prices() const {
   return [d = device](DType dt, uint64_t m, uint64_t n, uint64_t k, uint64_t batch, bool ta, bool tb) {
-    return d->gemm_streamed((int32_t)dt, (int64_t)m, (int64_t)n, (int64_t)k, (int64_t)batch, ta, tb) != 0;
+    auto ask = [&](auto f) { return f((int32_t)dt, (int64_t)m, (int64_t)n, (int64_t)k, (int64_t)batch, (int32_t)ta, (int32_t)tb); };
+    if (d->gemm_streamed && ask(d->gemm_streamed) != 0) return 0.0;
+    return d->gemm_peak_factor ? ask(d->gemm_peak_factor) : 1.0;
   };
 }
 
@@ -842,7 +843,7 @@ Json Compiled::profile(const std::vector<Tensor>& inputs, size_t repeats) const 
   }
   // Each operation's algorithmic work (flops against the matrix-core peak, or bytes against HBM
   // bandwidth), as the device runs it, and the device's published peaks when it reports them.
-  const StreamedFn streamed = streamed_products();
+  const PriceFn price = product_prices();
   double peaks[3] = {0, 0, 0};
   Json roofline = Json::obj();
   bool have_peaks = false;
@@ -864,6 +865,7 @@ Json Compiled::profile(const std::vector<Tensor>& inputs, size_t repeats) const 
     double seconds = 0, flops = 0, executed_flops = 0, bytes = 0;
     size_t count = 0;
     bool compute = false, f64 = false;
+    double peak_factor = 1;
   };
   std::map<std::string, Row> rows;
   auto shape_str = [](const Shape& s) {
@@ -906,9 +908,9 @@ Json Compiled::profile(const std::vector<Tensor>& inputs, size_t repeats) const 
     double all = 0, flops = 0;
     for (size_t q : g) {
       all += sec[q];
-      flops += step_work(plan.steps[q], streamed).flops;
+      flops += step_work(plan.steps[q], price).flops;
     }
-    for (size_t q : g) sec[q] = flops > 0 ? all * step_work(plan.steps[q], streamed).flops / flops : all / (double)g.size();
+    for (size_t q : g) sec[q] = flops > 0 ? all * step_work(plan.steps[q], price).flops / flops : all / (double)g.size();
   }
   for (size_t s0 = 0; s0 < plan.steps.size(); s0++) {
     const size_t s = row_of[s0];
@@ -931,11 +933,11 @@ Json Compiled::profile(const std::vector<Tensor>& inputs, size_t repeats) const 
       dt = st.instr.dtype;
     }
     if (dt == DType::F64) key += " f64";
-    const StepWork w = step_work(st, streamed);
+    const StepWork w = step_work(st, price);
     Row& r = rows[key];
     r.seconds += sec[s0];
     if (s0 != s) {  // the group in the product's epilogue
-      r.bytes += step_work(plan.steps[s0], streamed).bytes;
+      r.bytes += step_work(plan.steps[s0], price).bytes;
       continue;
     }
     r.count++;
@@ -943,6 +945,7 @@ Json Compiled::profile(const std::vector<Tensor>& inputs, size_t repeats) const 
     r.executed_flops += w.executed_flops;
     r.bytes += w.bytes;
     r.compute = w.compute;
+    r.peak_factor = w.peak_factor;
     r.f64 = dt == DType::F64;
   }
   double total = 0;
@@ -966,7 +969,7 @@ Json Compiled::profile(const std::vector<Tensor>& inputs, size_t repeats) const 
     o["unit"] = v.compute ? "TFLOP/s" : "GB/s";
     if (per_run > 0) o["achieved"] = work / per_run;
     if (have_peaks) {
-      const double peak = v.compute ? (v.f64 ? peaks[2] : peaks[1]) : peaks[0];
+      const double peak = v.compute ? (v.f64 ? peaks[2] : peaks[1]) * v.peak_factor : peaks[0];
       o["peak"] = peak;
       if (per_run > 0) o["fraction_of_peak"] = work / per_run / peak;
       // Attention skips the tiles a mask hides: its rate over the products it executes.

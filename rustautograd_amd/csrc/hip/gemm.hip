@@ -926,6 +926,10 @@ bool gemm_streamed(int dtype, uint64_t m, uint64_t n, uint64_t k, uint64_t batch
   return sk.kind != SKINNY_NONE && !(sk.kind == SKINNY_DOT && k % 256 != 0);
 }
 
+bool gemm_on_bf16_terms(int dtype, uint64_t m, uint64_t n, uint64_t k, uint64_t batch, bool ta, bool tb) {
+  return skinny_plan(dtype, m, n, k, batch, ta, tb).kind == SKINNY_NONE && use_mfma(dtype, m, n, k) && pick_tile(m, n, k, batch).split != 0;
+}
+
 int gemm_splits(int dtype, uint64_t m, uint64_t n, uint64_t k, uint64_t batch, bool ta, bool tb) {
   if (m == 0 || n == 0 || batch == 0) return 1;
   const Skinny sk = skinny_plan(dtype, m, n, k, batch, ta, tb);

@@ -186,9 +186,10 @@ void attention_backward(hipStream_t s, const AttnArgs& a);
 // problem for each pass, which holds all of the problem's rows.
 bool attention_backward_column_sums(const AttnArgs& a);
 
-// Whether the product runs through the bandwidth-bound skinny kernels (alignment aside: an
-// unaligned operand falls back to the general kernels at launch).
+// Whether the product is priced by its bytes (rg_hip_gemm_streamed), and whether it runs on the bf16
+// matrix cores (gemm_split.h).
 bool gemm_streamed(int dtype, uint64_t m, uint64_t n, uint64_t k, uint64_t batch, bool ta, bool tb);
+bool gemm_on_bf16_terms(int dtype, uint64_t m, uint64_t n, uint64_t k, uint64_t batch, bool ta, bool tb);
 
 // The number of K splits the product runs with (1: none), and the workspace bytes its split-K
 // partials need.

@@ -2013,6 +2013,11 @@ int rg_hip_gemm_streamed(int32_t dtype, int64_t m, int64_t n, int64_t k, int64_t
   return rgk::gemm_streamed(dtype, (uint64_t)m, (uint64_t)n, (uint64_t)k, (uint64_t)batch, ta != 0, tb != 0) ? 1 : 0;
 }
 
+double rg_hip_gemm_peak_factor(int32_t dtype, int64_t m, int64_t n, int64_t k, int64_t batch, int32_t ta, int32_t tb) {
+  if (m <= 0 || n <= 0 || k <= 0 || batch <= 0) return 1.0;
+  return rgk::gemm_on_bf16_terms(dtype, (uint64_t)m, (uint64_t)n, (uint64_t)k, (uint64_t)batch, ta != 0, tb != 0) ? 16.0 / 6.0 : 1.0;
+}
+
 int rg_hip_device_peaks(double* peaks, char* name, size_t len) {
   int dev = 0, n = 0;
   hipDeviceProp_t prop;

@@ -151,6 +151,20 @@ def test_the_backend_says_which_products_it_streams(m, n, k, batch, ta, tb, want
     assert _hip().rg_hip_gemm_streamed(1, m, n, k, batch, ta, tb) == 0
 
 
+@pytest.mark.parametrize("m,n,k,batch,ta,tb,bf16", [
+    (4096, 2048, 2048, 1, 0, 0, True), (1000, 1028, 100, 1, 1, 1, True), (300, 300, 64, 20, 0, 1, True),   # a block of the split tile per CU
+    (1024, 1024, 128, 1, 0, 0, True), (960, 1024, 128, 1, 0, 0, False),                                    # just that, and one row of tiles less
+    (512, 512, 512, 1, 0, 0, False), (64, 63, 4096, 600, 0, 0, False), (8, 4096, 4096, 1, 0, 0, False),    # fp32 tiles, a short side, streamed
+])
+def test_the_backend_says_which_products_run_on_the_bf16_cores(m, n, k, batch, ta, tb, bf16):
+    """Six bf16 terms a product at 16 times the fp32 matrix cores' rate."""
+    lib = ctypes.CDLL(_native.HIP_LIBRARY)
+    lib.rg_hip_gemm_peak_factor.restype = ctypes.c_double
+    lib.rg_hip_gemm_peak_factor.argtypes = [ctypes.c_int32] + [ctypes.c_int64] * 4 + [ctypes.c_int32] * 2
+    assert lib.rg_hip_gemm_peak_factor(0, m, n, k, batch, ta, tb) == (16 / 6 if bf16 else 1.0)
+    assert lib.rg_hip_gemm_peak_factor(1, m, n, k, batch, ta, tb) == 1.0  # float64
+
+
 def test_without_a_device_the_backend_reports_no_peaks():
     lib = _hip()
     peaks = (ctypes.c_double * 3)()
