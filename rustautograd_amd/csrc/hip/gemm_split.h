@@ -6,15 +6,19 @@
 // Every fp32 operand value is split exactly into three bf16 values, each the rounding of what the
 // ones before it left (8 bits of the 24 each): x = x1 + x2 + x3. A product is the sum of the six
 // terms a1 b1, a1 b2, a2 b1, a2 b2, a1 b3 and a3 b1; what is left out, a2 b3 + a3 b2 + a3 b3, is at
-// most 2^-25 of it, half an fp32 rounding. v_mfma_f32_16x16x32_bf16 sums a lane's eight exact terms
+// most 2^-24 of it, one fp32 rounding (a2 up to 2^-8 and a3 up to 2^-17 of a, two such terms). v_mfma_f32_16x16x32_bf16 sums a lane's eight exact terms
 // on the largest one's scale (bits below 2^-24 of it cut off) and adds the four lanes' sums to the
 // accumulator one after the other, each addition rounded, with a small bias downwards. So the terms
 // of one K step of 32 are summed from zero, small terms first, and the step's sum is added to the
 // running one by an ordinary addition: the MFMA's roundings are then on the scale of one step. Odd
 // steps form the sum of a (-b) and subtract it, which turns their bias the other way (without that
 // it made up a quarter of the error at K = 5000 and showed in sums over a gradient's rows). Against
-// 64-bit sums the relative error is 0.25-0.3 of the fp32 MFMA tile's for K = 256 to 8192 (normal
-// operands, 2048: 1.8e-7 against 7.9e-7).
+// 64-bit sums the relative error is 0.40 of the fp32 MFMA tile's at K = 24, 0.24 at 256 and 0.13 from
+// 2048 on (normal operands, 4096: 1.0e-7 against 8.1e-7). Only where a sum has few terms that are not
+// zero is it larger: a single product errs by 3.5e-8 in the mean and 1.6e-7 at most (fp32: one rounding,
+// 2.5e-8 and 6e-8), sums of four by 5.0e-8 (4.0e-8). (With the a1 b1 sums formed apart from the small
+// terms' and added by fp32 additions, 2.6e-8 and 4.4e-8; but the 128x128 tile, at its 128 registers,
+// spills: 4096 x 512 x 2048 MLP steps 20 % slower.)
 // A value that is not finite, or that rounds past the largest bf16 value (scaled: see SPLIT_SCALE),
 // leaves NaN in every sum it enters. Sums that end not finite are formed again with fp32 MFMAs
 // straight from memory: such outputs are the fp32 tile's, all others are not touched.

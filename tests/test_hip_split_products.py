@@ -5,7 +5,7 @@ ones too, so that rows start at any 4-byte address), K remainders and a K below 
 over blocks, batches, every transposition.
 
 Bounds. An operand's three bf16 parts are exact, and the terms left out of a product are at most
-2^-25 of it. Within a step of 32 k a sum meets at most 24 roundings of 2^-24 and seven cut-off terms
+2^-24 of it. Within a step of 32 k a sum meets at most 24 roundings of 2^-24 and seven cut-off terms
 of 2^-24 per eight, relative to the step's sum of magnitudes; each step's sum is then added with one
 rounding, and so are K-split partials: an output is within (32 + K / 32 + 16) 2^-24 of the sum of its
 products' magnitudes. Those roundings are random, so over a whole result the relative error is far
@@ -72,6 +72,37 @@ def test_batched_split_products_match_64_bit_sums(m, n, k):
     got = _product(a, b, False, True).astype(np.float64)
     want = _wide(a, False) @ _wide(b, True)
     assert np.linalg.norm(got - want) <= 3e-7 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("m,n,k", [(1024, 1024, 96), (4096, 2048, 288)])
+def test_one_product_in_a_sum(m, n, k):
+    """Sums with a single term that is not zero: the terms left out (1), the cut of the a1 b1 product to
+    the sum of the small terms (2, a truncation) and the small terms' own roundings (2^-8 of as much):
+    3.1 2^-24 of the product at most, and 4e-8 in the mean (3.5e-8 measured, an fp32 rounding is 2.5e-8)."""
+    gen = np.random.default_rng(k)
+    a, b = np.zeros((m, k), np.float32), gen.standard_normal((k, n), dtype=np.float32)
+    a[np.arange(m), gen.integers(0, k, m)] = gen.standard_normal(m, dtype=np.float32)
+    print(f"one product in a sum, {m} x {n} x {k}", flush=True)
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    err = np.abs(_product(a, b) - want)
+    assert np.all(err <= 3.1 * 2.0 ** -24 * np.abs(want)) and np.linalg.norm(err) <= 4e-8 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("signs", [False, True])
+@pytest.mark.parametrize("k", [64, 1000])
+def test_operands_whose_left_out_terms_are_the_largest(k, signs):
+    """1 + 2^-8 - 2^-17 squared: a2 b3 + a3 b2 + a3 b3 is 0.99 2^-24 of it, all one way, in every product
+    (of either sign). Beside that a K step's sum meets the roundings above."""
+    x = np.float32(1 + 2.0 ** -8 - 2.0 ** -17)
+    gen = np.random.default_rng(k)
+    a, b = np.full((1024, k), x), np.full((k, 1024), x)
+    if signs:
+        a, b = (v * gen.choice(np.float32([-1, 1]), v.shape) for v in (a, b))
+    print(f"the largest terms left out, K {k}, signs {signs}", flush=True)
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    err = np.abs(_product(a, b) - want)
+    assert np.all(err <= (32 + k / 32 + 16) * 2.0 ** -24 * k * float(x) ** 2)
+    assert np.linalg.norm(err) <= 3e-7 * np.linalg.norm(want)
 
 
 def test_integers_up_to_24_bits_stay_exact():
