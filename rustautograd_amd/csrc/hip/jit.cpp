@@ -263,8 +263,9 @@ std::string generate_gemm(const rgplan::Fused& f, int64_t c_slot, bool store_c, 
   // At least two waves per SIMD (at most 256 registers a wave, far above what the tile uses): with
   // that bound the compiler keeps the MFMA accumulators in ordinary VGPRs, as the precompiled
   // tiles are built (-amdgpu-mfma-vgpr-form), rather than copying them through AGPRs. Eight-wave
-  // tiles of one step share a CU in pairs: at most 128 registers.
-  const char* regs = nt > 256 && t.steps == 1 ? ", amdgpu_num_vgpr(128)" : "";
+  // tiles of one step share a CU in pairs, at most 128 registers a wave: the launch bound is the
+  // pair's threads (amdgpu_num_vgpr(128) did not hold the compiler to it).
+  const int bound = nt > 256 && t.steps == 1 ? 2 * nt : nt;
   // The epilogue's pointers arrive as kernel parameters, restrict-qualified when no output shares
   // a slot with an input or the product, so that the compiler may issue an output's loads before
   // the stores of the outputs before it.
@@ -274,7 +275,7 @@ std::string generate_gemm(const rgplan::Fused& f, int64_t c_slot, bool store_c, 
     for (auto& in : f.inputs) alias |= in.slot == o.second;
   }
   const char* R = alias ? "" : "__restrict__ ";
-  s << "extern \"C\" __global__ void __launch_bounds__(" << nt << ") __attribute__((amdgpu_waves_per_eu(2)" << regs << ")) " << name
+  s << "extern \"C\" __global__ void __launch_bounds__(" << bound << ") __attribute__((amdgpu_waves_per_eu(2))) " << name
     << "(const float* __restrict__ A, const float* __restrict__ B, int M, int N, int K, const rgg::int64_t* a_off, const rgg::int64_t* b_off, "
        "rgg::uint64_t a_stride, rgg::uint64_t b_stride, int splits, int kps, const float* __restrict__ bias, rgg::uint32_t tiles_m, "
        "rgg::uint32_t tiles_n, float* "

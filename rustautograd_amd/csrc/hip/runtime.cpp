@@ -786,10 +786,10 @@ bool flat_product(const Instr& i, uint64_t* m, uint64_t* n, uint64_t* k, bool* t
 //    activation gradient that reads it, whose output reuses the slot the weight gradient reads).
 // Groups small enough to be merged are left to the merged launches. The product's kernel also
 // stores its own output when another step reads it. Only large products are taken, of 2^23 outputs
-// at K up to 1024 and 2^24 above: the epilogue's loads and stores run beside little matrix work, and
-// what is saved is one pass over the product's output (measured on MI355X with fp32 MFMA tiles: C4's
-// GELU forward and backward, 8192 x 1024 outputs at K = 256, 1.7 % off the step; C2's activation
-// gradient at K = 2048 and its 2048 x 2048 AdamW update 1.1 % slower fused). RG_HIP_EPILOGUE=0 turns
+// at K up to 1024 and 2^24 above: what is saved is one pass over the product's output (C4's GELU
+// forward and backward, 8192 x 1024 outputs at K = 256: the step 3006 -> 2882 us). The line dates from
+// the fp32 MFMA tiles, on which products under it were slower fused; on split tiles they no longer
+// are (every product that qualifies, C2: 897 -> 858 us, C3: 723 -> 700 us). RG_HIP_EPILOGUE=0 turns
 // this off; RG_HIP_EPILOGUE=all takes every product that qualifies otherwise.
 uint64_t epilogue_min_outputs(uint64_t k) { return k <= 1024 ? 1ull << 23 : 1ull << 24; }
 

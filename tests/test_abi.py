@@ -195,6 +195,16 @@ def test_product_epilogue_kernels_compile_for_gfx950(monkeypatch):
     assert n >= 5, err
 
 
+def test_eight_wave_product_epilogues_leave_room_for_two_blocks():
+    """A kernel of 512 threads whose tile holds one K step is compiled for two blocks' threads a CU: at most
+    128 registers a wave. With 155, one block ran on a CU at a time and the epilogue cost more than it saved."""
+    g = G()
+    x, w = g.input((8192, 256), "float32"), g.input((256, 1024), "float32")
+    words, _ = _rg.plan_words(g.g, [g.un("tanh", g.op("matmul", [x, w]))], "hip", "standard")
+    src = _kernel_source(words)
+    assert "rgg::gemm_mfma_block<128, 128, 2, 4, 1," in src and "__launch_bounds__(1024)" in src
+
+
 def test_c3_program_compiles_for_gfx950():
     """Every fused kernel of a whole GPT training step (C3 at reduced depth) compiles."""
     cfg = workloads.GPT_CONFIGS["C3"]._replace(batch=2, block=16, layers=1)
