@@ -200,7 +200,8 @@ def test_eight_wave_product_epilogues_leave_room_for_two_blocks():
     128 registers a wave. With 155, one block ran on a CU at a time and the epilogue cost more than it saved."""
     g = G()
     x, w = g.input((8192, 256), "float32"), g.input((256, 1024), "float32")
-    words, _ = _rg.plan_words(g.g, [g.un("tanh", g.op("matmul", [x, w]))], "hip", "standard")
+    y = g.op("matmul", [x, w])
+    words, _ = _rg.plan_words(g.g, [g.un("tanh", g.bin("mul", y, y))], "hip", "standard")
     src = _kernel_source(words)
     assert "rgg::gemm_mfma_block<128, 128, 2, 4, 1," in src and "__launch_bounds__(1024)" in src
 
