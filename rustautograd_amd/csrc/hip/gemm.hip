@@ -38,15 +38,15 @@ namespace {
 
 using namespace rgg;
 
-template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB, int MODE, int MS>
+template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB, int MODE>
 __global__ void __launch_bounds__(64 * WM * WN) k_gemm_f32(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C,
                                                            int M, int N, int K, const int64_t* a_off, const int64_t* b_off,
                                                            uint64_t a_stride, uint64_t b_stride, int splits, int k_per_split,
-                                                          float* __restrict__ partial, const float* __restrict__ bias, uint32_t tiles_m,
-                                                          uint32_t tiles_n, int swizzle) {
+                                                           float* __restrict__ partial, const float* __restrict__ bias, uint32_t tiles_m,
+                                                           uint32_t tiles_n) {
   rgg::StoreC epi{C, partial, splits, (uint64_t)M * N};
-  rgg::gemm_f32_block<BM, BN, BK, WM, WN, TA, TB, MODE, MS>(A, B, M, N, K, a_off, b_off, a_stride, b_stride, splits, k_per_split, bias,
-                                                              tiles_m, tiles_n, swizzle, epi);
+  rgg::gemm_f32_block<BM, BN, BK, WM, WN, TA, TB, MODE>(A, B, M, N, K, a_off, b_off, a_stride, b_stride, splits, k_per_split, bias, tiles_m,
+                                                        tiles_n, epi);
 }
 
 // Waves per SIMD the registers must leave room for: two 128x128 blocks of eight waves per CU (one
@@ -115,8 +115,8 @@ template <int FLAGS, int I>
 __device__ __forceinline__ void small_part(const GroupPart& p, uint32_t bid, float* smem) {
   constexpr bool TA = (FLAGS >> (2 * I + 1)) & 1, TB = (FLAGS >> (2 * I)) & 1;
   StoreC epi{p.c, p.part, p.splits, (uint64_t)p.m * p.n};
-  gemm_f32_tile<32, 32, 32, 2, 2, TA, TB, LOAD_EVEN, 16>(p.a, p.b, p.m, p.n, p.k, nullptr, nullptr, 0, 0, p.splits, p.kps, p.bias, p.tm, p.tn, 1,
-                                                         epi, bid, p.blocks, smem);
+  gemm_f32_tile<32, 32, 32, 2, 2, TA, TB, LOAD_EVEN>(p.a, p.b, p.m, p.n, p.k, nullptr, nullptr, 0, 0, p.splits, p.kps, p.bias, p.tm, p.tn, epi,
+                                                     bid, p.blocks, smem);
 }
 
 template <int N, int FLAGS>
@@ -250,7 +250,7 @@ __global__ void __launch_bounds__(256) k_gemm_f64(const double* __restrict__ A, 
   __shared__ double part[WK > 1 ? (WK - 1) * BM * BN : 1];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, lo = lane >> 4;
   const int wk = wave / (WM * WN), wm = wave / WN % WM, wn = wave % WN;
-  const TileIndex ti = tile_of(blockIdx.x, gridDim.x, tiles_m, tiles_n, 1);
+  const TileIndex ti = tile_of(blockIdx.x, gridDim.x, tiles_m, tiles_n);
   const int m0 = ti.tm * BM, n0 = ti.tn * BN;
   const double* a = A + batch_offset(a_off, a_stride, ti.z);
   const double* b = B + batch_offset(b_off, b_stride, ti.z);
@@ -883,8 +883,8 @@ void launch_mode(hipStream_t s, int mode, const Launch& l) {
 #undef RG_GEMM
   } else {
 #define RG_GEMM(MODE_)                                                                                                                \
-  hipLaunchKernelGGL((k_gemm_f32<BM, BN, 32, WM, WN, TA, TB, MODE_, 16>), l.grid, block, 0, s, l.a, l.b, l.c, l.m, l.n, l.k, l.a_off, l.b_off, \
-                     l.as, l.bs, l.splits, l.kps, l.part, l.bias, l.tm, l.tn, 1)
+  hipLaunchKernelGGL((k_gemm_f32<BM, BN, 32, WM, WN, TA, TB, MODE_>), l.grid, block, 0, s, l.a, l.b, l.c, l.m, l.n, l.k, l.a_off, l.b_off, \
+                     l.as, l.bs, l.splits, l.kps, l.part, l.bias, l.tm, l.tn)
     if (mode == LOAD_EVEN) RG_GEMM(LOAD_EVEN);
     else if (mode == LOAD_VEC) RG_GEMM(LOAD_VEC);
     else RG_GEMM(LOAD_SCALAR);

@@ -7,26 +7,6 @@
 
 namespace rgg {
 
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-
-// One MFMA step of shape MS x MS (16x16x4 or 32x32x2 f32): lane l supplies row (A) / column (B)
-// l % MS at k = l / MS, and register r of its accumulator holds row 8 (r / 4) + 4 (l / MS) + r % 4,
-// column l % MS.
-template <int MS>
-struct Mfma;
-template <>
-struct Mfma<16> {
-  typedef floatx4 acc_t;
-  static constexpr int REGS = 4;
-  static __device__ __forceinline__ acc_t step(float a, float b, acc_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-};
-template <>
-struct Mfma<32> {
-  typedef floatx16 acc_t;
-  static constexpr int REGS = 16;
-  static __device__ __forceinline__ acc_t step(float a, float b, acc_t c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
-};
-
 // Load modes: every vector inside the operand (no checks), checked 16-byte vectors, or checked
 // scalar loads (operands whose rows are not 16-byte aligned).
 enum LoadMode { LOAD_EVEN = 0, LOAD_VEC = 1, LOAD_SCALAR = 2 };
@@ -100,18 +80,18 @@ struct TileLds {
 // The tile of block `bid` of a product launched as `nb` blocks, staging through `smem` (at least
 // TileLds<...>::FLOATS floats of LDS): a kernel that runs two products side by side gives each
 // its share of the grid and the same LDS.
-template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB, int MODE, int MS, class Epi>
+template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB, int MODE, class Epi>
 __device__ __forceinline__ void gemm_f32_tile(const float* __restrict__ A, const float* __restrict__ B, int M, int N, int K,
                                                const int64_t* a_off, const int64_t* b_off, uint64_t a_stride, uint64_t b_stride, int splits,
                                                int k_per_split, const float* __restrict__ bias, uint32_t tiles_m, uint32_t tiles_n,
-                                               int swizzle, Epi& epi, uint32_t bid, uint32_t nb, float* smem) {
+                                               Epi& epi, uint32_t bid, uint32_t nb, float* smem) {
   constexpr int NT = 64 * WM * WN;
-  constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / MS, TN = WTN / MS;
-  static_assert(TM >= 1 && TN >= 1 && TM <= 4 && TN <= 4 && (TM & (TM - 1)) == 0 && (TN & (TN - 1)) == 0, "wave tiles");
-  // A group of KG k: four MFMA steps, lane l taking k = 4 (l / MS) + j at step j in both operands.
-  constexpr int KG = 4 * (64 / MS);
-  static_assert(BK % KG == 0, "K step");
-  typedef Mfma<MS> MF;
+  constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 16, TN = WTN / 16;
+  static_assert(TM >= 1 && TN >= 1 && TM <= 2 && TN <= 2, "wave tiles");
+  // A group of 16 k: four MFMA steps, lane l taking k = 4 (l / 16) + j at step j in both operands.
+  // v_mfma_f32_16x16x4_f32: lane l supplies row (A) / column (B) l % 16, and register r of its
+  // accumulator holds row 4 (l / 16) + r, column l % 16.
+  static_assert(BK % 16 == 0, "K step");
   constexpr bool AK = !TA, BKC = TB;  // K-contiguous operands
   typedef TileLds<BM, BN, BK, TA, TB> L;
   constexpr int LDA = L::LDA, LDB = L::LDB, SA = L::SA, SB = L::SB;
@@ -119,7 +99,7 @@ __device__ __forceinline__ void gemm_f32_tile(const float* __restrict__ A, const
   float(*Bs)[SB] = (float(*)[SB])(smem + 2 * SA);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave / WN, wn = wave % WN;
-  const TileIndex ti = tile_of(bid, nb, tiles_m, tiles_n, swizzle);
+  const TileIndex ti = tile_of(bid, nb, tiles_m, tiles_n);
   const uint32_t b = ti.z / splits, sp = ti.z % splits;
   const int m0 = ti.tm * BM, n0 = ti.tn * BN;
   const float* Ab = A + batch_offset(a_off, a_stride, b);
@@ -152,13 +132,13 @@ __device__ __forceinline__ void gemm_f32_tile(const float* __restrict__ A, const
     else xb.load(Bb, N, k0, n0, kend, N, tid);
   };
 
-  typename MF::acc_t acc[TM][TN];
+  floatx4 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; i++)
 #pragma unroll
     for (int j = 0; j < TN; j++)
 #pragma unroll
-      for (int r = 0; r < MF::REGS; r++) acc[i][j][r] = 0.0f;
+      for (int r = 0; r < 4; r++) acc[i][j][r] = 0.0f;
 
   if (nk > 0) {
     load_tiles(0, IC<0>());
@@ -167,16 +147,16 @@ __device__ __forceinline__ void gemm_f32_tile(const float* __restrict__ A, const
     sb0.store(Bs[0], LDB, tid);
   }
   __syncthreads();
-  const int li = lane % MS, q4 = (lane / MS) * 4;
+  const int li = lane % 16, q4 = (lane / 16) * 4;
   auto multiply = [&](const float* as, const float* bs) __attribute__((always_inline)) {
 #pragma unroll
-    for (int kg = 0; kg < BK; kg += KG) {
+    for (int kg = 0; kg < BK; kg += 16) {
       float a[4][TM], bv[4][TN];  // [k-step][tile]
       if (AK) {
 #pragma unroll
         for (int i = 0; i < TM; i++) {
           float v[4];
-          lds_read<4>(as + (wm * WTM + i * MS + li) * LDA + kg + q4, v);
+          lds_read<4>(as + (wm * WTM + i * 16 + li) * LDA + kg + q4, v);
 #pragma unroll
           for (int j = 0; j < 4; j++) a[j][i] = v[j];
         }
@@ -188,7 +168,7 @@ __device__ __forceinline__ void gemm_f32_tile(const float* __restrict__ A, const
 #pragma unroll
         for (int i = 0; i < TN; i++) {
           float v[4];
-          lds_read<4>(bs + (wn * WTN + i * MS + li) * LDB + kg + q4, v);
+          lds_read<4>(bs + (wn * WTN + i * 16 + li) * LDB + kg + q4, v);
 #pragma unroll
           for (int j = 0; j < 4; j++) bv[j][i] = v[j];
         }
@@ -204,8 +184,8 @@ __device__ __forceinline__ void gemm_f32_tile(const float* __restrict__ A, const
           for (int n = 0; n < TN; n++) {
             // With a K-contiguous B the product is formed transposed (B supplies the MFMA rows), so
             // that each lane ends up with four adjacent output columns.
-            if constexpr (BKC) acc[i][n] = MF::step(bv[j][n], a[j][i], acc[i][n]);
-            else acc[i][n] = MF::step(a[j][i], bv[j][n], acc[i][n]);
+            if constexpr (BKC) acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[j][n], a[j][i], acc[i][n], 0, 0, 0);
+            else acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][i], bv[j][n], acc[i][n], 0, 0, 0);
           }
     }
   };
@@ -228,12 +208,11 @@ __device__ __forceinline__ void gemm_f32_tile(const float* __restrict__ A, const
     iteration(t + 1, IC<1>());
   }
   if (t < nk) iteration(t, IC<0>());
-  // Accumulator register r of lane l holds MFMA row rho(r) = 8 (r / 4) + 4 (l / MS) + r % 4, column
-  // l % MS (for the transposed form: output row l % MS, column rho(r)). MFMA tile i row rho is
-  // block row MS i + rho (K-contiguous A) or TM rho + i (M-contiguous A); tile n column gamma is
-  // block column MS n + gamma (K-contiguous B) or TN gamma + n (N-contiguous B). Either way a lane
-  // holds adjacent output columns: four per group of four registers in one tile (K-contiguous B)
-  // or one in each of its TN tiles.
+  // Accumulator register r of lane l holds MFMA row rho = 4 (l / 16) + r, column l % 16 (for the
+  // transposed form: output row l % 16, column rho). MFMA tile i row rho is block row 16 i + rho
+  // (K-contiguous A) or TM rho + i (M-contiguous A); tile n column gamma is block column
+  // 16 n + gamma (K-contiguous B) or TN gamma + n (N-contiguous B). Either way a lane holds adjacent
+  // output columns: four in one tile (K-contiguous B) or one in each of its TN tiles.
   epi.begin(b, sp);
   const bool vec_out = MODE != LOAD_SCALAR && N % 4 == 0;
   // A per-column bias (unsplit products only) added to the finished sums, as one fp32 addition.
@@ -242,20 +221,18 @@ __device__ __forceinline__ void gemm_f32_tile(const float* __restrict__ A, const
 #pragma unroll
       for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int n = 0; n < TN; n++)
+        for (int n = 0; n < TN; n++) {
+          const int col = n0 + wn * WTN + n * 16 + q4;
 #pragma unroll
-          for (int g = 0; g < MF::REGS / 4; g++) {
-            const int col = n0 + wn * WTN + n * MS + 8 * g + q4;
-#pragma unroll
-            for (int r = 0; r < 4; r++)
-              if (col + r < N) acc[i][n][4 * g + r] += bias[col + r];
-          }
+          for (int r = 0; r < 4; r++)
+            if (col + r < N) acc[i][n][r] += bias[col + r];
+        }
     } else {
       const int col = n0 + wn * WTN + TN * li;
 #pragma unroll
       for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int r = 0; r < MF::REGS; r++)
+        for (int r = 0; r < 4; r++)
 #pragma unroll
           for (int n = 0; n < TN; n++)
             if (col + n < N) acc[i][n][r] += bias[col + n];
@@ -264,37 +241,34 @@ __device__ __forceinline__ void gemm_f32_tile(const float* __restrict__ A, const
   if constexpr (BKC) {
 #pragma unroll
     for (int i = 0; i < TM; i++) {
-      const int row = m0 + wm * WTM + (AK ? i * MS + li : TM * li + i);
+      const int row = m0 + wm * WTM + (AK ? i * 16 + li : TM * li + i);
       if (row >= M) continue;
       const uint64_t erow = (uint64_t)row * N;
 #pragma unroll
-      for (int n = 0; n < TN; n++)
+      for (int n = 0; n < TN; n++) {
+        const int col = n0 + wn * WTN + n * 16 + q4;
+        const floatx4 c = acc[i][n];
+        if (vec_out && col + 4 <= N) {
+          epi.put4(erow + col, make_float4(c[0], c[1], c[2], c[3]));
+        } else {
 #pragma unroll
-        for (int g = 0; g < MF::REGS / 4; g++) {
-          const int col = n0 + wn * WTN + n * MS + 8 * g + q4;
-          const auto& c = acc[i][n];
-          if (vec_out && col + 4 <= N) {
-            epi.put4(erow + col, make_float4(c[4 * g], c[4 * g + 1], c[4 * g + 2], c[4 * g + 3]));
-          } else {
-#pragma unroll
-            for (int r = 0; r < 4; r++)
-              if (col + r < N) epi.put1(erow + col + r, c[4 * g + r]);
-          }
+          for (int r = 0; r < 4; r++)
+            if (col + r < N) epi.put1(erow + col + r, c[r]);
         }
+      }
     }
   } else {
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
-      for (int r = 0; r < MF::REGS; r++) {
-        const int rho = 8 * (r / 4) + q4 + r % 4;
-        const int row = m0 + wm * WTM + (AK ? i * MS + rho : TM * rho + i);
+      for (int r = 0; r < 4; r++) {
+        const int rho = q4 + r;
+        const int row = m0 + wm * WTM + (AK ? i * 16 + rho : TM * rho + i);
         if (row >= M) continue;
         const uint64_t erow = (uint64_t)row * N;
         const int col = n0 + wn * WTN + TN * li;
         if (TN > 1 && vec_out && col + TN <= N) {
-          if constexpr (TN == 4) epi.put4(erow + col, make_float4(acc[i][0][r], acc[i][1][r], acc[i][2][r], acc[i][3][r]));
-          else if constexpr (TN == 2) epi.put2(erow + col, make_float2(acc[i][0][r], acc[i][1][r]));
+          if constexpr (TN == 2) epi.put2(erow + col, make_float2(acc[i][0][r], acc[i][1][r]));
         } else {
 #pragma unroll
           for (int n = 0; n < TN; n++)
@@ -305,14 +279,14 @@ __device__ __forceinline__ void gemm_f32_tile(const float* __restrict__ A, const
 }
 
 // One product over the whole grid, with its own LDS.
-template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB, int MODE, int MS, class Epi>
+template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB, int MODE, class Epi>
 __device__ __forceinline__ void gemm_f32_block(const float* __restrict__ A, const float* __restrict__ B, int M, int N, int K,
                                                 const int64_t* a_off, const int64_t* b_off, uint64_t a_stride, uint64_t b_stride, int splits,
                                                 int k_per_split, const float* __restrict__ bias, uint32_t tiles_m, uint32_t tiles_n,
-                                                int swizzle, Epi& epi) {
+                                                Epi& epi) {
   __shared__ float smem[TileLds<BM, BN, BK, TA, TB>::FLOATS];
-  gemm_f32_tile<BM, BN, BK, WM, WN, TA, TB, MODE, MS>(A, B, M, N, K, a_off, b_off, a_stride, b_stride, splits, k_per_split, bias, tiles_m,
-                                                      tiles_n, swizzle, epi, blockIdx.x, gridDim.x, smem);
+  gemm_f32_tile<BM, BN, BK, WM, WN, TA, TB, MODE>(A, B, M, N, K, a_off, b_off, a_stride, b_stride, splits, k_per_split, bias, tiles_m, tiles_n,
+                                                  epi, blockIdx.x, gridDim.x, smem);
 }
 
 }  // namespace rgg

@@ -53,7 +53,7 @@ __device__ __forceinline__ int64_t batch_offset(const int64_t* offs, uint64_t st
 }
 
 // Which output tile a block computes. The dispatcher deals consecutive blocks round-robin over
-// the 8 XCDs, each with its own L2; with `swizzle`, XCD x instead receives the contiguous run
+// the 8 XCDs, each with its own L2; so XCD x is to receive the contiguous run
 // x*nb/8 ... (x+1)*nb/8 - 1 of tiles, and within a batch the tiles run in groups of 8 M-panels
 // per N sweep, so blocks resident on one XCD share their A and B panels in its L2.
 struct TileIndex {
@@ -61,9 +61,8 @@ struct TileIndex {
 };
 
 // Block `bid` of a product launched as `nb` blocks (its share of the grid).
-__device__ __forceinline__ TileIndex tile_of(uint32_t bid, uint32_t nb, uint32_t tiles_m, uint32_t tiles_n, int swizzle) {
+__device__ __forceinline__ TileIndex tile_of(uint32_t bid, uint32_t nb, uint32_t tiles_m, uint32_t tiles_n) {
   uint32_t per_batch = tiles_m * tiles_n;
-  if (!swizzle) return {(bid % per_batch) / tiles_n, bid % tiles_n, bid / per_batch};
   uint32_t lid = (nb % 8 == 0) ? (bid % 8) * (nb / 8) + bid / 8 : bid;
   uint32_t z = lid / per_batch, t = lid % per_batch;
   constexpr uint32_t GROUP = 8;
@@ -250,7 +249,7 @@ __device__ __forceinline__ void gemm_split_tile(const float* __restrict__ A, con
   typedef SplitGeo<BN, TB, NT> GB;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave / WN, wn = wave % WN, li = lane & 15, lo = lane >> 4;
-  const TileIndex ti = tile_of(bid, nb, tiles_m, tiles_n, 1);
+  const TileIndex ti = tile_of(bid, nb, tiles_m, tiles_n);
   const uint32_t b = ti.z / splits, sp = ti.z % splits;
   const int m_first = ti.tm * BM, n_first = ti.tn * BN, m0 = min(m_first, M - BM), n0 = min(n_first, N - BN);
   const int64_t lda = TA ? M : K, ldb = TB ? K : N;

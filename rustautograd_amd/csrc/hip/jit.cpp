@@ -305,7 +305,7 @@ std::string generate_gemm(const rgplan::Fused& f, int64_t c_slot, bool store_c, 
     s << "    if (lane < 8) *(float4*)&cs[wmi][wni * 32 + 4 * lane] = v;\n  }\n";
     s << "  __syncthreads();\n";
     s << "  if (threadIdx.x < " << t.bn << ") {\n";
-    s << "    const rgg::TileIndex ti = rgg::tile_of(blockIdx.x, gridDim.x, tiles_m, tiles_n, 1);\n";
+    s << "    const rgg::TileIndex ti = rgg::tile_of(blockIdx.x, gridDim.x, tiles_m, tiles_n);\n";
     s << "    float v = cs[0][threadIdx.x];\n";
     s << "    for (int w = 1; w < " << t.wm << "; w++) v = v + cs[w][threadIdx.x];\n";
     s << "    colp[(rgg::uint64_t)ti.tm * N + ti.tn * " << t.bn << " + threadIdx.x] = v;\n  }\n";
@@ -326,6 +326,7 @@ std::string generate_outer(const rgplan::Fused& f, int64_t m, int64_t n, const s
   k->name = name;
   k->vec = 4 * U;
   k->grid = (uint32_t)(gx * ((m + 4 * rows - 1) / (4 * rows)));
+  // Element indices are 32-bit: a program with a slot of 2^31 elements or more is refused when it is built.
   auto product_at = [&](int64_t slot) {
     for (size_t p = 0; p < products.size(); p++)
       if (products[p].slot == slot) return (int)p;

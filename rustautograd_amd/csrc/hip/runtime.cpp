@@ -1697,7 +1697,6 @@ void run_cond(hipStream_t s, const Program::Control& c, const Program& owner, co
   cp.flush();
 }
 
-// Every slot fits the device and the kernels' 32-bit element indexing.
 // The HIP source of every fused kernel of a plan and of its control-flow bodies (each body's
 // kernels under their own prefix), as the runtime generates it; `count` kernels.
 std::string plan_source(const Plan& root, int* count) {
@@ -1734,6 +1733,7 @@ std::string plan_source(const Plan& root, int* count) {
   return src.str();
 }
 
+// Every slot fits the device and the kernels' 32-bit element indexing.
 void check_slots(const Plan& plan) {
   size_t free_b = 0, total = 0;
   HIP_OK(hipMemGetInfo(&free_b, &total));
