@@ -1222,11 +1222,45 @@ size_t Plan::planned_bytes() const {
   return b;
 }
 
+// What each register of a row group holds: 0 a value per element, 1 one per row (it is read per row:
+// a splat, or a broadcast of a [rows..., 1] value; a last-axis reduction; or computed from such
+// registers alone), 2 one per column (a reduction over the rows).
+static std::vector<int> row_group_levels(const Fused& f) {
+  const size_t last = f.shape.size() - 1;
+  std::vector<int> level(f.regs, 0);
+  for (size_t j = 0; j < f.inputs.size(); j++) {
+    const FusedIn& in = f.inputs[j];
+    if (in.reg == SIZE_MAX) continue;
+    const Shape& xs = f.input_shapes[j];
+    level[in.reg] = in.kind == RG_ARG_SPLAT || (in.kind == RG_ARG_BROADCAST && (xs.empty() || xs.back() == 1)) ? 1 : 0;
+  }
+  for (auto& m : f.ops) {
+    if (m.op.kind == RG_OP_REDUCE) {
+      const bool over_last = std::find(m.op.v.begin(), m.op.v.end(), (int64_t)last) != m.op.v.end();
+      level[m.reg] = over_last ? 1 : 2;
+      continue;
+    }
+    bool per_row = true;
+    for (auto& a : m.args) per_row = per_row && a.first && level[a.second] == 1;
+    level[m.reg] = per_row ? 1 : 0;
+  }
+  return level;
+}
+
+// Elements a fused group writes.
+static size_t group_outputs(const Fused& f) {
+  if (f.row_len == 0) return f.n * f.outputs.size();
+  const std::vector<int> level = row_group_levels(f);
+  size_t n = 0;
+  for (auto& o : f.outputs) n += level[o.first] == 1 ? f.n / std::max<size_t>(f.row_len, 1) : level[o.first] == 2 ? f.row_len : f.n;
+  return n;
+}
+
 double Plan::gpu_cost_estimate(const Fuse& f) const {
   double c = 0;
   for (auto& s : steps) {
     double n = s.attn ? (double)(s.att.shape.bh * s.att.shape.tq * s.att.shape.hd * s.att.out.size())
-                      : (double)(s.fused ? s.group.n * s.group.outputs.size() : s.instr.n);
+                      : (double)(s.fused ? group_outputs(s.group) : s.instr.n);
     c += f.per_dispatch_ns + f.per_element_ns * n;
   }
   return c;
@@ -1276,28 +1310,7 @@ StepWork step_work(const Step& s, const PriceFn& price) {
       w.bytes += (double)(f.n * f.outputs.size()) * ds;
       return w;
     }
-    // A row group: a register holds one value per row when it is read per row (a splat, or a
-    // broadcast of a [rows..., 1] value), is a last-axis reduction, or is computed from such
-    // registers alone; a reduction over the rows holds one value per column.
-    const size_t L = f.row_len, rows = f.n / std::max<size_t>(L, 1), last = f.shape.size() - 1;
-    std::vector<int> level(f.regs, 0);  // 0 full, 1 per row, 2 per column
-    for (size_t j = 0; j < f.inputs.size(); j++) {
-      const FusedIn& in = f.inputs[j];
-      if (in.reg == SIZE_MAX) continue;
-      const Shape& xs = f.input_shapes[j];
-      level[in.reg] = in.kind == RG_ARG_SPLAT || (in.kind == RG_ARG_BROADCAST && (xs.empty() || xs.back() == 1)) ? 1 : 0;
-    }
-    for (auto& m : f.ops) {
-      if (m.op.kind == RG_OP_REDUCE) {
-        const bool over_last = std::find(m.op.v.begin(), m.op.v.end(), (int64_t)last) != m.op.v.end();
-        level[m.reg] = over_last ? 1 : 2;
-        continue;
-      }
-      bool per_row = true;
-      for (auto& a : m.args) per_row = per_row && a.first && level[a.second] == 1;
-      level[m.reg] = per_row ? 1 : 0;
-    }
-    for (auto& o : f.outputs) w.bytes += (double)(level[o.first] == 1 ? rows : level[o.first] == 2 ? L : f.n) * ds;
+    w.bytes += (double)group_outputs(f) * ds;
     return w;
   }
   const Instr& i = s.instr;

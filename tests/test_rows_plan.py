@@ -14,6 +14,9 @@ import json
 import numpy as np
 import pytest
 
+import rustautograd_amd as rg
+from rustautograd_amd import nn
+
 from conftest import DEVPLAN
 from helpers import G
 from test_hip_rows import _layer_norm
@@ -146,3 +149,14 @@ def test_bias_adds_fold_into_the_product(m, k, n, ta):
     got = g.eval(outs, inputs, device=DEVPLAN, optimize="standard")[0]
     want = g.eval(outs, inputs, device="cpu", optimize="standard")[0]
     np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("rows,length", [(4096, 2048), (20000, 1030), (1100, 8192), (8192, 1024)])
+def test_large_softmaxes_keep_their_row_group(rows, length):
+    """From 8 million elements on a plan is chosen by what its groups are estimated to write, and a
+    row group's per-row values (the sums beside the exponentials) count once per row: counted at
+    full size the group looked dearer than its operations one by one, which took a quarter longer
+    at 4096 x 2048 than with no row group in sight."""
+    x = rg.tensor(np.zeros((rows, length), np.float32))
+    steps = rg.compile(lambda x: nn.softmax(x), (x,), device=DEVPLAN, validate="none").plan_summary()
+    assert [(s["kind"], s.get("row_len")) for s in steps] == [("fused", length), ("fused", 0)], steps
