@@ -1264,12 +1264,15 @@ bool gemm_group(hipStream_t s, const GemmArgs* g, int count, bool launch) {
     }
   }
   // One tile for all. Split tiles: 128x128, since every split tile sums a K range's terms in the same
-  // order, so a product picked for a smaller one keeps its bits, and its K splits. fp32 tiles: 32x32
-  // whole ones. K-split partials, if any, must be the deferred kind: a split sum after the grouped
-  // launch would be a second launch anyway.
+  // order, so a product picked for a smaller one keeps its bits, and its K splits; one step in LDS, two
+  // blocks per CU (the 4096 x 512 x 2048 MLP's pair of 512 blocks each, 96 steps: 99.9 ms, 104.6 with two
+  // steps and a block per CU, 101.5 as single launches; the GPT of 8192 tokens, d = 256, 120 steps: 375,
+  // 375 and 394 ms, two steps for its pair of 256 blocks alone no faster). fp32 tiles: 32x32 whole ones.
+  // K-split partials, if any, must be the deferred kind: a split sum after the grouped launch would be a
+  // second launch anyway.
   const TileCfg first = pick_tile(g[0].m, g[0].n, g[0].k, 1);
   const bool split = first.split;
-  const TileCfg t = split ? SPLIT_128x128_2 : TileCfg{32, 32, 32, 2, 2, 0};
+  const TileCfg t = split ? SPLIT_128x128 : TileCfg{32, 32, 32, 2, 2, 0};
   int mode;
   Launch l[GROUP_MAX];
   int flags = 0;
@@ -1299,7 +1302,7 @@ bool gemm_group(hipStream_t s, const GemmArgs* g, int count, bool launch) {
   }
 #define RG_GROUP(COUNT_, FLAGS_)                                                                                                   \
   if (count == COUNT_ && flags == (FLAGS_)) {                                                                                      \
-    if (launch && split) hipLaunchKernelGGL((k_gemm_mfma_group<128, 128, 2, 4, 2, COUNT_, FLAGS_>), dim3(blocks), dim3(512), 0, s, parts); \
+    if (launch && split) hipLaunchKernelGGL((k_gemm_mfma_group<128, 128, 2, 4, 1, COUNT_, FLAGS_>), dim3(blocks), dim3(512), 0, s, parts); \
     else if (launch) hipLaunchKernelGGL((k_gemm_f32_group<COUNT_, FLAGS_>), dim3(blocks), dim3(256), 0, s, parts);                  \
     return true;                                                                                                                   \
   }
