@@ -729,7 +729,8 @@ struct Skinny {
 };
 
 // fp32 products on matrix cores: both sides at least 32, or at least 16 at a K under 512 (attention
-// heads of 16 or 24; a longer K streams).
+// heads of 16 or 24). With a longer K, 16 columns or rows stream, and sides of 17 to 31 take a block per
+// output (k_gemm_tiny_out) up to 16384 outputs and a thread per output above.
 bool use_mfma(int dtype, uint64_t m, uint64_t n, uint64_t k) {
   const uint64_t side = k < 512 ? 16 : 32;
   return dtype == RG_F32 && m >= side && n >= side && k >= 8 && m * n * k >= (1u << 18);

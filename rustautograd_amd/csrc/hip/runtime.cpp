@@ -1006,8 +1006,9 @@ void find_product_epilogues(const Plan& plan, Epilogues* found) {
       ep.moves(plan, from, to);
       // A column sum of one of the group's outputs a few steps later, with nothing between that
       // overwrites the output or needs the sum's slot (sum_moves): computed by the combined kernel
-      // from the values it stores, summed in registers (a K-contiguous B, whole tiles: every output
-      // goes through put4). RG_HIP_EPILOGUE_SUMS=0 leaves it to its own kernel.
+      // from the values it stores, summed in registers (whole tiles: every output goes through put4;
+      // asked for with a K-contiguous B only, though a lane stores the same four columns of every row
+      // with either layout). RG_HIP_EPILOGUE_SUMS=0 leaves it to its own kernel.
       const char* sums = getenv("RG_HIP_EPILOGUE_SUMS");
       if ((sums && sums[0] == '0') || !tb || !tile.whole) break;
       for (size_t q = j + 1; q < n && q <= j + 4; q++) {
