@@ -389,7 +389,9 @@ struct RowsLds {
 typedef const __attribute__((address_space(4))) float* ConstOperand;
 
 // Block (bx, by) of k_gemm_skinny_rows, its wave sums combined through `lds`.
-template <int MR>
+// AHEAD: B's next eight rows wait in registers of their own (3x2050x8192 35.3 us against 36.3, 8x8192x2048
+// 28.3 and 28.8; 154 registers for 8 rows, 120 without).
+template <int MR, bool AHEAD = true>
 __device__ __forceinline__ void skinny_rows_block(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ out, int M,
                                                   int N, int K, bool ta, int kps, uint32_t bx, uint32_t by, float4* lds) {
   float4(*red)[MR][64] = (float4(*)[MR][64])lds;
@@ -417,7 +419,7 @@ __device__ __forceinline__ void skinny_rows_block(const float* __restrict__ A, c
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
   };
-  auto load = [&](float4 (&b)[8], int k) __attribute__((always_inline)) {
+  auto load = [&](float4* b, int k) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < 8; u++) b[u] = row4(B + (uint64_t)(k + u) * N + colr);
   };
@@ -441,7 +443,7 @@ __device__ __forceinline__ void skinny_rows_block(const float* __restrict__ A, c
     }
   };
   const int whole = kw0 + (kw1 - kw0) / 8 * 8;
-  float4 b0[8], b1[8];
+  float4 b0[8], b1[AHEAD ? 8 : 1];
   if (kw0 < whole) load(b0, kw0);
   int kc = kw0;
   if (kw0 < kw1) stage(kw0);
@@ -449,13 +451,24 @@ __device__ __forceinline__ void skinny_rows_block(const float* __restrict__ A, c
   for (int k = kw0; k < whole; k += 16) {
     if (k - kc == 64) stage(kc = k);
     const bool second = k + 8 < whole;
-    if (second) load(b1, k + 8);
+    if constexpr (AHEAD) {
+      if (second) load(b1, k + 8);
 #pragma unroll
-    for (int u = 0; u < 8; u++) row(k - kc + u, b0[u]);
-    if (second) {
+      for (int u = 0; u < 8; u++) row(k - kc + u, b0[u]);
+      if (second) {
+        if (k + 16 < whole) load(b0, k + 16);
+#pragma unroll
+        for (int u = 0; u < 8; u++) row(k - kc + 8 + u, b1[u]);
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < 8; u++) row(k - kc + u, b0[u]);
+      if (second) {
+        load(b0, k + 8);
+#pragma unroll
+        for (int u = 0; u < 8; u++) row(k - kc + 8 + u, b0[u]);
+      }
       if (k + 16 < whole) load(b0, k + 16);
-#pragma unroll
-      for (int u = 0; u < 8; u++) row(k - kc + 8 + u, b1[u]);
     }
     add();
   }
@@ -691,7 +704,7 @@ struct StreamParts {
 __device__ __forceinline__ void stream_part(const StreamPart& p, uint32_t bid, float4* lds) {
   const uint32_t bx = bid % p.gx, by = bid / p.gx;
   switch (p.kind) {
-    case STREAM_ROWS8: skinny_rows_block<8>(p.a, p.b, p.out, p.m, p.n, p.k, p.ta, p.arg, bx, by, lds); break;
+    case STREAM_ROWS8: skinny_rows_block<8, false>(p.a, p.b, p.out, p.m, p.n, p.k, p.ta, p.arg, bx, by, lds); break;
     case STREAM_DOT8: skinny_dot_block<8, 4>(p.a, p.b, p.out, p.m, p.n, p.k, p.arg, bx, by, p.gy, lds); break;
     case STREAM_OUTER8_TN: outer_block<8, true, false>(p.a, p.b, p.out, p.m, p.n, p.k, p.arg, bx, by); break;
     case STREAM_OUTER8_NT: outer_block<8, false, true>(p.a, p.b, p.out, p.m, p.n, p.k, p.arg, bx, by); break;
@@ -706,7 +719,10 @@ __device__ __forceinline__ void stream_part(const StreamPart& p, uint32_t bid, f
 // outputs with a long K, in one launch: part i takes the next p[i].blocks blocks and runs its own
 // kernel's block code, with one LDS buffer. The reads of one product and the writes of another share HBM in the same launch, and
 // the launch's fixed cost is paid once.
-__global__ void __launch_bounds__(256) k_stream_group(StreamParts g) {
+// At most 128 registers, four waves per SIMD: the row kernel's blocks load B's next rows into the
+// registers of the last ones, the same sums (the chain of 4096 x 4096 by 8 rows, three such launches a
+// pass: 71.5 us, 75.0 with rows loaded ahead at 156 registers).
+__global__ void __launch_bounds__(256, 4) k_stream_group(StreamParts g) {
   constexpr int F = RowsLds<8>::FLOAT4S > DotLds<8>::FLOAT4S ? RowsLds<8>::FLOAT4S : DotLds<8>::FLOAT4S;
   __shared__ float4 lds[F];
   uint32_t bid = blockIdx.x;
