@@ -855,7 +855,8 @@ int split_count(const TileCfg& t, uint64_t m, uint64_t n, uint64_t k, uint64_t b
 // Below that a block runs alone on its CU and fp32 MFMA tiles are faster: 32-wide ones for outputs
 // 32..96 wide or 32 tall (attention heads, the vocabulary), 32x32 otherwise (256x768x256: 4.3
 // against 7.1 on bf16 terms; 4096x128x512: 8.6 and 13), or 64x64 where a side under 64 keeps a
-// large output off the tiles above.
+// large output off the tiles above. (Figures of single launches before the operands were scaled, which
+// adds up to 4 % to each of the bf16 tiles alike.)
 TileCfg pick_tile(uint64_t m, uint64_t n, uint64_t k, uint64_t batch) {
   auto filled = [&](const TileCfg& t) { return tile_count(t, m, n, batch) * (uint64_t)split_count(t, m, n, k, batch); };
   // A column-contiguous operand's offsets within 24 rows are 32-bit: sides of less than 2^25.
